@@ -18,7 +18,7 @@ LIB = os.path.join(HERE, "libmps_amd.so")
 ROOT = os.path.dirname(HERE)
 INCLUDE = os.path.join(ROOT, "include")
 
-SOURCES = ["grid.hip", "stages.hip", "ppe.hip", "mg.hip", "adjoint.hip", "capi.hip"]
+SOURCES = ["grid.hip", "stages.hip", "ppe.hip", "resident.hip", "mg.hip", "adjoint.hip", "capi.hip"]
 HOST = os.path.join(HERE, "host")
 HOST_SOURCES = ["particle.cpp", "logger.cpp", "settings.cpp", "exporter.cpp", "async_export.cpp", "bucket.cpp",
                 "mps.cpp", "simulation.cpp", "hooks.cpp"]
@@ -27,7 +27,8 @@ CLI = os.path.join(HERE, "mps")
 CXX = os.environ.get("CXX", "g++")
 HOST_FLAGS = ["-std=c++17", "-O2", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-parameter", "-ffp-contract=off",
               f"-I{INCLUDE}"]
-HEADERS = [os.path.join(CSRC, "mps_internal.hpp"), os.path.join(INCLUDE, "mps_amd.h")]
+HEADERS = [os.path.join(CSRC, "mps_internal.hpp"), os.path.join(CSRC, "cg_device.hpp"),
+           os.path.join(INCLUDE, "mps_amd.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("MPS_AMD_ARCH", "gfx950")

@@ -35,9 +35,10 @@
 #include <cstring>
 
 #include <algorithm>
+#include <atomic>
 #include <vector>
 
-#include "mps_internal.hpp"
+#include "cg_device.hpp"
 
 namespace mps {
 
@@ -368,10 +369,6 @@ hipError_t assemble_sell(int dim, const GridView& g, const SceneTab& tab, int n,
 //           p = r + beta p; s = w + beta s; y += alpha p; r -= alpha s
 // apply gathers only r, once per stored entry; step is elementwise.
 
-constexpr int kMaxBlocks = 1024;  // per segment
-// Threads per block of the per-iteration kernels (apply, step): 1024 blocks
-// of 512 fill every SIMD with 8 waves, twice the loads in flight of 256.
-constexpr int kCgBlock = 512;
 constexpr int kStepPre = 4;  // rows a thread of k_cg_step loads ahead of the partials' reduction
 // Below this many rows the V-cycle's setup and launches cost more than the
 // iterations it saves (measured: 584-particle dam break), so small systems
@@ -405,145 +402,6 @@ static int cg_blocks(int rows) {
     int nb = (rows + rpb - 1) / rpb;
     if (nb > kMaxBlocks) nb = kMaxBlocks;
     return nb < 1 ? 1 : nb;
-}
-
-struct CgScalars {
-    double gam[2];     // r.r by iteration parity
-    double alp[2];     // alpha by iteration parity
-    double thr;        // stop when rho2 <= thr
-    double rho2;       // latest residual^2 (unscaled sum a_ii r_i^2, or r.r for inner solves)
-    double red[3];     // results of k_reduce_parts
-    int iter;          // apply launches run (read by every block of k_cg_step)
-    int max_iter;
-    int done;
-    int converged;
-    int frozen;        // timing mode: kernels leave every scalar as it is
-    int fin;           // completed updates, written once when the segment stops
-};
-
-struct Seg {
-    int nseg;
-    const int* blk_off;  // nseg + 1: first block of each segment
-    const int* row_off;  // nseg + 1: first row of each segment
-};
-
-__device__ __forceinline__ int seg_of_block(const Seg& sg, int b) {
-    int lo = 0, hi = sg.nseg - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (sg.blk_off[mid] <= b)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return lo;
-}
-
-struct BlockRows {
-    int seg, v, nb, b0;  // segment, block within it, its block count, its first block
-    int lb;              // the block's place among the segment's contiguous row ranges
-    int r0, r1;          // rows of this block
-};
-
-// Row range of this block: contiguous within the segment, whole multiples of
-// 64 rows from the segment start, XCD-grouped.
-__device__ __forceinline__ BlockRows block_rows(const Seg& sg) {
-    BlockRows br;
-    br.seg = seg_of_block(sg, blockIdx.x);
-    br.b0 = sg.blk_off[br.seg];
-    br.v = blockIdx.x - br.b0;
-    br.nb = sg.blk_off[br.seg + 1] - br.b0;
-    const int base = sg.row_off[br.seg];
-    const int rows = sg.row_off[br.seg + 1] - base;
-    const int per = ((rows + br.nb - 1) / br.nb + 63) & ~63;
-    const int lb = xcd_block(br.v, br.nb);
-    br.lb = lb;
-    br.r0 = base + lb * per;
-    const int end = base + rows;
-    br.r1 = br.r0 + per < end ? br.r0 + per : end;
-    if (br.r0 > end) br.r0 = end;
-    return br;
-}
-
-// Fixed-order sum of NV interleaved partials (part[b*NV + k], b < nb) in every
-// block; result broadcast to all threads.
-template <int NV>
-__device__ __forceinline__ void reduce_partials(const double* __restrict__ part, int nb, double (&out)[NV],
-                                                double* red) {
-    double acc[NV];
-    for (int k = 0; k < NV; k++) acc[k] = 0.0;
-    for (int b = threadIdx.x; b < nb; b += blockDim.x)
-        for (int k = 0; k < NV; k++) acc[k] += part[(size_t) NV * b + k];
-    for (int k = 0; k < NV; k++) {
-        double a = acc[k];
-        for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-        if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * NV + k] = a;
-    }
-    __syncthreads();
-    for (int k = 0; k < NV; k++) {
-        double t = 0.0;
-        for (int w = 0; w < (int) (blockDim.x >> 6); w++) t += red[w * NV + k];
-        out[k] = t;
-    }
-    __syncthreads();
-}
-
-template <int NV>
-__device__ __forceinline__ void write_partials(const double (&v)[NV], double* __restrict__ part, double* red) {
-    for (int k = 0; k < NV; k++) {
-        double a = v[k];
-        for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-        if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * NV + k] = a;
-    }
-    __syncthreads();
-    if (threadIdx.x < NV) {
-        double t = 0.0;
-        for (int w = 0; w < (int) (blockDim.x >> 6); w++) t += red[w * NV + threadIdx.x];
-        part[(size_t) NV * blockIdx.x + threadIdx.x] = t;
-    }
-}
-
-__device__ __forceinline__ int block_uniform_done(CgScalars* sc) {
-    __shared__ int s_done;
-    if (threadIdx.x == 0) s_done = *(volatile int*) &sc->done;
-    __syncthreads();
-    return s_done;
-}
-
-// acc + sum_k val[k] x[col[k]] over the row's SELL entries, gathers issued in
-// batches of 4 for memory-level parallelism.  NT: the matrix is read with
-// nontemporal loads (the FP64 solve's apply: its 10 bytes an entry do not
-// fit the Infinity Cache beside the solver's vectors, and streaming them
-// keeps the vectors and coarse levels cached: 2M FP64 step -6 %; the FP32
-// matrix does fit and is read normally, as is the FP64 residual's, where
-// nontemporal loads made the mixed step 2 % slower).
-template <typename T, typename IDX, bool NT = false>
-__device__ __forceinline__ T sell_row(const int* __restrict__ slice_pos, const IDX* __restrict__ col,
-                                      const int* __restrict__ anc, const T* __restrict__ val,
-                                      const T* __restrict__ x, int row, T acc) {
-    const int sl = row >> 6, lane = row & 63;
-    const int s0 = slice_pos[sl], w = slice_pos[sl + 1] - s0;
-    const size_t base = (size_t) s0 * 64 + lane;
-    int lo, hi;
-    sell_anchors<IDX>(anc, row, lo, hi);
-    int k = 0;
-    for (; k + 4 <= w; k += 4) {
-        const size_t i0 = base + (size_t) k * 64;
-        const int c0 = sell_col<IDX, NT>(col, i0, row, lo, hi), c1 = sell_col<IDX, NT>(col, i0 + 64, row, lo, hi);
-        const int c2 = sell_col<IDX, NT>(col, i0 + 128, row, lo, hi), c3 = sell_col<IDX, NT>(col, i0 + 192, row, lo, hi);
-        const T v0 = ld_stream<NT>(val + i0), v1 = ld_stream<NT>(val + i0 + 64);
-        const T v2 = ld_stream<NT>(val + i0 + 128), v3 = ld_stream<NT>(val + i0 + 192);
-        const T x0 = x[c0], x1 = x[c1], x2 = x[c2], x3 = x[c3];
-        acc += v0 * x0;
-        acc += v1 * x1;
-        acc += v2 * x2;
-        acc += v3 * x3;
-    }
-    for (; k < w; k++) {
-        const size_t i0 = base + (size_t) k * 64;
-        acc += ld_stream<NT>(val + i0) * x[sell_col<IDX, NT>(col, i0, row, lo, hi)];
-    }
-    return acc;
 }
 
 // apply: w = Ahat u with u = M r (u = r without a preconditioner; unit
@@ -879,7 +737,7 @@ struct CgWork {
     // receive, the launch shape and the multigrid hierarchy's generation.
     // Any difference (a buffer reallocated by a larger system, another
     // column width) drops the cached graphs of that solver.
-    static constexpr int kSig = 24;
+    static constexpr int kSig = 29;
     uintptr_t graph_sig[2][kSig] = {};
     static constexpr int kPredSolves = 4;
     bool predict = true;  // MPS_AMD_CG_PREDICT=0: fixed chunks of the check interval
@@ -890,8 +748,24 @@ struct CgWork {
     long long graph_rebuilds = 0;  // times a solver's cached graphs were dropped
     long long vec_reallocs = 0;    // times the CG vectors were reallocated
     long long launched = 0;        // CG iterations enqueued, including those past convergence
+    // resident CG (resident.hip): exchange memory, the last tag handed out and
+    // the most blocks that can run at once (0: off, MPS_AMD_CG_RESIDENT=0 or
+    // after a launch that gave up)
+    CgExchange xch{};
+    unsigned tag = 0;
+    int res_blocks = 0;
+    int res_dev = 0;
+    unsigned res_ready = 0;  // kernel shapes prepared
+    hipGraphExec_t res_graph[2] = {};
     Seg seg() const { return Seg{nseg, blk_off, row_off}; }
 };
+
+// Blocks of resident CG launches in flight on each device.  All blocks of a
+// launch wait for each other, so launches of several handles together must
+// not need more than run at once: a solve that would exceed it runs by
+// launches instead, with the same bits.
+constexpr int kResDevices = 64;
+static std::atomic<int> g_res_in_flight[kResDevices];
 
 void cg_prediction_bank(CgWork* cw, int bank) { cw->pred_bank = bank ? 1 : 0; }
 
@@ -899,6 +773,17 @@ CgWork* cg_create() {
     CgWork* cw = new CgWork();
     if (const char* v = getenv("MPS_AMD_CG_PREDICT")) cw->predict = atoi(v) != 0;
     if (const char* v = getenv("MPS_AMD_CG_FUSE")) cw->fuse_ok = atoi(v) != 0;
+    const char* v = getenv("MPS_AMD_CG_RESIDENT");
+    int cus = 0;
+    if ((!v || atoi(v) != 0) && hipGetDevice(&cw->res_dev) == hipSuccess && cw->res_dev < kResDevices &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, cw->res_dev) == hipSuccess)
+        cw->res_blocks = cus;  // a block fits every CU (512 threads, at most 61 KB of LDS)
+    // MPS_AMD_CG_RESIDENT_HALO lowers the halo rows a block of the resident
+    // CG takes, so that a launch gives up and the solve runs by launches
+    // (tests; results unchanged)
+    cw->xch.halo_max = resident_halo_rows();
+    if (const char* hm = getenv("MPS_AMD_CG_RESIDENT_HALO"))
+        cw->xch.halo_max = std::min(cw->xch.halo_max, std::max(atoi(hm), 0));
     return cw;
 }
 
@@ -920,6 +805,10 @@ void cg_destroy(CgWork* cw) {
     hipHostFree(cw->h_blk);
     hipHostFree(cw->h_row);
     mailbox_free(cw->mb);
+    hipFree(cw->xch.w);
+    hipFree(cw->xch.part);
+    for (int k = 0; k < 2; k++)
+        if (cw->res_graph[k]) hipGraphExecDestroy(cw->res_graph[k]);
     for (int k = 0; k < 2; k++)
         for (int j = 0; j < CgWork::kGraphSlots; j++)
             if (cw->graph[k][j]) hipGraphExecDestroy(cw->graph[k][j]);
@@ -958,6 +847,16 @@ void cg_debug_counts(const CgWork* cw, long long out[4]) {
     out[3] = cw->graph_captures;
 }
 
+static void drop_graphs(CgWork* cw, int which) {
+    for (int j = 0; j < CgWork::kGraphSlots; j++) {
+        if (cw->graph[which][j]) hipGraphExecDestroy(cw->graph[which][j]);
+        cw->graph[which][j] = nullptr;
+        cw->graph_chunk[which][j] = 0;
+    }
+    if (cw->res_graph[which]) hipGraphExecDestroy(cw->res_graph[which]);
+    cw->res_graph[which] = nullptr;
+}
+
 hipError_t cg_reserve(CgWork* cw, int rows) {
     if (rows <= cw->cap && cw->y) return hipSuccess;
     const int cap = tight_caps() ? rows : rows + rows / 8 + 1024;
@@ -972,12 +871,7 @@ hipError_t cg_reserve(CgWork* cw, int rows) {
         (e = hipMalloc(&cw->u32, f)))
         return e;
     cw->cap = cap;
-    for (int k = 0; k < 2; k++)
-        for (int j = 0; j < CgWork::kGraphSlots; j++) {
-            if (cw->graph[k][j]) hipGraphExecDestroy(cw->graph[k][j]);
-            cw->graph[k][j] = nullptr;
-            cw->graph_chunk[k][j] = 0;
-        }
+    for (int k = 0; k < 2; k++) drop_graphs(cw, k);
     return hipSuccess;
 }
 
@@ -1050,10 +944,36 @@ static void enqueue_chunk(CgWork* cw, const Sell& A, const IDX* col, const T* va
     }
 }
 
+// Entries a slot of the SELL slices holds per row, on average (rounded up).
+static int mean_width(const Sell& A) {
+    const size_t per = (size_t) 64 * (size_t) std::max(A.nslices, 1);
+    return (int) ((A.entries + per - 1) / per);
+}
+
 static bool all_done(const CgWork* cw) {
     for (int s = 0; s < cw->nseg; s++)
         if (!cw->host[s].done) return false;
     return true;
+}
+
+// Drops the captured graphs of a solver when anything they bake in changed.
+static void check_graphs(CgWork* cw, int which, const Sell& A, const void* val, const void* col, int idx16,
+                         const void* y, const void* r, const void* p, const void* s, const void* w, const void* u,
+                         size_t lds) {
+    const uintptr_t sig[CgWork::kSig] = {
+        (uintptr_t) val,         (uintptr_t) col,          (uintptr_t) A.anc,       (uintptr_t) A.slice_off,
+        (uintptr_t) A.dgl,       (uintptr_t) y,            (uintptr_t) r,           (uintptr_t) p,
+        (uintptr_t) s,           (uintptr_t) w,            (uintptr_t) u,           (uintptr_t) cw->part,
+        (uintptr_t) cw->sc,      (uintptr_t) cw->blk_off,  (uintptr_t) cw->row_off, (uintptr_t) A.rows_dev,
+        (uintptr_t) cw->nseg,    (uintptr_t) cw->total_blocks, (uintptr_t) idx16,
+        (uintptr_t) (cw->mg_on ? mg_generation(cw->mg) + 1 : 0), (uintptr_t) cw->mg_on,
+        (uintptr_t) (cw->mg_on && cw->fused), (uintptr_t) cw->step_cells, (uintptr_t) lds, (uintptr_t) cw->xch.w,
+        (uintptr_t) cw->xch.part, (uintptr_t) cw->xch.w_half, (uintptr_t) cw->xch.p_half,
+        (uintptr_t) (lds ? 1 + (mean_width(A) <= 16) : 0)};
+    if (std::memcmp(sig, cw->graph_sig[which], sizeof(sig)) == 0) return;
+    drop_graphs(cw, which);
+    std::memcpy(cw->graph_sig[which], sig, sizeof(sig));
+    cw->graph_rebuilds++;
 }
 
 // Runs chunks of CG iterations (each a captured graph, or enqueued directly)
@@ -1068,25 +988,8 @@ static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* c
     const int idx16 = sizeof(IDX) == 4 ? 0 : (static_cast<IDX>(-1) < 0 ? 1 : 2);
     const size_t sbytes = sizeof(CgScalars) * (size_t) cw->nseg;
     hipError_t e;
-    if (o.use_graph) {
-        const uintptr_t sig[CgWork::kSig] = {
-            (uintptr_t) val,         (uintptr_t) col,          (uintptr_t) A.anc,       (uintptr_t) A.slice_off,
-            (uintptr_t) A.dgl,       (uintptr_t) y,            (uintptr_t) r,           (uintptr_t) p,
-            (uintptr_t) s,           (uintptr_t) w,            (uintptr_t) u_vec<T>(cw), (uintptr_t) cw->part,
-            (uintptr_t) cw->sc,      (uintptr_t) cw->blk_off,  (uintptr_t) cw->row_off, (uintptr_t) A.rows_dev,
-            (uintptr_t) cw->nseg,    (uintptr_t) cw->total_blocks, (uintptr_t) idx16,
-            (uintptr_t) (cw->mg_on ? mg_generation(cw->mg) + 1 : 0), (uintptr_t) cw->mg_on,
-            (uintptr_t) (cw->mg_on && cw->fused), (uintptr_t) cw->step_cells, 0};
-        if (std::memcmp(sig, cw->graph_sig[which], sizeof(sig)) != 0) {
-            for (int j = 0; j < CgWork::kGraphSlots; j++) {
-                if (cw->graph[which][j]) hipGraphExecDestroy(cw->graph[which][j]);
-                cw->graph[which][j] = nullptr;
-                cw->graph_chunk[which][j] = 0;
-            }
-            std::memcpy(cw->graph_sig[which], sig, sizeof(sig));
-            cw->graph_rebuilds++;
-        }
-    }
+    if (o.use_graph)
+        check_graphs(cw, which, A, val, col, idx16, y, r, p, s, w, u_vec<T>(cw), 0);
     int launched = 0, grow = 2;
     for (;;) {
         int chunk = interval;
@@ -1138,6 +1041,129 @@ static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* c
     }
 }
 
+// The whole Jacobi-scaled CG in one launch (resident.hip), for systems whose
+// blocks hold at most one row a thread and are no more than the CUs.  An
+// iteration costs 2.5-4 us that way against 8-11 us for the two kernels of a
+// chunk graph; beyond one block a CU (131k rows at 256 CUs) the two kernels
+// are bound by their bytes.  *ran: the solve was run and cw->host holds its
+// scalars; false: the caller takes the chunks (from a fresh start if
+// *restart: some segment's iterate may have been written).
+static hipError_t resident_reserve(CgWork* cw, int rows, hipStream_t st) {
+    const size_t w = 2 * (size_t) rows, p = 6 * (size_t) cw->total_blocks;  // FP64: two words a value
+    hipError_t e;
+    if (w > cw->xch.w_half) {
+        hipFree(cw->xch.w);
+        cw->xch.w = nullptr;
+        cw->xch.w_half = 0;
+        const size_t cap = w + w / 8 + 1024;
+        if ((e = hipMalloc(&cw->xch.w, 2 * cap * sizeof(unsigned long long)))) return e;
+        cw->xch.w_half = cap;
+        if ((e = fill_int((int*) cw->xch.w, 0, 4 * cap, st))) return e;
+    }
+    if (p > cw->xch.p_half) {
+        hipFree(cw->xch.part);
+        cw->xch.part = nullptr;
+        cw->xch.p_half = 0;
+        const size_t cap = p + 6 * 64;
+        if ((e = hipMalloc(&cw->xch.part, 2 * cap * sizeof(unsigned long long)))) return e;
+        cw->xch.p_half = cap;
+        if ((e = fill_int((int*) cw->xch.part, 0, 4 * cap, st))) return e;
+    }
+    return hipSuccess;
+}
+
+static size_t resident_fits(const CgWork* cw, int tsize) {
+    if (cw->mg_on || cw->total_blocks > cw->res_blocks) return 0;
+    int most = 0;
+    for (int k = 0; k < cw->nseg; k++) {
+        const int rows = cw->h_row[k + 1] - cw->h_row[k], nb = cw->h_blk[k + 1] - cw->h_blk[k];
+        if (((rows + nb - 1) / nb + 63) / 64 * 64 > kCgBlock) return 0;
+        most = std::max(most, rows);
+    }
+    return resident_lds(most, tsize);
+}
+
+static hipError_t upload_scalars(CgWork* cw, hipStream_t st);
+
+template <typename T, typename IDX, typename P>
+static hipError_t run_resident(CgWork* cw, int which, const Sell& A, const IDX* col, const T* val, T* y, T* r, T* p,
+                               T* s, T* w, const mps_solver_options& o, size_t lds, P&& prep, hipStream_t st,
+                               bool* ran, bool* restart) {
+    *ran = *restart = false;
+    std::atomic<int>& flight = g_res_in_flight[cw->res_dev];
+    const int want = cw->total_blocks;
+    if (flight.fetch_add(want) + want > cw->res_blocks) {
+        flight.fetch_sub(want);
+        return hipSuccess;
+    }
+    hipError_t e = hipSuccess;
+    const int idx16 = sizeof(IDX) == 4 ? 0 : (static_cast<IDX>(-1) < 0 ? 1 : 2);
+    const unsigned shape = 1u << (4 * idx16 + 2 * (int) (sizeof(T) == 8) + (int) (mean_width(A) <= 16));
+    if (!(cw->res_ready & shape)) {
+        e = resident_prepare<T, IDX>(mean_width(A));
+        cw->res_ready |= shape;
+    }
+    if (!e) e = resident_reserve(cw, A.rows, st);
+    if (!e) {
+        // this launch's tags: a range none of its words has held
+        unsigned span = 0;
+        for (int k = 0; k < cw->nseg; k++) span = std::max(span, (unsigned) cw->host[k].max_iter + 4u);
+        if (cw->tag > 0xffffffffu - span) {
+            cw->tag = 0;
+            e = fill_int((int*) cw->xch.w, 0, 4 * cw->xch.w_half, st);
+            if (!e) e = fill_int((int*) cw->xch.part, 0, 4 * cw->xch.p_half, st);
+        }
+        for (int k = 0; k < cw->nseg; k++) cw->host[k].tag0 = cw->tag;
+        cw->tag += span;
+    }
+    if (!e) e = upload_scalars(cw, st);
+    if (!e) prep();
+    auto go = [&]() {
+        return resident_launch<T, IDX>(cw->seg(), want, A.slice_off, col, A.anc, val, r, y, A.dgl, cw->sc, cw->xch,
+                                       mean_width(A), lds, st);
+    };
+    if (!e && o.use_graph) {
+        check_graphs(cw, which, A, val, col, idx16, y, r, p, s, w, u_vec<T>(cw), lds);
+        if (!cw->res_graph[which]) {
+            hipGraph_t gph;
+            e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
+            if (!e) {
+                const hipError_t le = go();
+                e = hipStreamEndCapture(st, &gph);
+                if (!e && le) {
+                    hipGraphDestroy(gph);
+                    e = le;
+                }
+            }
+            if (!e) {
+                e = hipGraphInstantiate(&cw->res_graph[which], gph, nullptr, nullptr, 0);
+                hipGraphDestroy(gph);
+                cw->graph_captures++;
+            }
+        }
+        if (!e) e = hipGraphLaunch(cw->res_graph[which], st);
+    } else if (!e) {
+        e = go();
+    }
+    if (!e) {
+        const MailSrc src{cw->sc, (int) (sizeof(CgScalars) * (size_t) cw->nseg)};
+        e = mailbox_read(cw->mb, &src, 1, cw->host, st);
+    }
+    flight.fetch_sub(want);
+    if (e) return e;
+    bool bail = false;
+    int it = 0;
+    for (int k = 0; k < cw->nseg; k++) {
+        bail = bail || cw->host[k].bail;
+        it = std::max(it, cw->host[k].fin);
+    }
+    cw->launched += it;
+    if (bail) cw->res_blocks = 0;  // a halo too large or CUs held by others: this handle stays with the chunks
+    *ran = !bail;
+    *restart = bail;
+    return hipSuccess;
+}
+
 static hipError_t upload_scalars(CgWork* cw, hipStream_t st) {
     return hipMemcpyAsync(cw->sc, cw->host, sizeof(CgScalars) * (size_t) cw->nseg, hipMemcpyHostToDevice, st);
 }
@@ -1170,21 +1196,41 @@ static void launch_residual(CgWork* cw, const Sell& A, hipStream_t st) {
 
 // `solve`: index of this solve within the step (0 for the FP64 CG, the
 // refinement for the inner CG); the last step's iteration count of the same
-// solve sizes the chunks.
-template <typename T, bool WEIGHTED>
+// solve sizes the chunks.  cw->host holds the scalars to start from: they
+// are uploaded here, then prep() enqueues what follows them.  fresh() puts
+// the start's vectors back after a resident launch that gave up.
+template <typename T, typename IDX, bool WEIGHTED, typename P, typename F>
+static hipError_t run_cg_idx(CgWork* cw, int which, const Sell& A, const IDX* col, const T* val, T* y, T* r, T* p,
+                             T* s, T* w, const mps_solver_options& o, int pred, P&& prep, F&& fresh,
+                             hipStream_t st) {
+    hipError_t e;
+    if (const size_t lds = resident_fits(cw, (int) sizeof(T))) {
+        const std::vector<CgScalars> start(cw->host, cw->host + cw->nseg);
+        bool ran, restart;
+        e = run_resident<T, IDX>(cw, which, A, col, val, y, r, p, s, w, o, lds, prep, st, &ran, &restart);
+        if (e || ran) return e;
+        if (restart && (e = fresh())) return e;
+        std::copy(start.begin(), start.end(), cw->host);
+    }
+    if ((e = upload_scalars(cw, st))) return e;
+    prep();
+    return run_cg_loop<T, IDX, WEIGHTED>(cw, which, A, col, val, y, r, p, s, w, o, pred, st);
+}
+
+template <typename T, bool WEIGHTED, typename P, typename F>
 static hipError_t run_cg(CgWork* cw, int which, int solve, const Sell& A, const T* val, T* y, T* r, T* p, T* s, T* w,
-                         const mps_solver_options& o, hipStream_t st) {
+                         const mps_solver_options& o, P&& prep, F&& fresh, hipStream_t st) {
     const int slot = solve < CgWork::kPredSolves ? solve : CgWork::kPredSolves - 1;
     int* const last = &cw->pred[cw->pred_bank][which][slot];
     const int pred = cw->predict ? *last : 0;
     hipError_t e;
     if (A.use16 && A.dim == 3)
-        e = run_cg_loop<T, unsigned short, WEIGHTED>(cw, which, A, (const unsigned short*) A.dcol, val, y, r, p, s, w, o,
-                                                     pred, st);
+        e = run_cg_idx<T, unsigned short, WEIGHTED>(cw, which, A, (const unsigned short*) A.dcol, val, y, r, p, s, w, o,
+                                                    pred, prep, fresh, st);
     else if (A.use16)
-        e = run_cg_loop<T, short, WEIGHTED>(cw, which, A, A.dcol, val, y, r, p, s, w, o, pred, st);
+        e = run_cg_idx<T, short, WEIGHTED>(cw, which, A, A.dcol, val, y, r, p, s, w, o, pred, prep, fresh, st);
     else
-        e = run_cg_loop<T, int, WEIGHTED>(cw, which, A, A.col, val, y, r, p, s, w, o, pred, st);
+        e = run_cg_idx<T, int, WEIGHTED>(cw, which, A, A.col, val, y, r, p, s, w, o, pred, prep, fresh, st);
     if (e) return e;
     int it = 0;  // the segment that took longest sets the chunk
     for (int k = 0; k < cw->nseg; k++) it = std::max(it, cw->host[k].fin);
@@ -1236,8 +1282,11 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
         }
     }
 
-    hipLaunchKernelGGL(k_cg_init, gr, bl, 0, st, sg, A.row_slot, h.id, b_s, o.warm_start ? pprev_id : nullptr,
-                       o.warm_start == 2 ? pprev2_id : nullptr, A.sdiag, cw->y, cw->bh, cw->part);
+    auto init_y = [&]() {
+        hipLaunchKernelGGL(k_cg_init, gr, bl, 0, st, sg, A.row_slot, h.id, b_s, o.warm_start ? pprev_id : nullptr,
+                           o.warm_start == 2 ? pprev2_id : nullptr, A.sdiag, cw->y, cw->bh, cw->part);
+    };
+    init_y();
     // ||b||^2 into red[2], then the initial residual: one read for both
     // (and for the multigrid setup's stencil check)
     hipLaunchKernelGGL((k_reduce_parts<1, 2>), dim3(nseg), dim3(kBlock), 0, st, sg, cw->part, cw->sc);
@@ -1270,14 +1319,16 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
     // are discarded for such segments
     bool any_zero = false;
     for (int s = 0; s < nseg; s++) any_zero |= bn2[s] == 0.0;
+    auto zero_y = [&]() -> hipError_t {
+        if (!any_zero) return hipSuccess;
+        if (nseg == 1) return fill_double(cw->y, 0.0, (size_t) rows, st);
+        for (int s = 0; s < nseg; s++)
+            if (bn2[s] == 0.0 && segrows[s] > 0)
+                if (const hipError_t ze = fill_double(cw->y + cw->h_row[s], 0.0, (size_t) segrows[s], st)) return ze;
+        return hipSuccess;
+    };
     if (any_zero) {
-        if (nseg == 1) {
-            if ((e = fill_double(cw->y, 0.0, (size_t) rows, st))) return e;
-        } else {
-            for (int s = 0; s < nseg; s++)
-                if (bn2[s] == 0.0 && segrows[s] > 0)
-                    if ((e = fill_double(cw->y + cw->h_row[s], 0.0, (size_t) segrows[s], st))) return e;
-        }
+        if ((e = zero_y())) return e;
         launch_residual(cw, A, st);
         if ((e = reduce_and_read(cw, 2, st))) return e;
         for (int s = 0; s < nseg; s++) rho2[s] = cw->host[s].red[1];
@@ -1308,9 +1359,16 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
                 cw->host[s] = z;
             }
             if (!any) break;
-            if ((e = upload_scalars(cw, st))) return e;
+            auto fresh = [&]() -> hipError_t {
+                if (pass == 0) {
+                    init_y();
+                    if (const hipError_t ze = zero_y()) return ze;
+                }
+                launch_residual(cw, A, st);  // of whatever iterate y now holds
+                return hipGetLastError();
+            };
             if ((e = run_cg<double, true>(cw, 0, pass, A, A.val64, cw->y, cw->r64, cw->p64, cw->s64, cw->w64, o,
-                                          st)))
+                                          [] {}, fresh, st)))
                 return e;
             for (int s = 0; s < nseg; s++)
                 if (ran[s]) total_it[s] += cw->host[s].fin;
@@ -1333,7 +1391,11 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
             for (int s = 0; s < nseg; s++)
                 active = active || (!conv[s] && refinements[s] < max_ref && total_it[s] < max_it[s]);
             if (!active) break;
-            hipLaunchKernelGGL(k_inner_init, gr, bl, 0, st, sg, cw->r64, cw->r32, cw->e32, cw->part);
+            auto inner_init = [&]() -> hipError_t {
+                hipLaunchKernelGGL(k_inner_init, gr, bl, 0, st, sg, cw->r64, cw->r32, cw->e32, cw->part);
+                return hipGetLastError();
+            };
+            if ((e = inner_init())) return e;
             std::vector<int> run(nseg, 0);
             for (int s = 0; s < nseg; s++) {
                 CgScalars z{};
@@ -1350,10 +1412,11 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
                 z.done = run[s] ? 0 : 1;
                 cw->host[s] = z;
             }
-            if ((e = upload_scalars(cw, st))) return e;
-            hipLaunchKernelGGL(k_inner_prep, dim3(nseg), dim3(kBlock), 0, st, sg, cw->part, cw->sc);
+            auto inner_prep = [&] {
+                hipLaunchKernelGGL(k_inner_prep, dim3(nseg), dim3(kBlock), 0, st, sg, cw->part, cw->sc);
+            };
             if ((e = run_cg<float, false>(cw, 1, round, A, A.val32, cw->e32, cw->r32, cw->p32, cw->s32, cw->w32, o,
-                                          st)))
+                                          inner_prep, inner_init, st)))
                 return e;
             for (int s = 0; s < nseg; s++)
                 if (run[s]) total_it[s] += cw->host[s].fin;
