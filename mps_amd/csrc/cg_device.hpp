@@ -53,13 +53,13 @@ struct BlockRows {
     int r0, r1;          // rows of this block
 };
 
-// Row range of this block: contiguous within the segment, whole multiples of
+// Row range of a block: contiguous within the segment, whole multiples of
 // 64 rows from the segment start, XCD-grouped.
-__device__ __forceinline__ BlockRows block_rows(const Seg& sg) {
+__device__ __forceinline__ BlockRows block_rows(const Seg& sg, int block) {
     BlockRows br;
-    br.seg = seg_of_block(sg, blockIdx.x);
+    br.seg = seg_of_block(sg, block);
     br.b0 = sg.blk_off[br.seg];
-    br.v = blockIdx.x - br.b0;
+    br.v = block - br.b0;
     br.nb = sg.blk_off[br.seg + 1] - br.b0;
     const int base = sg.row_off[br.seg];
     const int rows = sg.row_off[br.seg + 1] - base;
@@ -72,6 +72,82 @@ __device__ __forceinline__ BlockRows block_rows(const Seg& sg) {
     if (br.r0 > end) br.r0 = end;
     return br;
 }
+__device__ __forceinline__ BlockRows block_rows(const Seg& sg) { return block_rows(sg, blockIdx.x); }
+
+// a of the lane CTRL places up in the row of 16 (0 past its end).
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double a) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(a), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(a), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+
+// Sum over the wavefront by the tree a += a[lane + 32], + 16, ... + 1, valid
+// in lane 0: the sums of a __shfl_down loop bit for bit, with register moves
+// (lane swaps of gfx950 for 32 and 16, DPP row shifts for 8 to 1) in place of
+// LDS permutes, whose latency is several times an add's.
+__device__ __forceinline__ double wave_sum(double a) {
+    {
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(a), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(a), false, false);
+        a += __hiloint2double((int) hi[1], (int) lo[1]);
+    }
+    {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(a), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(a), false, false);
+        a += __hiloint2double((int) hi[1], (int) lo[1]);
+    }
+    a += dpp_f64<0x108>(a);
+    a += dpp_f64<0x104>(a);
+    a += dpp_f64<0x102>(a);
+    a += dpp_f64<0x101>(a);
+    return a;
+}
+
+// wave_sum of three values at once: a's sum in lane 0, b's in lane 32, c's in
+// lane 16.  The first two levels' lane swaps put different values into the
+// halves and rows that a single sum leaves idle (after the level of 32 a sum
+// lives in half the lanes, after 16 in a quarter), so three trees cost little
+// more than one; each value is still added in the order of its own tree.
+__device__ __forceinline__ double wave_sum3(double a, double b, double c) {
+    auto swap_add32 = [](double x, double y) {  // x[i] + x[i + 32] below lane 32, y's above
+        const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(x), __double2loint(y), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(x), __double2hiint(y), false, false);
+        return __hiloint2double((int) hi[0], (int) lo[0]) + __hiloint2double((int) hi[1], (int) lo[1]);
+    };
+    const double ab = swap_add32(a, b), cc = swap_add32(c, 0.0);
+    double t;
+    {
+        const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(ab), __double2loint(cc), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(ab), __double2hiint(cc), false, false);
+        t = __hiloint2double((int) hi[0], (int) lo[0]) + __hiloint2double((int) hi[1], (int) lo[1]);
+    }
+    t += dpp_f64<0x108>(t);
+    t += dpp_f64<0x104>(t);
+    t += dpp_f64<0x102>(t);
+    t += dpp_f64<0x101>(t);
+    return t;
+}
+// The value of wave_sum3 (0, 1, 2) a lane holds, -1 for none.
+__device__ __forceinline__ int sum3_of_lane(int lane) {
+    return lane == 0 ? 0 : (lane == 32 ? 1 : (lane == 16 ? 2 : -1));
+}
+
+// Each wavefront's sums of NV values into red[wavefront * NV + k].
+template <int NV>
+__device__ __forceinline__ void wave_partials(const double (&v)[NV], double* red) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if constexpr (NV == 3) {
+        const double t = wave_sum3(v[0], v[1], v[2]);
+        const int k = sum3_of_lane(lane);
+        if (k >= 0) red[w * 3 + k] = t;
+    } else {
+        for (int k = 0; k < NV; k++) {
+            const double a = wave_sum(v[k]);
+            if (lane == 0) red[w * NV + k] = a;
+        }
+    }
+}
 
 // Fixed-order sum of NV interleaved partials (part[b*NV + k], b < nb) in every
 // block; result broadcast to all threads.
@@ -82,11 +158,7 @@ __device__ __forceinline__ void reduce_partials(const double* __restrict__ part,
     for (int k = 0; k < NV; k++) acc[k] = 0.0;
     for (int b = threadIdx.x; b < nb; b += blockDim.x)
         for (int k = 0; k < NV; k++) acc[k] += part[(size_t) NV * b + k];
-    for (int k = 0; k < NV; k++) {
-        double a = acc[k];
-        for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-        if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * NV + k] = a;
-    }
+    wave_partials<NV>(acc, red);
     __syncthreads();
     for (int k = 0; k < NV; k++) {
         double t = 0.0;
@@ -98,11 +170,7 @@ __device__ __forceinline__ void reduce_partials(const double* __restrict__ part,
 
 template <int NV>
 __device__ __forceinline__ void write_partials(const double (&v)[NV], double* __restrict__ part, double* red) {
-    for (int k = 0; k < NV; k++) {
-        double a = v[k];
-        for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-        if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * NV + k] = a;
-    }
+    wave_partials<NV>(v, red);
     __syncthreads();
     if (threadIdx.x < NV) {
         double t = 0.0;
@@ -160,24 +228,34 @@ __device__ __forceinline__ T sell_row(const int* __restrict__ slice_pos, const I
 // Exchange memory of the resident CG's workgroups: tagged words (a 32-bit
 // value below a 32-bit tag) in two alternating halves.
 struct CgExchange {
-    unsigned long long* w;     // 2 x w_half: A r of every row
-    unsigned long long* part;  // 2 x p_half: 3 partial sums of every block
-    size_t w_half, p_half;
-    int halo_max;              // most halo rows a block takes (resident_halo_rows() at most)
+    unsigned long long* w;     // 2 halves x 2 words x w_rows: A r of every row
+    unsigned long long* part;  // 2 halves x p_sums places: 3 partial sums of every block or wavefront
+    size_t w_rows, p_sums;
+    int halo_max;              // lowers the halo rows a workgroup takes (tests)
 };
-// LDS the kernel needs for segments of at most max_rows rows; 0 if it cannot
-// take them.
-size_t resident_lds(int max_rows, int tsize);
-int resident_halo_rows();
-// Lets the kernel of this shape use its LDS (once per device before a launch).
+// Shape of a launch: workgroups per block of the layout (1 or kResSplit),
+// matrix entries a thread holds in registers, dynamic LDS.
+constexpr int kResSplit = 4;
+struct ResidentShape {
+    int split;  // 0: the kernel does not take this system
+    int emax;
+    size_t lds;
+};
+// The shape for segments of at most max_rows rows in at most max_nb blocks,
+// total_blocks in all, with at most `most` workgroups at once.
+ResidentShape resident_shape(int max_rows, int max_nb, int total_blocks, int mean_width, int most, int tsize);
+// Places for partial sums (CgExchange::p_sums) a launch needs.
+size_t resident_sums(int total_blocks);
+size_t resident_sum_words(size_t p_sums);  // words both halves take
+// Lets the kernel of this shape use its LDS (once before its first launch).
 template <typename T, typename IDX>
-hipError_t resident_prepare(int mean_width);
+hipError_t resident_prepare(const ResidentShape& s);
 // Enqueues the whole CG (every iteration up to each segment's stop) as one
-// launch of total_blocks workgroups, one per block of the layout.  All of
-// them must be able to run at once.
+// launch of split * total_blocks workgroups.  All of them must be able to run
+// at once.
 template <typename T, typename IDX>
-hipError_t resident_launch(const Seg& sg, int total_blocks, const int* slice_off, const IDX* col, const int* anc,
-                           const T* val, const T* r, T* y, const double* dgl, CgScalars* sc, const CgExchange& x,
-                           int mean_width, size_t lds, hipStream_t st);
+hipError_t resident_launch(const ResidentShape& s, const Seg& sg, int total_blocks, const int* slice_off,
+                           const IDX* col, const int* anc, const T* val, const T* r, T* y, const double* dgl,
+                           CgScalars* sc, const CgExchange& x, hipStream_t st);
 
 }  // namespace mps

@@ -781,9 +781,8 @@ CgWork* cg_create() {
     // MPS_AMD_CG_RESIDENT_HALO lowers the halo rows a block of the resident
     // CG takes, so that a launch gives up and the solve runs by launches
     // (tests; results unchanged)
-    cw->xch.halo_max = resident_halo_rows();
-    if (const char* hm = getenv("MPS_AMD_CG_RESIDENT_HALO"))
-        cw->xch.halo_max = std::min(cw->xch.halo_max, std::max(atoi(hm), 0));
+    cw->xch.halo_max = 1 << 30;
+    if (const char* hm = getenv("MPS_AMD_CG_RESIDENT_HALO")) cw->xch.halo_max = std::max(atoi(hm), 0);
     return cw;
 }
 
@@ -959,7 +958,7 @@ static bool all_done(const CgWork* cw) {
 // Drops the captured graphs of a solver when anything they bake in changed.
 static void check_graphs(CgWork* cw, int which, const Sell& A, const void* val, const void* col, int idx16,
                          const void* y, const void* r, const void* p, const void* s, const void* w, const void* u,
-                         size_t lds) {
+                         const ResidentShape& shape) {
     const uintptr_t sig[CgWork::kSig] = {
         (uintptr_t) val,         (uintptr_t) col,          (uintptr_t) A.anc,       (uintptr_t) A.slice_off,
         (uintptr_t) A.dgl,       (uintptr_t) y,            (uintptr_t) r,           (uintptr_t) p,
@@ -967,9 +966,9 @@ static void check_graphs(CgWork* cw, int which, const Sell& A, const void* val, 
         (uintptr_t) cw->sc,      (uintptr_t) cw->blk_off,  (uintptr_t) cw->row_off, (uintptr_t) A.rows_dev,
         (uintptr_t) cw->nseg,    (uintptr_t) cw->total_blocks, (uintptr_t) idx16,
         (uintptr_t) (cw->mg_on ? mg_generation(cw->mg) + 1 : 0), (uintptr_t) cw->mg_on,
-        (uintptr_t) (cw->mg_on && cw->fused), (uintptr_t) cw->step_cells, (uintptr_t) lds, (uintptr_t) cw->xch.w,
-        (uintptr_t) cw->xch.part, (uintptr_t) cw->xch.w_half, (uintptr_t) cw->xch.p_half,
-        (uintptr_t) (lds ? 1 + (mean_width(A) <= 16) : 0)};
+        (uintptr_t) (cw->mg_on && cw->fused), (uintptr_t) cw->step_cells, (uintptr_t) shape.lds, (uintptr_t) cw->xch.w,
+        (uintptr_t) cw->xch.part, (uintptr_t) cw->xch.w_rows, (uintptr_t) cw->xch.p_sums,
+        (uintptr_t) (64 * shape.split + shape.emax)};
     if (std::memcmp(sig, cw->graph_sig[which], sizeof(sig)) == 0) return;
     drop_graphs(cw, which);
     std::memcpy(cw->graph_sig[which], sig, sizeof(sig));
@@ -989,7 +988,7 @@ static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* c
     const size_t sbytes = sizeof(CgScalars) * (size_t) cw->nseg;
     hipError_t e;
     if (o.use_graph)
-        check_graphs(cw, which, A, val, col, idx16, y, r, p, s, w, u_vec<T>(cw), 0);
+        check_graphs(cw, which, A, val, col, idx16, y, r, p, s, w, u_vec<T>(cw), ResidentShape{});
     int launched = 0, grow = 2;
     for (;;) {
         int chunk = interval;
@@ -1043,65 +1042,67 @@ static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* c
 
 // The whole Jacobi-scaled CG in one launch (resident.hip), for systems whose
 // blocks hold at most one row a thread and are no more than the CUs.  An
-// iteration costs 2.5-4 us that way against 8-11 us for the two kernels of a
+// iteration costs 1.5-3.6 us that way against 8-11 us for the two kernels of a
 // chunk graph; beyond one block a CU (131k rows at 256 CUs) the two kernels
 // are bound by their bytes.  *ran: the solve was run and cw->host holds its
 // scalars; false: the caller takes the chunks (from a fresh start if
 // *restart: some segment's iterate may have been written).
 static hipError_t resident_reserve(CgWork* cw, int rows, hipStream_t st) {
-    const size_t w = 2 * (size_t) rows, p = 6 * (size_t) cw->total_blocks;  // FP64: two words a value
+    const size_t w = (size_t) rows, p = resident_sums(cw->total_blocks);
     hipError_t e;
-    if (w > cw->xch.w_half) {
+    if (w > cw->xch.w_rows) {
         hipFree(cw->xch.w);
         cw->xch.w = nullptr;
-        cw->xch.w_half = 0;
+        cw->xch.w_rows = 0;
         const size_t cap = w + w / 8 + 1024;
-        if ((e = hipMalloc(&cw->xch.w, 2 * cap * sizeof(unsigned long long)))) return e;
-        cw->xch.w_half = cap;
-        if ((e = fill_int((int*) cw->xch.w, 0, 4 * cap, st))) return e;
+        if ((e = hipMalloc(&cw->xch.w, 4 * cap * sizeof(unsigned long long)))) return e;
+        cw->xch.w_rows = cap;
+        if ((e = fill_int((int*) cw->xch.w, 0, 8 * cap, st))) return e;
     }
-    if (p > cw->xch.p_half) {
+    if (p > cw->xch.p_sums) {
         hipFree(cw->xch.part);
         cw->xch.part = nullptr;
-        cw->xch.p_half = 0;
-        const size_t cap = p + 6 * 64;
-        if ((e = hipMalloc(&cw->xch.part, 2 * cap * sizeof(unsigned long long)))) return e;
-        cw->xch.p_half = cap;
-        if ((e = fill_int((int*) cw->xch.part, 0, 4 * cap, st))) return e;
+        cw->xch.p_sums = 0;
+        const size_t cap = p + 64;
+        if ((e = hipMalloc(&cw->xch.part, resident_sum_words(cap) * sizeof(unsigned long long)))) return e;
+        cw->xch.p_sums = cap;
+        if ((e = fill_int((int*) cw->xch.part, 0, 2 * resident_sum_words(cap), st))) return e;
     }
     return hipSuccess;
 }
 
-static size_t resident_fits(const CgWork* cw, int tsize) {
-    if (cw->mg_on || cw->total_blocks > cw->res_blocks) return 0;
-    int most = 0;
+static ResidentShape resident_fits(const CgWork* cw, const Sell& A, int tsize) {
+    if (cw->mg_on || cw->res_blocks == 0) return ResidentShape{};
+    int most = 0, most_nb = 0;
     for (int k = 0; k < cw->nseg; k++) {
         const int rows = cw->h_row[k + 1] - cw->h_row[k], nb = cw->h_blk[k + 1] - cw->h_blk[k];
-        if (((rows + nb - 1) / nb + 63) / 64 * 64 > kCgBlock) return 0;
+        if (((rows + nb - 1) / nb + 63) / 64 * 64 > kCgBlock) return ResidentShape{};
         most = std::max(most, rows);
+        most_nb = std::max(most_nb, nb);
     }
-    return resident_lds(most, tsize);
+    return resident_shape(most, most_nb, cw->total_blocks, mean_width(A), cw->res_blocks, tsize);
 }
 
 static hipError_t upload_scalars(CgWork* cw, hipStream_t st);
 
 template <typename T, typename IDX, typename P>
 static hipError_t run_resident(CgWork* cw, int which, const Sell& A, const IDX* col, const T* val, T* y, T* r, T* p,
-                               T* s, T* w, const mps_solver_options& o, size_t lds, P&& prep, hipStream_t st,
+                               T* s, T* w, const mps_solver_options& o, const ResidentShape& shape, P&& prep, hipStream_t st,
                                bool* ran, bool* restart) {
     *ran = *restart = false;
     std::atomic<int>& flight = g_res_in_flight[cw->res_dev];
-    const int want = cw->total_blocks;
+    const int want = shape.split * cw->total_blocks;
     if (flight.fetch_add(want) + want > cw->res_blocks) {
         flight.fetch_sub(want);
         return hipSuccess;
     }
     hipError_t e = hipSuccess;
     const int idx16 = sizeof(IDX) == 4 ? 0 : (static_cast<IDX>(-1) < 0 ? 1 : 2);
-    const unsigned shape = 1u << (4 * idx16 + 2 * (int) (sizeof(T) == 8) + (int) (mean_width(A) <= 16));
-    if (!(cw->res_ready & shape)) {
-        e = resident_prepare<T, IDX>(mean_width(A));
-        cw->res_ready |= shape;
+    const unsigned kernel = 1u << (8 * idx16 + 4 * (int) (sizeof(T) == 8) + 2 * (int) (shape.split > 1) +
+                                   (int) (shape.emax > 16));
+    if (!(cw->res_ready & kernel)) {
+        e = resident_prepare<T, IDX>(shape);
+        cw->res_ready |= kernel;
     }
     if (!e) e = resident_reserve(cw, A.rows, st);
     if (!e) {
@@ -1110,8 +1111,8 @@ static hipError_t run_resident(CgWork* cw, int which, const Sell& A, const IDX* 
         for (int k = 0; k < cw->nseg; k++) span = std::max(span, (unsigned) cw->host[k].max_iter + 4u);
         if (cw->tag > 0xffffffffu - span) {
             cw->tag = 0;
-            e = fill_int((int*) cw->xch.w, 0, 4 * cw->xch.w_half, st);
-            if (!e) e = fill_int((int*) cw->xch.part, 0, 4 * cw->xch.p_half, st);
+            e = fill_int((int*) cw->xch.w, 0, 8 * cw->xch.w_rows, st);
+            if (!e) e = fill_int((int*) cw->xch.part, 0, 2 * resident_sum_words(cw->xch.p_sums), st);
         }
         for (int k = 0; k < cw->nseg; k++) cw->host[k].tag0 = cw->tag;
         cw->tag += span;
@@ -1119,11 +1120,11 @@ static hipError_t run_resident(CgWork* cw, int which, const Sell& A, const IDX* 
     if (!e) e = upload_scalars(cw, st);
     if (!e) prep();
     auto go = [&]() {
-        return resident_launch<T, IDX>(cw->seg(), want, A.slice_off, col, A.anc, val, r, y, A.dgl, cw->sc, cw->xch,
-                                       mean_width(A), lds, st);
+        return resident_launch<T, IDX>(shape, cw->seg(), cw->total_blocks, A.slice_off, col, A.anc, val, r, y, A.dgl,
+                                       cw->sc, cw->xch, st);
     };
     if (!e && o.use_graph) {
-        check_graphs(cw, which, A, val, col, idx16, y, r, p, s, w, u_vec<T>(cw), lds);
+        check_graphs(cw, which, A, val, col, idx16, y, r, p, s, w, u_vec<T>(cw), shape);
         if (!cw->res_graph[which]) {
             hipGraph_t gph;
             e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
@@ -1204,10 +1205,11 @@ static hipError_t run_cg_idx(CgWork* cw, int which, const Sell& A, const IDX* co
                              T* s, T* w, const mps_solver_options& o, int pred, P&& prep, F&& fresh,
                              hipStream_t st) {
     hipError_t e;
-    if (const size_t lds = resident_fits(cw, (int) sizeof(T))) {
+    const ResidentShape shape = resident_fits(cw, A, (int) sizeof(T));
+    if (shape.split) {
         const std::vector<CgScalars> start(cw->host, cw->host + cw->nseg);
         bool ran, restart;
-        e = run_resident<T, IDX>(cw, which, A, col, val, y, r, p, s, w, o, lds, prep, st, &ran, &restart);
+        e = run_resident<T, IDX>(cw, which, A, col, val, y, r, p, s, w, o, shape, prep, st, &ran, &restart);
         if (e || ran) return e;
         if (restart && (e = fresh())) return e;
         std::copy(start.begin(), start.end(), cw->host);

@@ -14,15 +14,17 @@
 // The exchange is of tagged words: 32 bits of the value below a 32-bit tag,
 // stored and polled as relaxed device-scope 64-bit atomics.  A word carries
 // its own readiness, so it needs no flag, fence or counter after it, and one
-// store-to-load latency is the whole exchange (measured between 64 blocks
-// spread over the 8 XCDs: 2.3 us an iteration with the reductions, 3.0 us
-// between 256).  Two halves alternate: a block writes a half again only
+// store-to-load latency is the whole exchange (1.4-1.5 us between 2 to 64
+// workgroups spread over the 8 XCDs; on one XCD it is the same).  Two halves alternate: a block writes a half again only
 // after it has every block's partials of the iteration between, which each
 // block sends after it has read the half.
 //
 // Measured (2D, FP64, launches -> resident): 2,520 rows of 28 entries at
-// machine epsilon 3.87 -> 1.60 ms a step of ~280 iterations; 32k rows of 12,
-// ~21,500 iterations of a gradient evaluation 112 -> 59 ms.
+// machine epsilon 3.80 -> 1.28 ms a step of ~280 iterations; 32k rows of 12,
+// ~10,700 iterations of a gradient evaluation 111 -> 44 ms.  What an
+// iteration spends now (2.4 GHz cycles, FP64, 64 blocks): row product and
+// wavefront sums 1700, exchange 3500 (one uncached store and load), adding
+// the sums up 900, three divisions 700, updates 800.
 //
 // Sums are taken in the order and with the arithmetic of the two kernels, so
 // the iterates are theirs bit for bit, and an ensemble member keeps its solo
@@ -39,10 +41,16 @@
 
 namespace mps {
 
-constexpr int kResHalo = 8;                           // halo rows a thread updates
-constexpr int kResHaloRows = kResHalo * kCgBlock;     // halo rows of a block at most
-constexpr int kResMaxRows = 131072;                   // rows of a segment (bits of the halo map)
-constexpr long long kResWait = 5000000;               // ticks of the 100 MHz clock a wait may take (50 ms)
+constexpr int kResHalo = 8;               // halo rows a thread updates
+constexpr int kResMaxRows = 131072;       // rows of a segment (bits of the halo map)
+constexpr long long kResWait = 5000000;   // ticks of the 100 MHz clock a wait may take (50 ms)
+constexpr int kResWaves = kCgBlock / 64;  // wavefronts of a block of the layout
+constexpr int kResMaxBlocks = 256;        // blocks of a segment
+constexpr int kResSplitSums = 128;        // wavefronts of a segment with split blocks
+// Words from one place of partial sums to the next: three doubles are six;
+// at eight a place has a 64-byte line to itself and is sent by one store of
+// six lanes.
+constexpr int kSumWords = 8;
 
 __device__ __forceinline__ void put_word(unsigned long long* p, unsigned v, unsigned tag) {
     __hip_atomic_store(p, ((unsigned long long) tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -50,20 +58,35 @@ __device__ __forceinline__ void put_word(unsigned long long* p, unsigned v, unsi
 __device__ __forceinline__ unsigned long long get_word(const unsigned long long* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// The word at a byte offset from a base that is the same in every lane.
+__device__ __forceinline__ unsigned long long get_word_at(const unsigned long long* base, unsigned bytes) {
+    return get_word((const unsigned long long*) ((const char*) base + bytes));
+}
 __device__ __forceinline__ unsigned tag_of(unsigned long long w) { return (unsigned) (w >> 32); }
 
-// A value of T in kWords<T> tagged words.
+// A value of T in kWords<T> tagged words, `stride` words apart: a word of all
+// rows, then the next, so that a wavefront's words share cache lines (these
+// accesses bypass the caches, every line is a request of its own).
 template <typename T>
 constexpr int kWords = (int) (sizeof(T) / 4);
 template <typename T>
-__device__ __forceinline__ void put_value(unsigned long long* p, T v, unsigned tag) {
+__device__ __forceinline__ void put_value(unsigned long long* p, size_t stride, T v, unsigned tag) {
     if constexpr (sizeof(T) == 8) {
         const unsigned long long b = (unsigned long long) __double_as_longlong(v);
         put_word(p, (unsigned) b, tag);
-        put_word(p + 1, (unsigned) (b >> 32), tag);
+        put_word(p + stride, (unsigned) (b >> 32), tag);
     } else {
         put_word(p, __float_as_uint(v), tag);
     }
+}
+// A wavefront's three sums as wave_sum3 leaves them (lanes 0, 32, 16), sent
+// by six lanes.
+__device__ __forceinline__ void send_sums(unsigned long long* p, double ws, unsigned tag) {
+    const int lane = threadIdx.x & 63;
+    const int from = lane >> 1 == 0 ? 0 : (lane >> 1 == 1 ? 32 : 16);
+    const int lo = __builtin_amdgcn_ds_bpermute(4 * from, __double2loint(ws));
+    const int hi = __builtin_amdgcn_ds_bpermute(4 * from, __double2hiint(ws));
+    if (lane < 6) put_word(p + lane, (unsigned) (lane & 1 ? hi : lo), tag);
 }
 template <typename T>
 __device__ __forceinline__ T value_of(const unsigned long long* w) {
@@ -87,62 +110,92 @@ struct Wait {
 
 // acc + sum of val[k] * x[idx[k]] in entry order, each product and sum
 // rounded by itself as sell_row does (contraction is off here).
+template <typename T>
+__device__ __forceinline__ T add_product(T acc, T v, T x) {
+    acc += v * x;
+    return acc;
+}
 template <typename T, int EMAX>
 __device__ __forceinline__ T resident_row(const T (&v)[EMAX], const unsigned (&ix)[EMAX / 2],
-                                          const T* __restrict__ x, int w, T acc) {
+                                          const T* __restrict__ x, T acc) {
+    T xv[EMAX];
 #pragma unroll
-    for (int k = 0; k < EMAX; k += 4) {
-        if (k < w) {
-            T xv[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const unsigned pair = ix[(k + q) / 2];
-                xv[q] = x[(k + q) & 1 ? pair >> 16 : pair & 0xffffu];
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) acc += v[k + q] * xv[q];  // entries past w: value 0, own row
-        }
+    for (int k = 0; k < EMAX; k++) {
+        const unsigned pair = ix[k / 2];
+        xv[k] = x[k & 1 ? pair >> 16 : pair & 0xffffu];
     }
+#pragma unroll
+    for (int k = 0; k < EMAX; k++) acc += v[k] * xv[k];  // entries past the row's: value 0, own row
     return acc;
 }
 
-template <typename T, typename IDX, int EMAX>
-__global__ void __launch_bounds__(kCgBlock) k_cg_resident(Seg sg, const int* __restrict__ slice_pos,
-                                                          const IDX* __restrict__ col, const int* __restrict__ anc,
-                                                          const T* __restrict__ val, const T* __restrict__ r_in,
-                                                          T* __restrict__ y_io, const double* __restrict__ dgl,
-                                                          CgScalars* scs, CgExchange X) {
+// BT rows a workgroup.  BT == kCgBlock: one workgroup a block of the layout;
+// it sends the block's three sums, and every workgroup adds the blocks' sums
+// up as k_cg_step does.  BT < kCgBlock: kCgBlock / BT workgroups a block, the
+// wavefronts' sums are sent, and every workgroup adds them up to the blocks'
+// sums first, in k_cg_apply's order.
+//
+// Every thread sends its own row and polls right after.  A wavefront's loads
+// and stores complete in order, so its first poll also waits for its stores'
+// acknowledgement; a load that bypasses the L2s takes as long anyway (2500
+// cycles) and mostly finds the others' words in that time.  Separate sending
+// and polling wavefronts were slower (2,520 rows 26.1 -> 30.5 ms per 20
+// steps): the poll sampled memory too early and had to be repeated.
+template <typename T, typename IDX, int EMAX, int BT>
+__global__ void __launch_bounds__(BT)
+    k_cg_resident(Seg sg, const int* __restrict__ slice_pos, const IDX* __restrict__ col, const int* __restrict__ anc,
+                  const T* __restrict__ val, const T* __restrict__ r_in, T* __restrict__ y_io,
+                  const double* __restrict__ dgl, CgScalars* scs, CgExchange X) {
 #pragma clang fp contract(fast)
-    static_assert(EMAX % 4 == 0, "entries are taken four at a time");
+    static_assert(EMAX % 2 == 0, "two places share a word");
     constexpr bool kWeighted = sizeof(T) == 8;  // the FP64 solve stops on the unscaled residual
-    constexpr int NW = kCgBlock / 64;
+    constexpr int NW = BT / 64;
+    constexpr int kSplit = kCgBlock / BT;
+    constexpr bool kByWave = kSplit > 1;
+    constexpr int kHaloRows = kResHalo * BT;
+    // sums sent per workgroup: its block's, or its wavefronts'; and the most
+    // a workgroup waits for
+    constexpr int kSent = kByWave ? NW : 1;
+    constexpr int kMaxSums = kByWave ? kResSplitSums : kResMaxBlocks;
+    constexpr int kPoll = kMaxSums * kSumWords / BT;  // words of them a thread polls
     extern __shared__ __align__(16) unsigned char smem[];
-    __shared__ double s_wave[3 * NW], s_red[3 * NW];
-    __shared__ int s_scan[NW + 1];
+    __shared__ __align__(16) unsigned s_sum[kMaxSums * 6];  // the doubles of all sums, 3 a place
+    __shared__ __align__(16) double s_wave[3][NW];
+    __shared__ int s_scan[NW];
     __shared__ int s_bad;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    const BlockRows br = block_rows(sg);
+    BlockRows br = block_rows(sg, blockIdx.x / kSplit);
     CgScalars* sc = scs + br.seg;
     if (block_uniform_done(sc)) return;
     const int base = sg.row_off[br.seg];
     const int rows = sg.row_off[br.seg + 1] - base;
     const int nb = br.nb;
+    if (kByWave) {  // this workgroup's share of the block
+        const int part = blockIdx.x % kSplit;
+        br.r0 = br.r0 + part * BT < br.r1 ? br.r0 + part * BT : br.r1;
+        br.r1 = br.r0 + BT < br.r1 ? br.r0 + BT : br.r1;
+    }
     const int own = br.r1 - br.r0;
+    const bool alone = !kByWave && nb == 1;  // the segment is this workgroup's
     const int words = (rows + 31) >> 5;
-    T* const x = (T*) smem;                                             // r: own rows, then the halo
-    unsigned* const bits = (unsigned*) (smem + sizeof(T) * (kCgBlock + kResHaloRows));
+    T* const x = (T*) smem;  // r: own rows, then the halo
+    unsigned* const bits = (unsigned*) (smem + sizeof(T) * (BT + kHaloRows));
     unsigned short* const pre = (unsigned short*) (bits + words);
-    int* const hcol = (int*) x;                                         // while the halo is listed
+    int* const hcol = (int*) x;  // while the halo is listed
     const unsigned tag0 = sc->tag0;
     const int max_iter = sc->max_iter;
     const double thr = sc->thr;
     const unsigned poison = tag0 + (unsigned) max_iter + 3u;
     const int row = br.r0 + tid;
     const bool live = tid < own;
+    // the sums this thread waits for, and where this workgroup's go
+    const int nsum = kByWave ? nb * kResWaves : nb;
+    const size_t sum0 = (size_t) br.b0 * (kByWave ? kResWaves : 1);
+    const size_t mine = (size_t) blockIdx.x * kSent;
 
-    // ---- the row's entries, and the halo: the rows of the segment outside
-    // the block that some entry names, numbered in row order
-    for (int i = tid; i < words; i += kCgBlock) bits[i] = 0;
+    // ---- the halo: the rows of the segment outside the workgroup's that
+    // some entry names, numbered in row order
+    for (int i = tid; i < words; i += BT) bits[i] = 0;
     if (tid == 0) s_bad = 0;
     int w = 0, lo = 0, hi = 0;
     size_t eb = 0;
@@ -153,17 +206,9 @@ __global__ void __launch_bounds__(kCgBlock) k_cg_resident(Seg sg, const int* __r
         eb = (size_t) s0 * 64 + (row & 63);
         sell_anchors<IDX>(anc, row, lo, hi);
     }
-    T v[EMAX];
     int c[EMAX];
 #pragma unroll
-    for (int k = 0; k < EMAX; k++) {
-        v[k] = (T) 0;
-        c[k] = row;
-        if (k < w) {
-            v[k] = val[eb + (size_t) k * 64];
-            c[k] = sell_col<IDX>(col, eb + (size_t) k * 64, row, lo, hi);
-        }
-    }
+    for (int k = 0; k < EMAX; k++) c[k] = k < w ? sell_col<IDX>(col, eb + (size_t) k * 64, row, lo, hi) : row;
     __syncthreads();
     auto mark = [&](int cc) {
         if (cc < br.r0 || cc >= br.r1) atomicOr(&bits[(cc - base) >> 5], 1u << ((cc - base) & 31));
@@ -175,7 +220,7 @@ __global__ void __launch_bounds__(kCgBlock) k_cg_resident(Seg sg, const int* __r
         for (int k = EMAX; k < w; k++) mark(sell_col<IDX>(col, eb + (size_t) k * 64, row, lo, hi));
     }
     __syncthreads();
-    const int per = (words + kCgBlock - 1) / kCgBlock;
+    const int per = (words + BT - 1) / BT;
     int cnt = 0;
     for (int i = 0; i < per; i++) {
         const int q = tid * per + i;
@@ -193,82 +238,80 @@ __global__ void __launch_bounds__(kCgBlock) k_cg_resident(Seg sg, const int* __r
         if (k < wid) off += s_scan[k];
         H += s_scan[k];
     }
-    const bool fits = H <= X.halo_max;  // block-uniform
+    auto leave = [&]() {  // every thread of the workgroup
+        if (tid == 0) atomicOr(&sc->bail, 1);
+        if (tid < 2 * kSent * kSumWords && !alone) {
+            const int half = tid / (kSent * kSumWords), at = tid % (kSent * kSumWords);
+            put_word(X.part + (size_t) half * kSumWords * X.p_sums + mine * kSumWords + at, 0u, poison);
+        }
+    };
+    if (H > kHaloRows || H > X.halo_max) {  // uniform in the workgroup
+        leave();
+        return;
+    }
+    for (int i = 0; i < per; i++) {
+        const int q = tid * per + i;
+        if (q >= words) break;
+        unsigned m = bits[q];
+        pre[q] = (unsigned short) off;
+        while (m) {
+            hcol[off++] = base + 32 * q + __builtin_ctz(m);
+            m &= m - 1;
+        }
+    }
+    __syncthreads();
     int hc[kResHalo];
     T hs[kResHalo];
-    if (fits) {
-        for (int i = 0; i < per; i++) {
-            const int q = tid * per + i;
-            if (q >= words) break;
-            unsigned m = bits[q];
-            pre[q] = (unsigned short) off;
-            while (m) {
-                hcol[off++] = base + 32 * q + __builtin_ctz(m);
-                m &= m - 1;
-            }
-        }
-        __syncthreads();
 #pragma unroll
-        for (int i = 0; i < kResHalo; i++) {
-            const int h = i * kCgBlock + tid;
-            hc[i] = h < H ? hcol[h] : -1;
-            hs[i] = (T) 0;
-        }
-        __syncthreads();
+    for (int i = 0; i < kResHalo; i++) {
+        const int h = i * BT + tid;
+        hc[i] = h < H ? hcol[h] : -1;
+        hs[i] = (T) 0;
     }
+    __syncthreads();
     // place in x of column cc
     auto place = [&](int cc) -> unsigned {
         if (cc >= br.r0 && cc < br.r1) return (unsigned) (cc - br.r0);
         const int q = cc - base;
-        return (unsigned) (kCgBlock + pre[q >> 5] + __popc(bits[q >> 5] & ((1u << (q & 31)) - 1u)));
+        return (unsigned) (BT + pre[q >> 5] + __popc(bits[q >> 5] & ((1u << (q & 31)) - 1u)));
     };
     unsigned ix[EMAX / 2];
+    T v[EMAX];
     T r = (T) 0, p = (T) 0, s = (T) 0, y = (T) 0;
     double dg = 0.0;
-    if (fits) {
 #pragma unroll
-        for (int k = 0; k < EMAX; k += 2) {
-            const unsigned a = live && k < w ? place(c[k]) : (unsigned) tid;
-            const unsigned b = live && k + 1 < w ? place(c[k + 1]) : (unsigned) tid;
-            ix[k / 2] = a | (b << 16);
-        }
-        if (live) {
-            r = r_in[row];
-            y = y_io[row];
-            if (kWeighted) dg = dgl[row];
-        }
-        x[tid] = r;
+    for (int k = 0; k < EMAX; k += 2) {
+        const unsigned a = live && k < w ? place(c[k]) : (unsigned) tid;
+        const unsigned b = live && k + 1 < w ? place(c[k + 1]) : (unsigned) tid;
+        ix[k / 2] = a | (b << 16);
+    }
 #pragma unroll
-        for (int i = 0; i < kResHalo; i++)
-            if (hc[i] >= 0) x[kCgBlock + i * kCgBlock + tid] = r_in[hc[i]];
-        __syncthreads();
+    for (int k = 0; k < EMAX; k++) v[k] = k < w ? val[eb + (size_t) k * 64] : (T) 0;
+    if (live) {
+        r = r_in[row];
+        y = y_io[row];
+        if (kWeighted) dg = dgl[row];
     }
-    auto leave = [&]() {  // block-uniform
-        if (tid == 0) atomicOr(&sc->bail, 1);
-        if (tid < 2 && nb > 1) put_word(X.part + (size_t) tid * X.p_half + (size_t) blockIdx.x * 6, 0u, poison);
-    };
-    if (!fits) {
-        leave();
-        return;
-    }
+    x[tid] = r;
+#pragma unroll
+    for (int i = 0; i < kResHalo; i++)
+        if (hc[i] >= 0) x[BT + i * BT + tid] = r_in[hc[i]];
+    __syncthreads();
 
     // ---- iterations
     double gam_old = 0.0, alp_old = 0.0;
     for (int it = 1;; it++) {
         const unsigned tag = tag0 + (unsigned) it;
-        unsigned long long* const xw = X.w + (size_t) (it & 1) * X.w_half;
-        unsigned long long* const xp = X.part + (size_t) (it & 1) * X.p_half;
+        unsigned long long* const xw = X.w + (size_t) (it & 1) * 2 * X.w_rows;
+        unsigned long long* const xp = X.part + (size_t) (it & 1) * kSumWords * X.p_sums;
         // A r of the own row (unit diagonal)
-        T ar = resident_row<T, EMAX>(v, ix, x, w, r);
+        T ar = resident_row<T, EMAX>(v, ix, x, r);
         for (int k = EMAX; k < w; k++) {
             const size_t e = eb + (size_t) k * 64;
-            const T one[4] = {val[e], (T) 0, (T) 0, (T) 0};
-            const unsigned at[2] = {place(sell_col<IDX>(col, e, row, lo, hi)) | ((unsigned) tid << 16),
-                                    (unsigned) tid | ((unsigned) tid << 16)};
-            ar = resident_row<T, 4>(one, at, x, 1, ar);
+            ar = add_product(ar, val[e], x[place(sell_col<IDX>(col, e, row, lo, hi))]);
         }
-        if (live && nb > 1) put_value<T>(xw + (size_t) row * kWords<T>, ar, tag);
-        // the block's partial sums: r.r, (A r).r and the stopping norm
+        if (live && !alone) put_value<T>(xw + row, X.w_rows, ar, tag);
+        // the wavefronts' partial sums: r.r, (A r).r and the stopping norm
         double part[3] = {0.0, 0.0, 0.0};
         if (live) {
             const double r2 = (double) r * (double) r;
@@ -276,96 +319,120 @@ __global__ void __launch_bounds__(kCgBlock) k_cg_resident(Seg sg, const int* __r
             part[1] += (double) ar * (double) r;
             part[2] += kWeighted ? dg * r2 : r2;
         }
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            double a = part[k];
-            for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-            if (lane == 0) s_wave[wid * 3 + k] = a;
+        const double ws = wave_sum3(part[0], part[1], part[2]);
+        const int k3 = sum3_of_lane(lane);
+        if (kByWave) {
+            send_sums(xp + (mine + wid) * kSumWords, ws, tag);
+        } else {
+            if (k3 >= 0) s_wave[k3][wid] = ws;
+            __syncthreads();
         }
-        __syncthreads();
         double sum[3];
-        T hw[kResHalo];
-        if (nb == 1) {
+        unsigned long long hm[kResHalo][kWords<T>];
+        if (alone) {
 #pragma unroll
             for (int k = 0; k < 3; k++) {
                 double t = 0.0;
-                for (int q = 0; q < NW; q++) t += s_wave[q * 3 + k];
+#pragma unroll
+                for (int q = 0; q < NW; q++) t += s_wave[k][q];
                 sum[k] = t;
             }
         } else {
-            if (tid < 3) {
+            if (!kByWave && tid < 6) {
                 double t = 0.0;
-                for (int q = 0; q < NW; q++) t += s_wave[q * 3 + tid];
-                put_value<double>(xp + (size_t) blockIdx.x * 6 + 2 * tid, t, tag);
+#pragma unroll
+                for (int q = 0; q < NW; q++) t += s_wave[tid >> 1][q];
+                put_word(xp + mine * kSumWords + tid, (unsigned) (tid & 1 ? __double2hiint(t) : __double2loint(t)), tag);
             }
+            // wait for the sums and for A r of the thread's halo rows
             bool bad = false;
-            double acc[3] = {0.0, 0.0, 0.0};
-            if (tid < nb) {
-                const unsigned long long* q = xp + (size_t) (br.b0 + tid) * 6;
-                unsigned long long m[6];
-                Wait wt;
-                for (;;) {
-                    bool ok = true;
-#pragma unroll
-                    for (int k = 0; k < 6; k++) m[k] = get_word(q + k);
-#pragma unroll
-                    for (int k = 0; k < 6; k++) ok = ok && tag_of(m[k]) == tag;
-                    if (ok) break;
-                    if (tag_of(m[0]) == poison || wt.expired()) {
-                        bad = true;
-                        break;
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < 3; k++) acc[k] += value_of<double>(m + 2 * k);
-            }
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                double a = acc[k];
-                for (int o = 32; o > 0; o >>= 1) a += __shfl_down(a, o, 64);
-                if (lane == 0) s_red[wid * 3 + k] = a;
-            }
-            // A r of the thread's halo rows
+            unsigned long long m[kPoll];
+            const bool sums = (tid & (kSumWords - 1)) < 6;
             {
                 Wait wt;
                 for (;;) {
                     bool ok = true;
 #pragma unroll
-                    for (int i = 0; i < kResHalo; i++) {
-                        if (hc[i] < 0) continue;
-                        unsigned long long m[kWords<T>];
+                    for (int i = 0; i < kPoll; i++)
+                        if (sums && i * BT + tid < nsum * kSumWords)
+                            m[i] = get_word_at(xp + sum0 * kSumWords + (size_t) i * BT, (unsigned) tid * 8u);
 #pragma unroll
-                        for (int k = 0; k < kWords<T>; k++) m[k] = get_word(xw + (size_t) hc[i] * kWords<T> + k);
+                    for (int i = 0; i < kResHalo; i++)
+                        if (i * BT < H && hc[i] >= 0) {
 #pragma unroll
-                        for (int k = 0; k < kWords<T>; k++) ok = ok && tag_of(m[k]) == tag;
-                        hw[i] = value_of<T>(m);
-                    }
+                            for (int k = 0; k < kWords<T>; k++)
+                                hm[i][k] = get_word_at(xw + (size_t) k * X.w_rows, (unsigned) hc[i] * 8u);
+                        }
+#pragma unroll
+                    for (int i = 0; i < kPoll; i++)
+                        if (sums && i * BT + tid < nsum * kSumWords) {
+                            ok = ok && tag_of(m[i]) == tag;
+                            bad = bad || tag_of(m[i]) == poison;
+                        }
+#pragma unroll
+                    for (int i = 0; i < kResHalo; i++)
+                        if (i * BT < H && hc[i] >= 0) {
+#pragma unroll
+                            for (int k = 0; k < kWords<T>; k++) ok = ok && tag_of(hm[i][k]) == tag;
+                        }
                     if (ok) break;
-                    if (wt.expired()) {
-                        bad = true;
-                        break;
-                    }
+                    bad = bad || wt.expired();
+                    if (bad) break;
                 }
+            }
+#pragma unroll
+            for (int i = 0; i < kPoll; i++) {
+                const int at = i * BT + tid;
+                if (sums && at < nsum * kSumWords) s_sum[at / kSumWords * 6 + at % kSumWords] = (unsigned) m[i];
             }
             if (bad) s_bad = 1;
             __syncthreads();
+            // every wavefront adds them up: lane 0, 32, 16 of total hold the
+            // segment's three sums
+            const double* const ss = (const double*) s_sum;
+            double total;
+            if (kByWave) {
+                // lanes 16 k + b: sum k of block b, then the blocks (16 at
+                // most, so the tree's upper levels add zeros)
+                static_assert(kResSplitSums <= 16 * kResWaves, "a row of lanes holds the blocks");
+                const int k = lane < 16 ? 0 : (lane < 32 ? 2 : (lane < 48 ? 1 : 3));
+                const int b = lane & 15;
+                total = 0.0;
+                if (k < 3 && b < nb) {
 #pragma unroll
-            for (int k = 0; k < 3; k++) {
-                double t = 0.0;
-                for (int q = 0; q < NW; q++) t += s_red[q * 3 + k];
-                sum[k] = t;
+                    for (int q = 0; q < kResWaves; q++) total += ss[(b * kResWaves + q) * 3 + k];
+                }
+                total += 0.0;
+                total += dpp_f64<0x108>(total);
+                total += dpp_f64<0x104>(total);
+                total += dpp_f64<0x102>(total);
+                total += dpp_f64<0x101>(total);
+            } else {
+                total = 0.0;
+                for (int q = 0; q < nb; q += 64) {  // the blocks of one wavefront of k_cg_step's reduction
+                    const bool in = q + lane < nb;
+                    const double* const c3 = ss + (q + lane) * 3;
+                    total += wave_sum3(in ? c3[0] : 0.0, in ? c3[1] : 0.0, in ? c3[2] : 0.0);
+                }
             }
             if (s_bad) {
                 leave();
                 return;
             }
+            auto from = [&](int l) {
+                return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(total), l),
+                                        __builtin_amdgcn_readlane(__double2loint(total), l));
+            };
+            sum[0] = from(0);
+            sum[1] = from(32);
+            sum[2] = from(16);
         }
         const double g = sum[0], dd = sum[1], rho = sum[2];
         const bool first = it == 1;
         const bool conv = rho <= thr;
         if (conv || it > max_iter || !(rho == rho)) {
             if (live) y_io[row] = y;
-            if (br.v == 0 && tid == 0) {
+            if (br.v == 0 && blockIdx.x % kSplit == 0 && tid == 0) {
                 sc->done = 1;
                 sc->converged = conv ? 1 : 0;
                 sc->rho2 = rho;
@@ -385,54 +452,75 @@ __global__ void __launch_bounds__(kCgBlock) k_cg_resident(Seg sg, const int* __r
         x[tid] = r;
 #pragma unroll
         for (int i = 0; i < kResHalo; i++) {
-            if (hc[i] < 0) continue;
-            T* const xh = x + kCgBlock + i * kCgBlock + tid;
-            hs[i] = first ? hw[i] : hw[i] + beta * hs[i];
+            if (i * BT >= H || hc[i] < 0) continue;  // the first test is uniform
+            T* const xh = x + BT + i * BT + tid;
+            const T hw = value_of<T>(hm[i]);
+            hs[i] = first ? hw : hw + beta * hs[i];
             *xh = *xh - alpha * hs[i];
         }
         __syncthreads();
     }
 }
 
-size_t resident_lds(int max_rows, int tsize) {
-    if (max_rows > kResMaxRows) return 0;
+constexpr int kSplitThreads = kCgBlock / kResSplit;
+
+static size_t resident_lds(int max_rows, int threads, int tsize) {
     const size_t words = (size_t) (max_rows + 31) / 32;
-    return (size_t) tsize * (kCgBlock + kResHaloRows) + words * 4 + ((words * 2 + 15) & ~(size_t) 15);
+    return (size_t) tsize * (threads + kResHalo * threads) + words * 4 + ((words * 2 + 15) & ~(size_t) 15);
 }
 
-int resident_halo_rows() { return kResHaloRows; }
-
 // Entries held in registers: 16 covers a 2D system at 2.1 l0 (12-14 a row),
-// 36 one at 3.1 l0 (28-32) and 3D at 2.1 l0 (32-34); a wider row reads the
+// 36 one at 3.1 l0 (28-34) and 3D at 2.1 l0 (32-36); a wider row reads the
 // rest from memory every iteration.
 constexpr int kResFew = 16, kResMany = 36;
 
+ResidentShape resident_shape(int max_rows, int max_nb, int total_blocks, int mean_width, int most, int tsize) {
+    ResidentShape s{};
+    if (max_rows > kResMaxRows || max_nb > kResMaxBlocks || total_blocks > most) return s;
+    // Systems of few blocks leave the chip idle: four workgroups a block cut
+    // the row products' LDS reads per CU.  A block alone needs no exchange
+    // and stays whole; beyond 16 blocks the wavefronts' sums are more than
+    // the threads of a split workgroup can wait for.
+    s.split = max_nb > 1 && max_nb * kResWaves <= kResSplitSums && kResSplit * total_blocks <= most ? kResSplit : 1;
+    s.emax = mean_width <= kResFew ? kResFew : kResMany;
+    s.lds = resident_lds(max_rows, kCgBlock / s.split, tsize);
+    return s;
+}
+
+size_t resident_sums(int total_blocks) { return (size_t) kResWaves * total_blocks; }
+size_t resident_sum_words(size_t p_sums) { return 2 * (size_t) kSumWords * p_sums; }
+
 template <typename T, typename IDX>
-hipError_t resident_prepare(int mean_width) {
-    const int bytes = (int) resident_lds(kResMaxRows, (int) sizeof(T));
-    return hipFuncSetAttribute(mean_width <= kResFew ? (const void*) k_cg_resident<T, IDX, kResFew>
-                                                     : (const void*) k_cg_resident<T, IDX, kResMany>,
-                               hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+static const void* resident_kernel(const ResidentShape& s) {
+    if (s.split > 1)
+        return s.emax == kResFew ? (const void*) k_cg_resident<T, IDX, kResFew, kSplitThreads>
+                                 : (const void*) k_cg_resident<T, IDX, kResMany, kSplitThreads>;
+    return s.emax == kResFew ? (const void*) k_cg_resident<T, IDX, kResFew, kCgBlock>
+                             : (const void*) k_cg_resident<T, IDX, kResMany, kCgBlock>;
 }
 
 template <typename T, typename IDX>
-hipError_t resident_launch(const Seg& sg, int total_blocks, const int* slice_off, const IDX* col, const int* anc,
-                           const T* val, const T* r, T* y, const double* dgl, CgScalars* sc, const CgExchange& x,
-                           int mean_width, size_t lds, hipStream_t st) {
-    if (mean_width <= kResFew)
-        hipLaunchKernelGGL((k_cg_resident<T, IDX, kResFew>), dim3(total_blocks), dim3(kCgBlock), lds, st, sg, slice_off,
-                           col, anc, val, r, y, dgl, sc, x);
-    else
-        hipLaunchKernelGGL((k_cg_resident<T, IDX, kResMany>), dim3(total_blocks), dim3(kCgBlock), lds, st, sg,
-                           slice_off, col, anc, val, r, y, dgl, sc, x);
-    return hipGetLastError();
+hipError_t resident_prepare(const ResidentShape& s) {
+    return hipFuncSetAttribute(resident_kernel<T, IDX>(s), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int) resident_lds(kResMaxRows, kCgBlock / s.split, (int) sizeof(T)));
 }
 
-#define RESIDENT_INST(T, IDX)                                                                                       \
-    template hipError_t resident_prepare<T, IDX>(int);                                                              \
-    template hipError_t resident_launch<T, IDX>(const Seg&, int, const int*, const IDX*, const int*, const T*,      \
-                                                const T*, T*, const double*, CgScalars*, const CgExchange&, int,    \
-                                                size_t, hipStream_t);
+template <typename T, typename IDX>
+hipError_t resident_launch(const ResidentShape& s, const Seg& sg, int total_blocks, const int* slice_off,
+                           const IDX* col, const int* anc, const T* val, const T* r, T* y, const double* dgl,
+                           CgScalars* sc, const CgExchange& x, hipStream_t st) {
+    Seg a0 = sg;
+    CgExchange a9 = x;
+    void* args[] = {&a0, &slice_off, &col, &anc, &val, &r, &y, &dgl, &sc, &a9};
+    return hipLaunchKernel(resident_kernel<T, IDX>(s), dim3(s.split * total_blocks), dim3(kCgBlock / s.split), args,
+                           s.lds, st);
+}
+
+#define RESIDENT_INST(T, IDX)                                                                                      \
+    template hipError_t resident_prepare<T, IDX>(const ResidentShape&);                                            \
+    template hipError_t resident_launch<T, IDX>(const ResidentShape&, const Seg&, int, const int*, const IDX*,     \
+                                                const int*, const T*, const T*, T*, const double*, CgScalars*,     \
+                                                const CgExchange&, hipStream_t);
 RESIDENT_INST(double, short)
 RESIDENT_INST(double, unsigned short)
 RESIDENT_INST(double, int)
