@@ -44,6 +44,11 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     f"-I{INCLUDE}",
 ]
+# Flags of single sources.  The resident solver is written to keep its uniform
+# values within the scalar registers; where a compiler runs out of them all the
+# same they go to scratch memory, not to lanes of vector registers: from there
+# some came back wrong in this kernel (mixed precision, 128 threads).
+SOURCE_FLAGS = {"resident.hip": ["-mllvm", "-amdgpu-spill-sgpr-to-vgpr=0"]}
 
 
 def _stale(target, deps):
@@ -58,7 +63,7 @@ def _compile(src, force):
     path = os.path.join(CSRC, src)
     if not force and not _stale(obj, [path] + HEADERS):
         return obj, None
-    cmd = [HIPCC] + FLAGS + ["-c", path, "-o", obj]
+    cmd = [HIPCC] + FLAGS + SOURCE_FLAGS.get(src, []) + ["-c", path, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         return obj, f"$ {' '.join(cmd)}\n{r.stdout}\n{r.stderr}"

@@ -25,8 +25,6 @@ struct CgScalars {
     int converged;
     int frozen;        // timing mode: kernels leave every scalar as it is
     int fin;           // completed updates, written once when the segment stops
-    int bail;          // resident CG: a workgroup gave up; the host runs the solve again by launches
-    unsigned tag0;     // resident CG: exchange tags of this launch start after it
 };
 
 struct Seg {
@@ -223,15 +221,61 @@ __device__ __forceinline__ T sell_row(const int* __restrict__ slice_pos, const I
 }
 
 
-// ---- resident CG (resident.hip) ----
+// FP64 CG restarts from the current iterate when the true residual of the
+// recurrence's answer misses the tolerance.
+constexpr int kMaxRestarts = 3;
+
+// ---- resident solves (resident.hip) ----
 //
-// Exchange memory of the resident CG's workgroups: tagged words (a 32-bit
-// value below a 32-bit tag) in two alternating halves.
+// Exchange memory of the workgroups: tagged words (a 32-bit value below a
+// 32-bit tag) in two alternating halves.
 struct CgExchange {
-    unsigned long long* w;     // 2 halves x 2 words x w_rows: A r of every row
+    unsigned long long* w;     // 2 halves x 2 words x w_rows: a value of every row
     unsigned long long* part;  // 2 halves x p_sums places: 3 partial sums of every block or wavefront
     size_t w_rows, p_sums;
     int halo_max;              // lowers the halo rows a workgroup takes (tests)
+};
+// Options of a solve, read by its launch (pinned host memory).
+struct ResidentIn {
+    double tol2;           // tolerance^2
+    double eta2;           // inner tolerance^2 (mixed)
+    int max_iterations;    // <= 0: 2 x the segment's rows
+    int max_refinements;   // restarts (FP64) or refinements (mixed) at most
+    unsigned tag0;         // the launch's exchange tags follow it
+    unsigned poison;       // the tag of a workgroup that gave up
+    unsigned seq;          // the solve's number
+};
+// Results of a segment, written by its last workgroup (pinned host memory).
+struct ResidentOut {
+    double bn2;            // ||b||^2
+    double rho2_start;     // residual^2 of the start
+    double rho2;           // true residual^2 of the result
+    int iterations;
+    int rounds;            // restarts or refinements
+    int converged;
+    int bail;              // some workgroup gave up: x is not set
+    unsigned seq;          // ResidentIn::seq, written last
+};
+// Everything a launch receives (compared as bytes: captured graphs bake it in).
+struct ResidentArgs {
+    Seg sg;
+    const int* slice_pos;
+    const void* col;       // IDX
+    const int* anc;
+    const void* val;       // T
+    const double* val64;
+    const int* row_slot;
+    const int32_t* id;     // null without a warm start
+    const double* b;       // by slot
+    const double* pprev;
+    const double* pprev2;
+    const double* sdiag;
+    const double* dgl;
+    double* x;             // by slot
+    CgExchange X;
+    int* count;            // per segment: workgroups that have left
+    const ResidentIn* in;
+    ResidentOut* out;
 };
 // Shape of a launch: workgroups per block of the layout (1 or kResSplit),
 // matrix entries a thread holds in registers, dynamic LDS.
@@ -243,19 +287,20 @@ struct ResidentShape {
 };
 // The shape for segments of at most max_rows rows in at most max_nb blocks,
 // total_blocks in all, with at most `most` workgroups at once.
-ResidentShape resident_shape(int max_rows, int max_nb, int total_blocks, int mean_width, int most, int tsize);
-// Places for partial sums (CgExchange::p_sums) a launch needs.
+ResidentShape resident_shape(int max_rows, int max_nb, int total_blocks, int mean_width, int most, bool mixed);
+// Tags a launch may use: its iterations and rounds bound its exchanges.
+long long resident_tags(long long max_iterations, int max_rounds);
+// Places for partial sums (CgExchange::p_sums) a launch needs, and the words
+// both halves of them take.
 size_t resident_sums(int total_blocks);
-size_t resident_sum_words(size_t p_sums);  // words both halves take
+size_t resident_sum_words(size_t p_sums);
 // Lets the kernel of this shape use its LDS (once before its first launch).
 template <typename T, typename IDX>
 hipError_t resident_prepare(const ResidentShape& s);
-// Enqueues the whole CG (every iteration up to each segment's stop) as one
-// launch of split * total_blocks workgroups.  All of them must be able to run
-// at once.
+// Enqueues the solve of every segment as one launch of `grid` workgroups
+// (split x blocks), all of which must be able to run at once.
+// T: double, the FP64 path; float, the mixed path.
 template <typename T, typename IDX>
-hipError_t resident_launch(const ResidentShape& s, const Seg& sg, int total_blocks, const int* slice_off,
-                           const IDX* col, const int* anc, const T* val, const T* r, T* y, const double* dgl,
-                           CgScalars* sc, const CgExchange& x, hipStream_t st);
+hipError_t resident_launch(const ResidentShape& s, int grid, const ResidentArgs& a, hipStream_t st);
 
 }  // namespace mps

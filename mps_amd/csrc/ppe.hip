@@ -36,6 +36,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <vector>
 
 #include "cg_device.hpp"
@@ -374,9 +375,6 @@ constexpr int kStepPre = 4;  // rows a thread of k_cg_step loads ahead of the pa
 // iterations it saves (measured: 584-particle dam break), so small systems
 // keep the Jacobi scaling alone.
 constexpr int kMgMinRows = 8192;
-// FP64 CG restarts from the current iterate when the true residual of the
-// recurrence's answer misses the tolerance.
-constexpr int kMaxRestarts = 3;
 
 // Rows per block of a segment below kMaxBlocks blocks: one per thread.
 // Segments large enough to fill the chip (the 2M and 3.6M dam breaks) take
@@ -737,7 +735,7 @@ struct CgWork {
     // receive, the launch shape and the multigrid hierarchy's generation.
     // Any difference (a buffer reallocated by a larger system, another
     // column width) drops the cached graphs of that solver.
-    static constexpr int kSig = 29;
+    static constexpr int kSig = 24;
     uintptr_t graph_sig[2][kSig] = {};
     static constexpr int kPredSolves = 4;
     bool predict = true;  // MPS_AMD_CG_PREDICT=0: fixed chunks of the check interval
@@ -748,22 +746,35 @@ struct CgWork {
     long long graph_rebuilds = 0;  // times a solver's cached graphs were dropped
     long long vec_reallocs = 0;    // times the CG vectors were reallocated
     long long launched = 0;        // CG iterations enqueued, including those past convergence
-    // resident CG (resident.hip): exchange memory, the last tag handed out and
-    // the most blocks that can run at once (0: off, MPS_AMD_CG_RESIDENT=0 or
-    // after a launch that gave up)
+    // resident solves (resident.hip): exchange memory, the last tag handed
+    // out, the most workgroups that can run at once (0: off, as set by
+    // MPS_AMD_CG_RESIDENT=0 or after a launch that gave up), the launches'
+    // captured graphs (one per signature: the particle arrays alternate) and
+    // the pinned blocks through which a solve's options go in and its
+    // results come out
     CgExchange xch{};
     unsigned tag = 0;
-    int res_blocks = 0;
+    int res_groups = 0;
     int res_dev = 0;
     unsigned res_ready = 0;  // kernel shapes prepared
-    hipGraphExec_t res_graph[2] = {};
+    static constexpr int kResGraphs = 4;
+    hipGraphExec_t res_graph[kResGraphs] = {};
+    ResidentArgs res_sig[kResGraphs] = {};
+    ResidentShape res_shape[kResGraphs] = {};
+    int res_grid[kResGraphs] = {};
+    long long res_used[kResGraphs] = {};
+    ResidentIn* res_in = nullptr;
+    ResidentOut* res_out = nullptr;
+    int* res_count = nullptr;  // device, per segment: workgroups that have left
+    int res_segs = 0;          // segments res_out and res_count hold
+    std::vector<int> up_row, up_blk;  // segment layout the device holds
     Seg seg() const { return Seg{nseg, blk_off, row_off}; }
 };
 
-// Blocks of resident CG launches in flight on each device.  All blocks of a
-// launch wait for each other, so launches of several handles together must
-// not need more than run at once: a solve that would exceed it runs by
-// launches instead, with the same bits.
+// Workgroups of resident launches in flight on each device.  All workgroups
+// of a launch wait for each other, so launches of several handles together
+// must not need more than run at once: a solve that would exceed it runs by
+// kernels instead, with the same bits.
 constexpr int kResDevices = 64;
 static std::atomic<int> g_res_in_flight[kResDevices];
 
@@ -777,9 +788,9 @@ CgWork* cg_create() {
     int cus = 0;
     if ((!v || atoi(v) != 0) && hipGetDevice(&cw->res_dev) == hipSuccess && cw->res_dev < kResDevices &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, cw->res_dev) == hipSuccess)
-        cw->res_blocks = cus;  // a block fits every CU (512 threads, at most 61 KB of LDS)
-    // MPS_AMD_CG_RESIDENT_HALO lowers the halo rows a block of the resident
-    // CG takes, so that a launch gives up and the solve runs by launches
+        cw->res_groups = cus;  // one fits every CU (512 threads, at most 68 KB of LDS)
+    // MPS_AMD_CG_RESIDENT_HALO lowers the halo rows a workgroup of a resident
+    // solve takes, so that a launch gives up and the solve runs by kernels
     // (tests; results unchanged)
     cw->xch.halo_max = 1 << 30;
     if (const char* hm = getenv("MPS_AMD_CG_RESIDENT_HALO")) cw->xch.halo_max = std::max(atoi(hm), 0);
@@ -806,7 +817,10 @@ void cg_destroy(CgWork* cw) {
     mailbox_free(cw->mb);
     hipFree(cw->xch.w);
     hipFree(cw->xch.part);
-    for (int k = 0; k < 2; k++)
+    hipFree(cw->res_count);
+    hipHostFree(cw->res_in);
+    hipHostFree(cw->res_out);
+    for (int k = 0; k < CgWork::kResGraphs; k++)
         if (cw->res_graph[k]) hipGraphExecDestroy(cw->res_graph[k]);
     for (int k = 0; k < 2; k++)
         for (int j = 0; j < CgWork::kGraphSlots; j++)
@@ -831,6 +845,8 @@ static hipError_t cg_reserve_segs(CgWork* cw, int nseg) {
     if ((e = hipHostMalloc(&cw->h_blk, sizeof(int) * (size_t) (nseg + 1), hipHostMallocDefault))) return e;
     if ((e = hipHostMalloc(&cw->h_row, sizeof(int) * (size_t) (nseg + 1), hipHostMallocDefault))) return e;
     cw->nseg_cap = nseg;
+    cw->up_row.clear();  // the new tables hold nothing yet
+    cw->up_blk.clear();
     return hipSuccess;
 }
 
@@ -844,16 +860,6 @@ void cg_debug_counts(const CgWork* cw, long long out[4]) {
     out[1] = cw->vec_reallocs;
     out[2] = cw->launched;
     out[3] = cw->graph_captures;
-}
-
-static void drop_graphs(CgWork* cw, int which) {
-    for (int j = 0; j < CgWork::kGraphSlots; j++) {
-        if (cw->graph[which][j]) hipGraphExecDestroy(cw->graph[which][j]);
-        cw->graph[which][j] = nullptr;
-        cw->graph_chunk[which][j] = 0;
-    }
-    if (cw->res_graph[which]) hipGraphExecDestroy(cw->res_graph[which]);
-    cw->res_graph[which] = nullptr;
 }
 
 hipError_t cg_reserve(CgWork* cw, int rows) {
@@ -870,7 +876,12 @@ hipError_t cg_reserve(CgWork* cw, int rows) {
         (e = hipMalloc(&cw->u32, f)))
         return e;
     cw->cap = cap;
-    for (int k = 0; k < 2; k++) drop_graphs(cw, k);
+    for (int k = 0; k < 2; k++)
+        for (int j = 0; j < CgWork::kGraphSlots; j++) {
+            if (cw->graph[k][j]) hipGraphExecDestroy(cw->graph[k][j]);
+            cw->graph[k][j] = nullptr;
+            cw->graph_chunk[k][j] = 0;
+        }
     return hipSuccess;
 }
 
@@ -899,11 +910,16 @@ static hipError_t cg_layout(CgWork* cw, const Sell& A, hipStream_t st) {
         if ((e = hipMalloc(&cw->part, sizeof(double) * (need + 3 * 1024)))) return e;
         cw->part_cap = need + 3 * 1024;
     }
-    if ((e = hipMemcpyAsync(cw->blk_off, cw->h_blk, sizeof(int) * (size_t) (A.nseg + 1), hipMemcpyHostToDevice, st)))
-        return e;
-    if (A.nseg == 1 &&
-        (e = hipMemcpyAsync(cw->row_off, cw->h_row, sizeof(int) * 2, hipMemcpyHostToDevice, st)))
-        return e;
+    // the device holds the last system's layout: small systems often keep it
+    const std::vector<int> blk(cw->h_blk, cw->h_blk + A.nseg + 1), row(cw->h_row, cw->h_row + A.nseg + 1);
+    if (cw->up_blk != blk) {
+        if ((e = hipMemcpyAsync(cw->blk_off, cw->h_blk, sizeof(int) * blk.size(), hipMemcpyHostToDevice, st))) return e;
+        cw->up_blk = blk;
+    }
+    if (A.nseg == 1 && cw->up_row != row) {
+        if ((e = hipMemcpyAsync(cw->row_off, cw->h_row, sizeof(int) * 2, hipMemcpyHostToDevice, st))) return e;
+        cw->up_row = row;
+    }
     return hipSuccess;
 }
 
@@ -943,36 +959,10 @@ static void enqueue_chunk(CgWork* cw, const Sell& A, const IDX* col, const T* va
     }
 }
 
-// Entries a slot of the SELL slices holds per row, on average (rounded up).
-static int mean_width(const Sell& A) {
-    const size_t per = (size_t) 64 * (size_t) std::max(A.nslices, 1);
-    return (int) ((A.entries + per - 1) / per);
-}
-
 static bool all_done(const CgWork* cw) {
     for (int s = 0; s < cw->nseg; s++)
         if (!cw->host[s].done) return false;
     return true;
-}
-
-// Drops the captured graphs of a solver when anything they bake in changed.
-static void check_graphs(CgWork* cw, int which, const Sell& A, const void* val, const void* col, int idx16,
-                         const void* y, const void* r, const void* p, const void* s, const void* w, const void* u,
-                         const ResidentShape& shape) {
-    const uintptr_t sig[CgWork::kSig] = {
-        (uintptr_t) val,         (uintptr_t) col,          (uintptr_t) A.anc,       (uintptr_t) A.slice_off,
-        (uintptr_t) A.dgl,       (uintptr_t) y,            (uintptr_t) r,           (uintptr_t) p,
-        (uintptr_t) s,           (uintptr_t) w,            (uintptr_t) u,           (uintptr_t) cw->part,
-        (uintptr_t) cw->sc,      (uintptr_t) cw->blk_off,  (uintptr_t) cw->row_off, (uintptr_t) A.rows_dev,
-        (uintptr_t) cw->nseg,    (uintptr_t) cw->total_blocks, (uintptr_t) idx16,
-        (uintptr_t) (cw->mg_on ? mg_generation(cw->mg) + 1 : 0), (uintptr_t) cw->mg_on,
-        (uintptr_t) (cw->mg_on && cw->fused), (uintptr_t) cw->step_cells, (uintptr_t) shape.lds, (uintptr_t) cw->xch.w,
-        (uintptr_t) cw->xch.part, (uintptr_t) cw->xch.w_rows, (uintptr_t) cw->xch.p_sums,
-        (uintptr_t) (64 * shape.split + shape.emax)};
-    if (std::memcmp(sig, cw->graph_sig[which], sizeof(sig)) == 0) return;
-    drop_graphs(cw, which);
-    std::memcpy(cw->graph_sig[which], sig, sizeof(sig));
-    cw->graph_rebuilds++;
 }
 
 // Runs chunks of CG iterations (each a captured graph, or enqueued directly)
@@ -987,8 +977,25 @@ static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* c
     const int idx16 = sizeof(IDX) == 4 ? 0 : (static_cast<IDX>(-1) < 0 ? 1 : 2);
     const size_t sbytes = sizeof(CgScalars) * (size_t) cw->nseg;
     hipError_t e;
-    if (o.use_graph)
-        check_graphs(cw, which, A, val, col, idx16, y, r, p, s, w, u_vec<T>(cw), ResidentShape{});
+    if (o.use_graph) {
+        const uintptr_t sig[CgWork::kSig] = {
+            (uintptr_t) val,         (uintptr_t) col,          (uintptr_t) A.anc,       (uintptr_t) A.slice_off,
+            (uintptr_t) A.dgl,       (uintptr_t) y,            (uintptr_t) r,           (uintptr_t) p,
+            (uintptr_t) s,           (uintptr_t) w,            (uintptr_t) u_vec<T>(cw), (uintptr_t) cw->part,
+            (uintptr_t) cw->sc,      (uintptr_t) cw->blk_off,  (uintptr_t) cw->row_off, (uintptr_t) A.rows_dev,
+            (uintptr_t) cw->nseg,    (uintptr_t) cw->total_blocks, (uintptr_t) idx16,
+            (uintptr_t) (cw->mg_on ? mg_generation(cw->mg) + 1 : 0), (uintptr_t) cw->mg_on,
+            (uintptr_t) (cw->mg_on && cw->fused), (uintptr_t) cw->step_cells, 0};
+        if (std::memcmp(sig, cw->graph_sig[which], sizeof(sig)) != 0) {
+            for (int j = 0; j < CgWork::kGraphSlots; j++) {
+                if (cw->graph[which][j]) hipGraphExecDestroy(cw->graph[which][j]);
+                cw->graph[which][j] = nullptr;
+                cw->graph_chunk[which][j] = 0;
+            }
+            std::memcpy(cw->graph_sig[which], sig, sizeof(sig));
+            cw->graph_rebuilds++;
+        }
+    }
     int launched = 0, grow = 2;
     for (;;) {
         int chunk = interval;
@@ -1040,131 +1047,6 @@ static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* c
     }
 }
 
-// The whole Jacobi-scaled CG in one launch (resident.hip), for systems whose
-// blocks hold at most one row a thread and are no more than the CUs.  An
-// iteration costs 1.5-3.6 us that way against 8-11 us for the two kernels of a
-// chunk graph; beyond one block a CU (131k rows at 256 CUs) the two kernels
-// are bound by their bytes.  *ran: the solve was run and cw->host holds its
-// scalars; false: the caller takes the chunks (from a fresh start if
-// *restart: some segment's iterate may have been written).
-static hipError_t resident_reserve(CgWork* cw, int rows, hipStream_t st) {
-    const size_t w = (size_t) rows, p = resident_sums(cw->total_blocks);
-    hipError_t e;
-    if (w > cw->xch.w_rows) {
-        hipFree(cw->xch.w);
-        cw->xch.w = nullptr;
-        cw->xch.w_rows = 0;
-        const size_t cap = w + w / 8 + 1024;
-        if ((e = hipMalloc(&cw->xch.w, 4 * cap * sizeof(unsigned long long)))) return e;
-        cw->xch.w_rows = cap;
-        if ((e = fill_int((int*) cw->xch.w, 0, 8 * cap, st))) return e;
-    }
-    if (p > cw->xch.p_sums) {
-        hipFree(cw->xch.part);
-        cw->xch.part = nullptr;
-        cw->xch.p_sums = 0;
-        const size_t cap = p + 64;
-        if ((e = hipMalloc(&cw->xch.part, resident_sum_words(cap) * sizeof(unsigned long long)))) return e;
-        cw->xch.p_sums = cap;
-        if ((e = fill_int((int*) cw->xch.part, 0, 2 * resident_sum_words(cap), st))) return e;
-    }
-    return hipSuccess;
-}
-
-static ResidentShape resident_fits(const CgWork* cw, const Sell& A, int tsize) {
-    if (cw->mg_on || cw->res_blocks == 0) return ResidentShape{};
-    int most = 0, most_nb = 0;
-    for (int k = 0; k < cw->nseg; k++) {
-        const int rows = cw->h_row[k + 1] - cw->h_row[k], nb = cw->h_blk[k + 1] - cw->h_blk[k];
-        if (((rows + nb - 1) / nb + 63) / 64 * 64 > kCgBlock) return ResidentShape{};
-        most = std::max(most, rows);
-        most_nb = std::max(most_nb, nb);
-    }
-    return resident_shape(most, most_nb, cw->total_blocks, mean_width(A), cw->res_blocks, tsize);
-}
-
-static hipError_t upload_scalars(CgWork* cw, hipStream_t st);
-
-template <typename T, typename IDX, typename P>
-static hipError_t run_resident(CgWork* cw, int which, const Sell& A, const IDX* col, const T* val, T* y, T* r, T* p,
-                               T* s, T* w, const mps_solver_options& o, const ResidentShape& shape, P&& prep, hipStream_t st,
-                               bool* ran, bool* restart) {
-    *ran = *restart = false;
-    std::atomic<int>& flight = g_res_in_flight[cw->res_dev];
-    const int want = shape.split * cw->total_blocks;
-    if (flight.fetch_add(want) + want > cw->res_blocks) {
-        flight.fetch_sub(want);
-        return hipSuccess;
-    }
-    hipError_t e = hipSuccess;
-    const int idx16 = sizeof(IDX) == 4 ? 0 : (static_cast<IDX>(-1) < 0 ? 1 : 2);
-    const unsigned kernel = 1u << (8 * idx16 + 4 * (int) (sizeof(T) == 8) + 2 * (int) (shape.split > 1) +
-                                   (int) (shape.emax > 16));
-    if (!(cw->res_ready & kernel)) {
-        e = resident_prepare<T, IDX>(shape);
-        cw->res_ready |= kernel;
-    }
-    if (!e) e = resident_reserve(cw, A.rows, st);
-    if (!e) {
-        // this launch's tags: a range none of its words has held
-        unsigned span = 0;
-        for (int k = 0; k < cw->nseg; k++) span = std::max(span, (unsigned) cw->host[k].max_iter + 4u);
-        if (cw->tag > 0xffffffffu - span) {
-            cw->tag = 0;
-            e = fill_int((int*) cw->xch.w, 0, 8 * cw->xch.w_rows, st);
-            if (!e) e = fill_int((int*) cw->xch.part, 0, 2 * resident_sum_words(cw->xch.p_sums), st);
-        }
-        for (int k = 0; k < cw->nseg; k++) cw->host[k].tag0 = cw->tag;
-        cw->tag += span;
-    }
-    if (!e) e = upload_scalars(cw, st);
-    if (!e) prep();
-    auto go = [&]() {
-        return resident_launch<T, IDX>(shape, cw->seg(), cw->total_blocks, A.slice_off, col, A.anc, val, r, y, A.dgl,
-                                       cw->sc, cw->xch, st);
-    };
-    if (!e && o.use_graph) {
-        check_graphs(cw, which, A, val, col, idx16, y, r, p, s, w, u_vec<T>(cw), shape);
-        if (!cw->res_graph[which]) {
-            hipGraph_t gph;
-            e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
-            if (!e) {
-                const hipError_t le = go();
-                e = hipStreamEndCapture(st, &gph);
-                if (!e && le) {
-                    hipGraphDestroy(gph);
-                    e = le;
-                }
-            }
-            if (!e) {
-                e = hipGraphInstantiate(&cw->res_graph[which], gph, nullptr, nullptr, 0);
-                hipGraphDestroy(gph);
-                cw->graph_captures++;
-            }
-        }
-        if (!e) e = hipGraphLaunch(cw->res_graph[which], st);
-    } else if (!e) {
-        e = go();
-    }
-    if (!e) {
-        const MailSrc src{cw->sc, (int) (sizeof(CgScalars) * (size_t) cw->nseg)};
-        e = mailbox_read(cw->mb, &src, 1, cw->host, st);
-    }
-    flight.fetch_sub(want);
-    if (e) return e;
-    bool bail = false;
-    int it = 0;
-    for (int k = 0; k < cw->nseg; k++) {
-        bail = bail || cw->host[k].bail;
-        it = std::max(it, cw->host[k].fin);
-    }
-    cw->launched += it;
-    if (bail) cw->res_blocks = 0;  // a halo too large or CUs held by others: this handle stays with the chunks
-    *ran = !bail;
-    *restart = bail;
-    return hipSuccess;
-}
-
 static hipError_t upload_scalars(CgWork* cw, hipStream_t st) {
     return hipMemcpyAsync(cw->sc, cw->host, sizeof(CgScalars) * (size_t) cw->nseg, hipMemcpyHostToDevice, st);
 }
@@ -1197,46 +1079,256 @@ static void launch_residual(CgWork* cw, const Sell& A, hipStream_t st) {
 
 // `solve`: index of this solve within the step (0 for the FP64 CG, the
 // refinement for the inner CG); the last step's iteration count of the same
-// solve sizes the chunks.  cw->host holds the scalars to start from: they
-// are uploaded here, then prep() enqueues what follows them.  fresh() puts
-// the start's vectors back after a resident launch that gave up.
-template <typename T, typename IDX, bool WEIGHTED, typename P, typename F>
-static hipError_t run_cg_idx(CgWork* cw, int which, const Sell& A, const IDX* col, const T* val, T* y, T* r, T* p,
-                             T* s, T* w, const mps_solver_options& o, int pred, P&& prep, F&& fresh,
-                             hipStream_t st) {
-    hipError_t e;
-    const ResidentShape shape = resident_fits(cw, A, (int) sizeof(T));
-    if (shape.split) {
-        const std::vector<CgScalars> start(cw->host, cw->host + cw->nseg);
-        bool ran, restart;
-        e = run_resident<T, IDX>(cw, which, A, col, val, y, r, p, s, w, o, shape, prep, st, &ran, &restart);
-        if (e || ran) return e;
-        if (restart && (e = fresh())) return e;
-        std::copy(start.begin(), start.end(), cw->host);
-    }
-    if ((e = upload_scalars(cw, st))) return e;
-    prep();
-    return run_cg_loop<T, IDX, WEIGHTED>(cw, which, A, col, val, y, r, p, s, w, o, pred, st);
-}
-
-template <typename T, bool WEIGHTED, typename P, typename F>
+// solve sizes the chunks.
+template <typename T, bool WEIGHTED>
 static hipError_t run_cg(CgWork* cw, int which, int solve, const Sell& A, const T* val, T* y, T* r, T* p, T* s, T* w,
-                         const mps_solver_options& o, P&& prep, F&& fresh, hipStream_t st) {
+                         const mps_solver_options& o, hipStream_t st) {
     const int slot = solve < CgWork::kPredSolves ? solve : CgWork::kPredSolves - 1;
     int* const last = &cw->pred[cw->pred_bank][which][slot];
     const int pred = cw->predict ? *last : 0;
     hipError_t e;
     if (A.use16 && A.dim == 3)
-        e = run_cg_idx<T, unsigned short, WEIGHTED>(cw, which, A, (const unsigned short*) A.dcol, val, y, r, p, s, w, o,
-                                                    pred, prep, fresh, st);
+        e = run_cg_loop<T, unsigned short, WEIGHTED>(cw, which, A, (const unsigned short*) A.dcol, val, y, r, p, s, w, o,
+                                                     pred, st);
     else if (A.use16)
-        e = run_cg_idx<T, short, WEIGHTED>(cw, which, A, A.dcol, val, y, r, p, s, w, o, pred, prep, fresh, st);
+        e = run_cg_loop<T, short, WEIGHTED>(cw, which, A, A.dcol, val, y, r, p, s, w, o, pred, st);
     else
-        e = run_cg_idx<T, int, WEIGHTED>(cw, which, A, A.col, val, y, r, p, s, w, o, pred, prep, fresh, st);
+        e = run_cg_loop<T, int, WEIGHTED>(cw, which, A, A.col, val, y, r, p, s, w, o, pred, st);
     if (e) return e;
     int it = 0;  // the segment that took longest sets the chunk
     for (int k = 0; k < cw->nseg; k++) it = std::max(it, cw->host[k].fin);
     *last = it;
+    return hipSuccess;
+}
+
+// ---- resident solves ----
+
+// Entries a slot of the SELL slices holds per row, on average (rounded up).
+static int mean_width(const Sell& A) {
+    const size_t per = (size_t) 64 * (size_t) std::max(A.nslices, 1);
+    return (int) ((A.entries + per - 1) / per);
+}
+
+static ResidentShape resident_fits(const CgWork* cw, const Sell& A, int precision, int max_ref) {
+    // the refinements bound the tags of a launch (see resident_tags)
+    if (cw->res_groups == 0 || max_ref > 1000) return ResidentShape{};
+    int most = 0, most_nb = 0;
+    for (int k = 0; k < cw->nseg; k++) {
+        const int rows = cw->h_row[k + 1] - cw->h_row[k], nb = cw->h_blk[k + 1] - cw->h_blk[k];
+        if (((rows + nb - 1) / nb + 63) / 64 * 64 > kCgBlock) return ResidentShape{};
+        most = std::max(most, rows);
+        most_nb = std::max(most_nb, nb);
+    }
+    return resident_shape(most, most_nb, cw->total_blocks, mean_width(A), cw->res_groups,
+                          precision == MPS_PREC_MIXED);
+}
+
+static hipError_t resident_reserve(CgWork* cw, int rows, hipStream_t st) {
+    const size_t w = (size_t) rows, p = resident_sums(cw->total_blocks);
+    hipError_t e;
+    if (w > cw->xch.w_rows) {
+        hipFree(cw->xch.w);
+        cw->xch.w = nullptr;
+        cw->xch.w_rows = 0;
+        const size_t cap = w + w / 8 + 1024;
+        if ((e = hipMalloc(&cw->xch.w, 4 * cap * sizeof(unsigned long long)))) return e;
+        cw->xch.w_rows = cap;
+        if ((e = fill_int((int*) cw->xch.w, 0, 8 * cap, st))) return e;
+    }
+    if (p > cw->xch.p_sums) {
+        hipFree(cw->xch.part);
+        cw->xch.part = nullptr;
+        cw->xch.p_sums = 0;
+        const size_t cap = p + 64;
+        if ((e = hipMalloc(&cw->xch.part, resident_sum_words(cap) * sizeof(unsigned long long)))) return e;
+        cw->xch.p_sums = cap;
+        if ((e = fill_int((int*) cw->xch.part, 0, 2 * resident_sum_words(cap), st))) return e;
+    }
+    if (cw->nseg > cw->res_segs) {
+        hipFree(cw->res_count);
+        hipHostFree(cw->res_in);
+        hipHostFree(cw->res_out);
+        cw->res_count = nullptr;
+        cw->res_in = nullptr;
+        cw->res_out = nullptr;
+        cw->res_segs = 0;
+        const unsigned flags = hipHostMallocMapped | hipHostMallocCoherent;
+        if ((e = hipMalloc(&cw->res_count, sizeof(int) * (size_t) cw->nseg))) return e;
+        if ((e = hipHostMalloc((void**) &cw->res_in, sizeof(ResidentIn), flags))) return e;
+        if ((e = hipHostMalloc((void**) &cw->res_out, sizeof(ResidentOut) * (size_t) cw->nseg, flags))) return e;
+        std::memset(cw->res_out, 0, sizeof(ResidentOut) * (size_t) cw->nseg);
+        if ((e = fill_int(cw->res_count, 0, (size_t) cw->nseg, st))) return e;
+        cw->res_segs = cw->nseg;
+    }
+    return hipSuccess;
+}
+
+// Waits until every segment's last workgroup has written its results (spins
+// like mailbox_read, then waits on the stream).
+static hipError_t resident_wait(CgWork* cw, unsigned seq, hipStream_t st) {
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int k = 0; k < cw->nseg; k++)
+        for (unsigned spin = 0; __atomic_load_n(&cw->res_out[k].seq, __ATOMIC_ACQUIRE) != seq; spin++)
+            if ((spin & 1023) == 1023 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+                const hipError_t e = hipStreamSynchronize(st);
+                if (e) return e;
+                if (__atomic_load_n(&cw->res_out[k].seq, __ATOMIC_ACQUIRE) != seq) return hipErrorUnknown;
+            }
+    return hipSuccess;
+}
+
+template <typename T, typename IDX>
+static hipError_t resident_enqueue(CgWork* cw, const ResidentShape& shape, const ResidentArgs& a, bool graph,
+                                   hipStream_t st) {
+    const int idx16 = sizeof(IDX) == 4 ? 0 : (static_cast<IDX>(-1) < 0 ? 1 : 2);
+    const unsigned kernel = 1u << (8 * idx16 + 4 * (int) (sizeof(T) == 8) + 2 * (int) (shape.split > 1) +
+                                   (int) (shape.emax > 16));
+    hipError_t e;
+    if (!(cw->res_ready & kernel)) {
+        if ((e = resident_prepare<T, IDX>(shape))) return e;
+        cw->res_ready |= kernel;
+    }
+    const int grid = shape.split * cw->total_blocks;
+    if (!graph) return resident_launch<T, IDX>(shape, grid, a, st);
+    int slot = -1;
+    for (int k = 0; k < CgWork::kResGraphs; k++)
+        if (cw->res_graph[k] && cw->res_grid[k] == grid && std::memcmp(&cw->res_sig[k], &a, sizeof a) == 0 &&
+            std::memcmp(&cw->res_shape[k], &shape, sizeof shape) == 0)
+            slot = k;
+    if (slot < 0) {  // a free slot, else the least recently used one
+        slot = 0;
+        for (int k = 0; k < CgWork::kResGraphs; k++) {
+            if (!cw->res_graph[k]) {
+                slot = k;
+                break;
+            }
+            if (cw->res_used[k] < cw->res_used[slot]) slot = k;
+        }
+        if (cw->res_graph[slot]) hipGraphExecDestroy(cw->res_graph[slot]);
+        cw->res_graph[slot] = nullptr;
+        hipGraph_t gph;
+        if ((e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal))) return e;
+        const hipError_t le = resident_launch<T, IDX>(shape, grid, a, st);
+        if ((e = hipStreamEndCapture(st, &gph))) return e;
+        e = le ? le : hipGraphInstantiate(&cw->res_graph[slot], gph, nullptr, nullptr, 0);
+        hipGraphDestroy(gph);
+        if (e) return e;
+        std::memcpy(&cw->res_sig[slot], &a, sizeof a);
+        std::memcpy(&cw->res_shape[slot], &shape, sizeof shape);
+        cw->res_grid[slot] = grid;
+        cw->graph_rebuilds++;
+        cw->graph_captures++;
+    }
+    cw->res_used[slot] = ++cw->graph_clock;
+    return hipGraphLaunch(cw->res_graph[slot], st);
+}
+
+// The whole solve in one launch when the system takes it: *ran says whether
+// it did (stats and x_s are then set), else the caller solves by kernels.
+// An iteration costs 1.5-3.6 us that way against 8-11 us for the two kernels
+// of a chunk graph, and the start, the residuals, restarts and refinements
+// need neither launches nor host reads; beyond one workgroup a CU (131k rows
+// at 256 CUs) the kernels are bound by their bytes.
+static hipError_t resident_solve(CgWork* cw, const Sell& A, const Hot& h, const double* b_s, const double* pprev_id,
+                                 const double* pprev2_id, double* x_s, const mps_solver_options& o,
+                                 mps_solver_stats* stats, hipStream_t st, std::string& msg, bool* ran) {
+    *ran = false;
+    const bool mixed = o.precision == MPS_PREC_MIXED;
+    const int max_ref = mixed ? (o.max_refinements > 0 ? o.max_refinements : 20) : kMaxRestarts;
+    const ResidentShape shape = resident_fits(cw, A, o.precision, max_ref);
+    if (!shape.split) return hipSuccess;
+    int most = 0;
+    for (int k = 0; k < cw->nseg; k++) most = std::max(most, cw->h_row[k + 1] - cw->h_row[k]);
+    const long long its = o.max_iterations > 0 ? o.max_iterations : 2ll * most;
+    const long long span = resident_tags(its, max_ref);
+    if (span > 0x40000000ll) return hipSuccess;
+    std::atomic<int>& flight = g_res_in_flight[cw->res_dev];
+    const int want = shape.split * cw->total_blocks;
+    if (flight.fetch_add(want) + want > cw->res_groups) {
+        flight.fetch_sub(want);
+        return hipSuccess;
+    }
+    hipError_t e = resident_reserve(cw, A.rows, st);
+    if (!e && cw->tag > 0xffffffffu - (unsigned) span) {  // tags none of the words has held
+        cw->tag = 0;
+        e = fill_int((int*) cw->xch.w, 0, 8 * cw->xch.w_rows, st);
+        if (!e) e = fill_int((int*) cw->xch.part, 0, 2 * resident_sum_words(cw->xch.p_sums), st);
+    }
+    if (!e) {
+        ResidentIn& in = *cw->res_in;
+        in.tol2 = o.tolerance * o.tolerance;
+        const double eta = o.inner_tolerance > 0 ? o.inner_tolerance : 1e-4;
+        in.eta2 = eta * eta;
+        in.max_iterations = o.max_iterations;
+        in.max_refinements = max_ref;
+        in.tag0 = cw->tag;
+        in.poison = cw->tag + (unsigned) span;
+        in.seq++;
+        cw->tag += (unsigned) span;
+        ResidentArgs a;
+        std::memset(&a, 0, sizeof a);  // compared as bytes
+        a.sg = cw->seg();
+        a.slice_pos = A.slice_off;
+        a.col = A.use16 ? (const void*) A.dcol : (const void*) A.col;
+        a.anc = A.anc;
+        a.val = mixed ? (const void*) A.val32 : (const void*) A.val64;
+        a.val64 = A.val64;
+        a.row_slot = A.row_slot;
+        a.id = o.warm_start ? h.id : nullptr;
+        a.b = b_s;
+        a.pprev = o.warm_start ? pprev_id : nullptr;
+        a.pprev2 = o.warm_start == 2 ? pprev2_id : nullptr;
+        a.sdiag = A.sdiag;
+        a.dgl = A.dgl;
+        a.x = x_s;
+        a.X = cw->xch;
+        a.count = cw->res_count;
+        a.in = cw->res_in;
+        a.out = cw->res_out;
+        const bool g = o.use_graph != 0;
+        if (mixed) {
+            if (A.use16 && A.dim == 3)
+                e = resident_enqueue<float, unsigned short>(cw, shape, a, g, st);
+            else if (A.use16)
+                e = resident_enqueue<float, short>(cw, shape, a, g, st);
+            else
+                e = resident_enqueue<float, int>(cw, shape, a, g, st);
+        } else {
+            if (A.use16 && A.dim == 3)
+                e = resident_enqueue<double, unsigned short>(cw, shape, a, g, st);
+            else if (A.use16)
+                e = resident_enqueue<double, short>(cw, shape, a, g, st);
+            else
+                e = resident_enqueue<double, int>(cw, shape, a, g, st);
+        }
+        if (!e) e = resident_wait(cw, in.seq, st);
+    }
+    flight.fetch_sub(want);
+    if (e) return e;
+    bool bail = false, all_ok = true;
+    int it = 0;
+    for (int k = 0; k < cw->nseg; k++) {
+        bail = bail || cw->res_out[k].bail;
+        it = std::max(it, cw->res_out[k].iterations);
+    }
+    if (bail) {  // a halo too large, or CUs held by others: this handle stays with the kernels
+        cw->res_groups = 0;
+        return hipSuccess;
+    }
+    cw->launched += it;
+    for (int k = 0; k < cw->nseg; k++) {
+        const ResidentOut& r = cw->res_out[k];
+        stats[k].rows = cw->h_row[k + 1] - cw->h_row[k];
+        stats[k].iterations = r.iterations;
+        stats[k].refinements = r.rounds;
+        stats[k].converged = r.converged;
+        stats[k].rhs_norm = sqrt(r.bn2);
+        stats[k].rel_residual = r.bn2 > 0 ? sqrt(r.rho2 / r.bn2) : 0.0;
+        stats[k].initial_residual = r.bn2 > 0 ? sqrt(r.rho2_start / r.bn2) : 0.0;
+        all_ok = all_ok && r.converged;
+    }
+    if (!all_ok) msg = "pressure solve stopped above its tolerance";
+    *ran = true;
     return hipSuccess;
 }
 
@@ -1269,6 +1361,11 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
         else if (me != hipErrorInvalidValue)
             return me;
     }
+    if (!cw->mg_on) {
+        bool ran;
+        e = resident_solve(cw, A, h, b_s, pprev_id, pprev2_id, x_s, o, stats, st, msg, &ran);
+        if (e || ran) return e;
+    }
     cw->fused = 0;
     if (cw->mg_on && cw->fuse_ok && nseg == 1) {
         const int* cst1 = nullptr;
@@ -1284,11 +1381,8 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
         }
     }
 
-    auto init_y = [&]() {
-        hipLaunchKernelGGL(k_cg_init, gr, bl, 0, st, sg, A.row_slot, h.id, b_s, o.warm_start ? pprev_id : nullptr,
-                           o.warm_start == 2 ? pprev2_id : nullptr, A.sdiag, cw->y, cw->bh, cw->part);
-    };
-    init_y();
+    hipLaunchKernelGGL(k_cg_init, gr, bl, 0, st, sg, A.row_slot, h.id, b_s, o.warm_start ? pprev_id : nullptr,
+                       o.warm_start == 2 ? pprev2_id : nullptr, A.sdiag, cw->y, cw->bh, cw->part);
     // ||b||^2 into red[2], then the initial residual: one read for both
     // (and for the multigrid setup's stencil check)
     hipLaunchKernelGGL((k_reduce_parts<1, 2>), dim3(nseg), dim3(kBlock), 0, st, sg, cw->part, cw->sc);
@@ -1321,16 +1415,14 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
     // are discarded for such segments
     bool any_zero = false;
     for (int s = 0; s < nseg; s++) any_zero |= bn2[s] == 0.0;
-    auto zero_y = [&]() -> hipError_t {
-        if (!any_zero) return hipSuccess;
-        if (nseg == 1) return fill_double(cw->y, 0.0, (size_t) rows, st);
-        for (int s = 0; s < nseg; s++)
-            if (bn2[s] == 0.0 && segrows[s] > 0)
-                if (const hipError_t ze = fill_double(cw->y + cw->h_row[s], 0.0, (size_t) segrows[s], st)) return ze;
-        return hipSuccess;
-    };
     if (any_zero) {
-        if ((e = zero_y())) return e;
+        if (nseg == 1) {
+            if ((e = fill_double(cw->y, 0.0, (size_t) rows, st))) return e;
+        } else {
+            for (int s = 0; s < nseg; s++)
+                if (bn2[s] == 0.0 && segrows[s] > 0)
+                    if ((e = fill_double(cw->y + cw->h_row[s], 0.0, (size_t) segrows[s], st))) return e;
+        }
         launch_residual(cw, A, st);
         if ((e = reduce_and_read(cw, 2, st))) return e;
         for (int s = 0; s < nseg; s++) rho2[s] = cw->host[s].red[1];
@@ -1361,16 +1453,9 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
                 cw->host[s] = z;
             }
             if (!any) break;
-            auto fresh = [&]() -> hipError_t {
-                if (pass == 0) {
-                    init_y();
-                    if (const hipError_t ze = zero_y()) return ze;
-                }
-                launch_residual(cw, A, st);  // of whatever iterate y now holds
-                return hipGetLastError();
-            };
+            if ((e = upload_scalars(cw, st))) return e;
             if ((e = run_cg<double, true>(cw, 0, pass, A, A.val64, cw->y, cw->r64, cw->p64, cw->s64, cw->w64, o,
-                                          [] {}, fresh, st)))
+                                          st)))
                 return e;
             for (int s = 0; s < nseg; s++)
                 if (ran[s]) total_it[s] += cw->host[s].fin;
@@ -1393,11 +1478,7 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
             for (int s = 0; s < nseg; s++)
                 active = active || (!conv[s] && refinements[s] < max_ref && total_it[s] < max_it[s]);
             if (!active) break;
-            auto inner_init = [&]() -> hipError_t {
-                hipLaunchKernelGGL(k_inner_init, gr, bl, 0, st, sg, cw->r64, cw->r32, cw->e32, cw->part);
-                return hipGetLastError();
-            };
-            if ((e = inner_init())) return e;
+            hipLaunchKernelGGL(k_inner_init, gr, bl, 0, st, sg, cw->r64, cw->r32, cw->e32, cw->part);
             std::vector<int> run(nseg, 0);
             for (int s = 0; s < nseg; s++) {
                 CgScalars z{};
@@ -1414,11 +1495,10 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
                 z.done = run[s] ? 0 : 1;
                 cw->host[s] = z;
             }
-            auto inner_prep = [&] {
-                hipLaunchKernelGGL(k_inner_prep, dim3(nseg), dim3(kBlock), 0, st, sg, cw->part, cw->sc);
-            };
+            if ((e = upload_scalars(cw, st))) return e;
+            hipLaunchKernelGGL(k_inner_prep, dim3(nseg), dim3(kBlock), 0, st, sg, cw->part, cw->sc);
             if ((e = run_cg<float, false>(cw, 1, round, A, A.val32, cw->e32, cw->r32, cw->p32, cw->s32, cw->w32, o,
-                                          inner_prep, inner_init, st)))
+                                          st)))
                 return e;
             for (int s = 0; s < nseg; s++)
                 if (run[s]) total_it[s] += cw->host[s].fin;
