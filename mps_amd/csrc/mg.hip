@@ -560,6 +560,32 @@ __global__ void __launch_bounds__(kBlock) k_mg_restrict1(const int* __restrict__
 // -1, value 0, after the row's columns) is read at the row's own index and
 // left out of the sum, which keeps the entries' order of summation.
 
+// The forms of the coarse arithmetic, fused where they are fused whichever
+// kernel computes a level: x = omega D^-1 b, a neighbour's and the own value
+// with the coarse correction added, and the smoothed value.
+__device__ __forceinline__ double mg_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float mg_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+template <typename T>
+__device__ __forceinline__ T mg_pre(T omega, T b, T d) {
+    return omega * b * d;
+}
+template <typename T>
+__device__ __forceinline__ T mg_corrected(T pre, T cf, T xc) {
+    return mg_fma(cf, xc, pre);
+}
+template <typename T>
+__device__ __forceinline__ T mg_own_corrected(T omega, T b, T d, T cf, T xc) {
+    return mg_fma(omega * b, d, cf * xc);
+}
+template <typename T>
+__device__ __forceinline__ T mg_fine_start(T omega, T b, T cf, T x) {
+    return mg_fma(omega, b, cf * x);
+}
+template <typename T>
+__device__ __forceinline__ T mg_smoothed(T xx, T omega, T d, T b, T acc) {
+    return mg_fma(omega * d, b - acc, xx);
+}
+
 // Residual of level-l row K at x = omega D^-1 b (x recomputed where read).
 template <typename T, int W>
 __device__ __forceinline__ T mg_child_residual(int K, const int* __restrict__ col, const T* __restrict__ val,
@@ -650,12 +676,12 @@ __global__ void __launch_bounds__(kBlock) k_mg_up(const int* __restrict__ nrow, 
         const T xcK = xc[aK];
 #pragma unroll
         for (int j = 0; j < W; j++) xv[j] = xc[ag[j]];
-        const T xx = omega * bK * dK + cf * xcK;
+        const T xx = mg_own_corrected(omega, bK, dK, cf, xcK);
         T acc = gK * xx;
 #pragma unroll
         for (int j = 0; j < W; j++)
-            if (c[j] >= 0) acc += v[j] * (omega * bb[j] * dd[j] + cf * xv[j]);
-        xK = xx + omega * dK * (bK - acc);
+            if (c[j] >= 0) acc = mg_fma(v[j], mg_corrected(mg_pre(omega, bb[j], dd[j]), cf, xv[j]), acc);
+        xK = mg_smoothed(xx, omega, dK, bK, acc);
         x[K] = xK;
     }
     if (PRO) {
@@ -671,7 +697,7 @@ __global__ void __launch_bounds__(kBlock) k_mg_up(const int* __restrict__ nrow, 
         const int f0 = cst1[K0], f1 = cst1[K1];
         // the low byte of a row's cell is its place among the block's cells
         static_assert(kBlock == 256, "one byte holds a cell's place in the block");
-        for (int r = f0 + (int) threadIdx.x; r < f1; r += blockDim.x) xxf[r] = omega * bf[r] + cf * s_x[aggf[r]];
+        for (int r = f0 + (int) threadIdx.x; r < f1; r += blockDim.x) xxf[r] = mg_fine_start(omega, bf[r], cf, s_x[aggf[r]]);
     }
 }
 
@@ -687,6 +713,7 @@ struct MgLevelDesc {
     const int* child;
     void* b;
     void* x;
+    void* xch;  // k_mg_coarse: 2 halves x (b, x) x cap values, all ones while not yet computed
 };
 
 constexpr int kMgTailRows = 1024;       // levels this small may run inside the tail kernel
@@ -904,7 +931,7 @@ __global__ void __launch_bounds__(kMgTailThreads) k_mg_tail(const MgLevelDesc* _
         const int n = s_n[l];
         for (int K = tid; K < n; K += kMgTailThreads) {
             const T bK = a.b[K], dK = a.dinv[K];
-            const T xx = omega * bK * dK + cf * xc[a.agg[K]];
+            const T xx = mg_own_corrected(omega, bK, dK, cf, xc[a.agg[K]]);
             T acc = a.diag[K] * xx;
             for (int j0 = 0; j0 < W; j0 += kMgBatch) {
                 int c[kMgBatch], ag[kMgBatch];
@@ -926,15 +953,402 @@ __global__ void __launch_bounds__(kMgTailThreads) k_mg_tail(const MgLevelDesc* _
                 for (int q = 0; q < kMgBatch; q++) xv[q] = xc[ag[q]];
 #pragma unroll
                 for (int q = 0; q < kMgBatch; q++)
-                    if (c[q] >= 0) acc += vv[q] * (omega * bb[q] * dd[q] + cf * xv[q]);
+                    if (c[q] >= 0) acc = mg_fma(vv[q], mg_corrected(mg_pre(omega, bb[q], dd[q]), cf, xv[q]), acc);
             }
-            a.x[K] = xx + omega * dK * (bK - acc);
+            a.x[K] = mg_smoothed(xx, omega, dK, bK, acc);
         }
         __syncthreads();
     }
     T* xo = (T*) lv[l0].x;
     const MgLdsLevel<T, W, C> top = level(l0);
     for (int K = tid; K < s_n[l0]; K += kMgTailThreads) xo[K] = top.x[K];
+}
+
+// ---- the coarse levels as one launch
+//
+// A level's kernel down or up is 3-7 us whatever its size: launch, the done
+// flags, and two or three dependent round trips for the operator, with a few
+// arithmetic operations at their end.  k_mg_coarse takes levels lc .. L at
+// once: every row of lc .. lt - 1 has a thread of its own (grouped by parent,
+// as the restriction sums them) that reads its operator row when the launch
+// starts, all levels at the same time, and then waits for its inputs alone:
+// down, b of its neighbours from the rows one level finer; up, x of its and
+// its neighbours' parents.  Block 0 is the tail: the levels from lt on in one
+// workgroup.  So a level costs one store-to-load latency (about 1.5 us) and
+// the first loads are paid once.
+//
+// A value is exchanged as itself, through relaxed device-scope atomics: its
+// place holds all ones (a NaN no result is allowed to be) until it is stored.
+// Two halves alternate from launch to launch; each launch puts the half of
+// the next back to all ones, over the levels' whole capacity, so places that
+// no row writes now are clean when the level grows.  A launch knows its half
+// by an epoch that the last block to leave advances.
+//
+// Measured (launches a level and the tail -> this): 32k rows, 2D FP64 27 -> 10.5
+// us a cycle, 2.41 -> 1.89 ms a step; 252k rows, 2D mixed 33 -> 16.5 us, 3.85 ->
+// 3.12 ms; 74k rows, 3D FP64 4.11 -> 3.19 ms; 2M rows (levels 2 and on) 35 -> 20
+// us.  Of the 10.5 us, 3 are the top level's first loads, 1.3 each exchange,
+// 1.8 the tail, 1.2 the fine level's first step up.
+//
+// All blocks must run at once (the host sees to it); a wait is bounded, and
+// one that fails marks every segment done with the value 2, which tells the
+// host to solve again by a launch a level.
+template <typename T>
+struct MgBits;
+template <>
+struct MgBits<double> {
+    using U = unsigned long long;
+    __device__ static U to(double v) { return (U) __double_as_longlong(v); }
+    __device__ static double from(U u) { return __longlong_as_double((long long) u); }
+};
+template <>
+struct MgBits<float> {
+    using U = unsigned;
+    __device__ static U to(float v) { return __float_as_uint(v); }
+    __device__ static float from(U u) { return __uint_as_float(u); }
+};
+template <typename T>
+constexpr typename MgBits<T>::U kMgOpen = ~(typename MgBits<T>::U) 0;
+
+template <typename T>
+__device__ __forceinline__ void mg_put(typename MgBits<T>::U* p, T v) {
+    typename MgBits<T>::U u = MgBits<T>::to(v);
+    if (u == kMgOpen<T>) u ^= 1;  // another NaN
+    __hip_atomic_store(p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void mg_open(typename MgBits<T>::U* p) {
+    __hip_atomic_store(p, kMgOpen<T>, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Values at base[at[0 .. N)], once all of them are there; false after a wait
+// too long.  ahead: at[N - 1] alone is polled until it is there, then all.
+// A poll goes past the caches, and many of them at a few places are served
+// slowly: with every row polling all its places (3D, 6,500 and 36,000 rows
+// of 27 neighbours on the two finest levels) the loads of wavefronts that had
+// yet to store what the others waited for took milliseconds.  So rows of 27
+// neighbours (1,200 of them at a level: 100 -> 94 ms per 10 steps of the 1M
+// particle 3D case), the finest level, which waits longest, and levels of
+// more than kMgPollMost rows poll ahead (0.3 us more a wait), and a polling
+// wavefront pauses between polls and is the last of its CU to be served.
+constexpr int kMgPollMost = 8192;
+template <typename T, int N>
+__device__ __forceinline__ bool mg_get(const typename MgBits<T>::U* base, const int (&at)[N], T (&v)[N], bool ahead,
+                                       int polls) {
+    using U = typename MgBits<T>::U;
+    BoundedWait wt;
+    wt.most = polls;
+    __builtin_amdgcn_s_setprio(0);
+    bool got = true;
+    if (ahead)
+        while (__hip_atomic_load(base + at[N - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kMgOpen<T>) {
+            if (wt.expired()) {
+                got = false;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(4);
+        }
+    for (;;) {
+        U u[N];
+#pragma unroll
+        for (int j = 0; j < N; j++) u[j] = __hip_atomic_load(base + at[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        bool open = false;
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            open = open || u[j] == kMgOpen<T>;
+            v[j] = MgBits<T>::from(u[j]);
+        }
+        if (!open || !got) break;
+        if (wt.expired()) {
+            got = false;
+            break;
+        }
+        __builtin_amdgcn_s_sleep(2);
+    }
+    __builtin_amdgcn_s_setprio(2);
+    return got;
+}
+
+constexpr int kMgCoarseLevels = 10;  // levels lc .. lt at most
+template <typename T>
+struct MgCoarse {
+    MgLevelDesc lv[kMgCoarseLevels];   // of levels lc ..
+    int first[kMgCoarseLevels];        // their first blocks; [lt - lc]: all blocks
+    int each;                          // threads of a block that have a row (not the tail's)
+    const MgLevelDesc* all;
+    const int* nd;
+    int lc, lt, L;
+    T omega, cf;
+    int sweeps;
+    int polls;   // of a wait at most (0: as long as the clock allows)
+    MgDone done;
+    int* epoch;  // launches so far; then the blocks that have left this one
+    // level 1 also takes the fine level's first step up (see k_mg_up)
+    const int* cst1;
+    const T* bf;
+    T* xxf;
+};
+
+// The tail of k_mg_coarse: levels l0 .. L, a thread for every row of all of
+// them (at most BT together), its operator row in registers, b and x in LDS.
+// A level down or up is one round of LDS reads and a chain of W fused
+// multiply-adds: 0.2-0.4 us against 1 us with the operator in LDS too.
+// get_b(K) waits for b of level l0, put_x(K, x) passes its result on.
+template <typename T, int W, int C, int BT, typename GetB, typename PutX>
+__device__ __forceinline__ void mg_tail_rows(const MgLevelDesc* __restrict__ lv, const int* __restrict__ nd, int l0,
+                                             int L, T omega, T cf, int sweeps, GetB&& get_b, PutX&& put_x) {
+    __shared__ int s_row[kMgMaxLevels + 2];
+    __shared__ T s_b[BT], s_x[2][BT], s_r[BT], s_d[BT];
+    __shared__ int s_a[BT];
+    const int tid = threadIdx.x;
+    if (tid == 0) {
+        int r = 0;
+        for (int l = l0; l <= L; l++) {
+            s_row[l] = r;
+            r += nd[l];
+        }
+        s_row[L + 1] = r;
+    }
+    __syncthreads();
+    // threads past the rows follow the last row and are of no level
+    const int R = s_row[L + 1];
+    const int t = tid < R ? tid : R - 1;
+    int l = l0;
+    while (t >= s_row[l + 1]) l++;
+    const int base = s_row[l], K = t - base;
+    const int mine = tid < R ? l : -1;
+    const MgLevelDesc d = lv[l];
+    int at[W], ag[W], ch[C];
+    T v[W], pre[W];
+#pragma unroll
+    for (int j = 0; j < W; j++) {
+        const int c = d.col[(size_t) j * d.cap + K];
+        v[j] = ((const T*) d.val)[(size_t) j * d.cap + K];  // 0 where there is no neighbour
+        at[j] = base + (c >= 0 ? c : K);
+    }
+    const T gK = ((const T*) d.diag)[K], dK = ((const T*) d.dinv)[K];
+    const int aK = l < L ? s_row[l + 1] + d.agg[K] : 0;
+#pragma unroll
+    for (int q = 0; q < C; q++) ch[q] = l > l0 ? d.child[(size_t) q * d.cap + K] : -1;
+    s_d[tid] = dK;
+    s_a[tid] = aK;
+    s_x[0][tid] = (T) 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < W; j++) {
+        ag[j] = s_a[at[j]];
+        pre[j] = s_d[at[j]];
+    }
+    if (mine == l0) s_b[tid] = get_b(K);
+    __syncthreads();
+    T bK = s_b[t];
+    for (int k = l0; k < L; k++) {
+        if (mine == k) {
+            bK = s_b[t];
+            T acc = gK * (omega * bK * dK);
+#pragma unroll
+            for (int j = 0; j < W; j++) {
+                pre[j] = mg_pre(omega, s_b[at[j]], pre[j]);
+                acc = mg_fma(v[j], pre[j], acc);
+            }
+            s_r[tid] = bK - acc;
+        }
+        __syncthreads();
+        if (mine == k + 1) {  // the children's residuals, summed as k_mg_down does
+            T u[C];
+#pragma unroll
+            for (int q = 0; q < C; q++) u[q] = ch[q] >= 0 ? s_r[s_row[k] + ch[q]] : (T) 0;
+#pragma unroll
+            for (int o = C / 2; o > 0; o >>= 1)
+#pragma unroll
+                for (int q = 0; q < o; q++) u[q] += u[q + o];
+            s_b[tid] = u[0];
+        }
+        __syncthreads();
+    }
+    if (mine == L) bK = s_b[t];
+    int h = 0;
+    for (int it = 0; it < sweeps; it++) {
+        if (mine == L) {
+            const T xt = s_x[h][tid];
+            T xv[W];
+#pragma unroll
+            for (int j = 0; j < W; j++) xv[j] = s_x[h][at[j]];
+            T acc = gK * xt;
+#pragma unroll
+            for (int j = 0; j < W; j++) acc = mg_fma(v[j], xv[j], acc);
+            s_x[h ^ 1][tid] = mg_smoothed(xt, omega, dK, bK, acc);
+        }
+        __syncthreads();
+        h ^= 1;
+    }
+    for (int k = L - 1; k >= l0; k--) {
+        if (mine == k) {
+            T xv[W];
+            const T xc = s_x[h][aK];
+#pragma unroll
+            for (int j = 0; j < W; j++) xv[j] = s_x[h][ag[j]];
+            const T xx = mg_own_corrected(omega, bK, dK, cf, xc);
+            T acc = gK * xx;
+#pragma unroll
+            for (int j = 0; j < W; j++) acc = mg_fma(v[j], mg_corrected(pre[j], cf, xv[j]), acc);
+            const T x = mg_smoothed(xx, omega, dK, bK, acc);
+            s_x[h][tid] = x;
+            if (k == l0) put_x(K, x);
+        }
+        __syncthreads();
+    }
+    if (l0 == L && mine == L) put_x(K, s_x[h][tid]);
+}
+
+constexpr int kMgProRows = 8;  // fine rows of a cell in a round
+
+template <typename T, int W, int C, int BT>
+__global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
+    using U = typename MgBits<T>::U;
+    __shared__ int s_half, s_bad;
+    const int tid = threadIdx.x;
+    __builtin_amdgcn_s_setprio(2);
+    // the block's level (level lt: block 0, the tail) and the thread's row,
+    // read together with the flags
+    int i = 0;
+    while (i + 1 < a.lt - a.lc && (int) blockIdx.x >= a.first[i + 1]) i++;
+    const bool tail = blockIdx.x == 0;
+    if (tail) i = a.lt - a.lc;
+    const MgLevelDesc& d = a.lv[i];
+    const MgLevelDesc& dp = a.lv[tail ? i : i + 1];
+    const int t = ((int) blockIdx.x - a.first[i]) * a.each + tid;
+    const int P = t / C, q = t % C;
+    const bool mine = !tail && tid < a.each;
+    int np = 0, Kc = -1;
+    if (mine) {
+        np = a.nd[a.lc + i + 1];
+        Kc = P < dp.cap ? dp.child[(size_t) q * dp.cap + P] : -1;
+    }
+    if (tid == 0) {
+        s_half = *(volatile const int*) a.epoch & 1;
+        s_bad = 0;
+    }
+    if (mg_done_wave(a.done)) return;  // the same for the whole launch
+    __syncthreads();
+    const int half = s_half;
+    auto places = [&](const MgLevelDesc& e, int h, int x) { return (U*) e.xch + (size_t) (2 * h + x) * e.cap; };
+    bool ok = true;
+    if (tail) {
+        U* const bt = places(d, half, 0);
+        U* const xt = places(d, half, 1);
+        for (int k = tid; k < 2 * d.cap; k += BT) mg_open<T>(places(d, half ^ 1, 0) + k);
+        mg_tail_rows<T, W, C, BT>(
+            a.all, a.nd, a.lt, a.L, a.omega, a.cf, a.sweeps,
+            [&](int K) {
+                const int at[1] = {K};
+                T v[1];
+                ok = mg_get<T, 1>(bt, at, v, false, a.polls);
+                return v[0];
+            },
+            [&](int K, T v) { mg_put<T>(xt + K, v); });
+    } else if (mine) {
+        const bool top = i == 0;
+        // the next launch's half
+        if (!top) {
+            const int threads = (a.first[i + 1] - a.first[i]) * a.each;
+            for (int k = t; k < 2 * d.cap; k += threads) mg_open<T>(places(d, half ^ 1, 0) + k);
+        }
+        if ((t & ~63) / C < np) {  // else no row of this wavefront exists
+            const bool live = P < np && Kc >= 0;
+            // a thread without a row follows one of its wavefront that has (each
+            // parent has a child) and stores nothing: with all of them on one
+            // row, its places were polled thousands of times at once
+            const unsigned long long rows = __ballot(live);  // all lanes are here: not inside the choice below
+            const int some = __shfl(Kc, rows ? __ffsll(rows) - 1 : 0, 64);
+            const int K = live ? Kc : (rows ? some : 0);
+            const T* const val = (const T*) d.val;
+            const T* const dinv = (const T*) d.dinv;
+            int at[W + 1], ag[W + 1];
+            T v[W], pre[W], bb[W + 1];
+#pragma unroll
+            for (int j = 0; j < W; j++) {
+                at[j] = d.col[(size_t) j * d.cap + K];
+                v[j] = val[(size_t) j * d.cap + K];  // 0 where there is no neighbour
+            }
+            const T dK = dinv[K], gK = ((const T*) d.diag)[K];
+            ag[W] = d.agg[K];
+            const bool pro = a.xxf && a.lc == 1 && top;
+            int f0 = 0, f1 = 0;
+            if (pro) {
+                f0 = a.cst1[K];
+                f1 = a.cst1[K + 1];
+            }
+#pragma unroll
+            for (int j = 0; j < W; j++) at[j] = at[j] >= 0 ? at[j] : K;
+            at[W] = K;
+#pragma unroll
+            for (int j = 0; j < W; j++) {
+                pre[j] = dinv[at[j]];
+                ag[j] = d.agg[at[j]];
+            }
+            T bf[kMgProRows];
+            if (top) {
+                const T* const b = (const T*) d.b;
+#pragma unroll
+                for (int j = 0; j <= W; j++) bb[j] = b[at[j]];
+            }
+            if (pro) {
+#pragma unroll
+                for (int j = 0; j < kMgProRows; j++) bf[j] = a.bf[f0 + j < f1 ? f0 + j : f0];
+            }
+            // down
+            const bool many = W > 9 || a.nd[a.lc + i] > kMgPollMost;
+            if (!top) ok = mg_get<T, W + 1>(places(d, half, 0), at, bb, many, a.polls);
+            const T bK = bb[W];
+            {
+                T acc = gK * (a.omega * bK * dK);
+#pragma unroll
+                for (int j = 0; j < W; j++) {
+                    pre[j] = mg_pre(a.omega, bb[j], pre[j]);
+                    acc = mg_fma(v[j], pre[j], acc);
+                }
+                T res = live ? bK - acc : (T) 0;
+                for (int o = C / 2; o > 0; o >>= 1) res += __shfl_down(res, o, C);
+                if (P < np && q == 0) mg_put<T>(places(dp, half, 0) + P, res);
+            }
+            // up
+            T xv[W + 1];
+            ok = mg_get<T, W + 1>(places(dp, half, 1), ag, xv, top || many, a.polls) && ok;
+            const T xx = mg_own_corrected(a.omega, bK, dK, a.cf, xv[W]);
+            T acc = gK * xx;
+#pragma unroll
+            for (int j = 0; j < W; j++) acc = mg_fma(v[j], mg_corrected(pre[j], a.cf, xv[j]), acc);
+            const T xK = mg_smoothed(xx, a.omega, dK, bK, acc);
+            if (live) {
+                if (!top) mg_put<T>(places(d, half, 1) + K, xK);
+                if (top && !pro) ((T*) d.x)[K] = xK;
+                if (pro) {
+                    for (int r = f0;;) {
+#pragma unroll
+                        for (int j = 0; j < kMgProRows; j++)
+                            if (r + j < f1) a.xxf[r + j] = mg_fine_start(a.omega, bf[j], a.cf, xK);
+                        r += kMgProRows;
+                        if (r >= f1) break;
+#pragma unroll
+                        for (int j = 0; j < kMgProRows; j++) bf[j] = a.bf[r + j < f1 ? r + j : f0];
+                    }
+                }
+            }
+        }
+    }
+    if (!ok) s_bad = 1;
+    __syncthreads();
+    if (tid == 0) {
+        if (s_bad)
+            for (int k = 0; k < a.done.count; k++)
+                *(volatile int*) const_cast<int*>(a.done.flag + (size_t) k * a.done.stride) = 2;
+        // every block read the epoch before it leaves
+        const int left = __hip_atomic_fetch_add(a.epoch + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (left == (int) gridDim.x - 1) {
+            __hip_atomic_store(a.epoch + 1, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(a.epoch, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
 }
 
 // Fine level, up: xx = omega b + cf x1[agg0] ...
@@ -1042,6 +1456,19 @@ struct MgWork {
     int fine_mode = 0;               // 0: by size, 1: additive, 2: multiplicative
     bool fine_additive = false;      // the current hierarchy's choice
     int tail_rows = kMgTailRows;
+    // k_mg_coarse: the most workgroups it may take (0: off, by
+    // MPS_AMD_MG_COARSE or after a launch that gave up), its levels lc ..
+    // co_lt - 1 (none: not used) and its tail co_lt .. L, their first blocks,
+    // the exchange places and what they were last cleared for
+    int co_most = 0;
+    int co_polls = 0;
+    int lc = 1, co_lt = 1;
+    int co_each = 0;                 // rows of a block
+    int co_first[kMgCoarseLevels] = {};
+    void* xch[kMgMaxLevels + 1] = {};
+    int* epoch = nullptr;
+    int xch_key[3] = {};
+    bool xch_new = false;            // some level's places were reallocated
 };
 
 void mg_set_params(MgWork* m, double omega, double cf, int sweeps) {
@@ -1064,6 +1491,19 @@ MgWork* mg_create() {
         if (sscanf(v, "%lf,%lf,%d,%d", &om, &cf, &sw, &tr) >= 1) mg_set_params(m, om, cf, sw);
         if (tr > 0) m->tail_rows = tr;
     }
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+        m->co_most = cus;
+    // MPS_AMD_MG_COARSE="workgroups[,polls]": the workgroups k_mg_coarse may
+    // take at most (0: a launch a level), and the polls after which a wait
+    // gives up (tests; results unchanged)
+    if (const char* v = getenv("MPS_AMD_MG_COARSE")) {
+        int most = 0, polls = 0;
+        const int got = sscanf(v, "%d,%d", &most, &polls);
+        if (got >= 1) m->co_most = std::min(m->co_most, std::max(most, 0));
+        if (got >= 2) m->co_polls = std::max(polls, 0);
+    }
     if (const char* v = getenv("MPS_AMD_MG_FINE"))
         m->fine_mode = std::strcmp(v, "additive") == 0 ? 1 : (std::strcmp(v, "multiplicative") == 0 ? 2 : 0);
     return m;
@@ -1071,9 +1511,10 @@ MgWork* mg_create() {
 
 static void mg_free_level(MgWork* m, int l) {
     void* ps[] = {m->agg[l],  m->coord[l], m->child[l], m->col[l], m->val[l],
-                  m->diag[l], m->dinv[l],  m->b[l],     m->x[l],   m->scene[l]};
+                  m->diag[l], m->dinv[l],  m->b[l],     m->x[l],   m->scene[l], m->xch[l]};
     for (void* p : ps) hipFree(p);
     m->scene[l] = nullptr;
+    m->xch[l] = nullptr;
     m->agg[l] = m->coord[l] = m->child[l] = m->col[l] = nullptr;
     m->val[l] = m->diag[l] = m->dinv[l] = m->b[l] = m->x[l] = nullptr;
     m->cap[l] = 0;
@@ -1087,7 +1528,7 @@ void mg_destroy(MgWork* m) {
         hipFree(m->d_goff[l]);
     }
     void* ps[] = {m->nd,  m->err,   m->cst1,  m->head,     m->hscan, m->rkey,     m->agg0b,
-                  m->res0, m->xx0, m->flag, m->pscan, m->scan_tmp, m->desc, m->lsz};
+                  m->res0, m->xx0, m->flag, m->pscan, m->scan_tmp, m->desc, m->lsz, m->epoch};
     for (void* p : ps) hipFree(p);
     mailbox_free(m->mb);
     delete m;
@@ -1119,6 +1560,8 @@ static hipError_t mg_reserve_level(MgWork* m, int l, int need) {
         if ((er = mg_alloc(&m->dinv[l], e * cap))) return er;
         if ((er = mg_alloc(&m->b[l], e * cap))) return er;
         if ((er = mg_alloc(&m->x[l], e * cap))) return er;
+        if ((er = mg_alloc(&m->xch[l], 4 * e * cap))) return er;
+        m->xch_new = true;
     }
     m->cap[l] = cap;
     m->gen++;
@@ -1160,6 +1603,73 @@ static hipError_t mg_allow_tail_lds() {
     return once;
 }
 
+// 27 neighbours in FP64 take the registers of 256 threads
+template <typename T, int W>
+constexpr int kMgCoarseThreads = W == 27 && sizeof(T) == 8 ? 256 : 512;
+
+// The levels k_mg_coarse takes: its tail from the first level whose rows,
+// with those of the levels below, are at most a workgroup's threads, and from
+// the finest level whose blocks, with those of the levels below, all run at
+// once (counted one a CU).
+template <typename T>
+static hipError_t mg_coarse_plan(MgWork* m, int dim, hipStream_t st) {
+    const int bt = dim == 2 ? kMgCoarseThreads<T, 9> : kMgCoarseThreads<T, 27>;
+    int lt = m->L + 1, rows = 0;
+    while (lt > 1 && rows + m->n[lt - 1] <= bt) {
+        // a level joins the tail with some room to grow, and leaves it only
+        // when it does not fit
+        if (lt - 1 < m->co_lt && rows + m->n[lt - 1] > bt - bt / 8) break;
+        rows += m->n[--lt];
+    }
+    // the fewer rows a block has the sooner their operator rows are there (a
+    // CU takes a wavefront's scattered load at a time: 512 rows 3.5 us, 64
+    // rows 2), up to three quarters of the blocks there may be
+    int lc = lt, each = bt, first[kMgCoarseLevels] = {};
+    const auto blocks = [&](int l, int rows) { return (m->C * m->cap[l + 1] + rows - 1) / rows; };
+    if (lt <= m->L) {
+        int sum = 1;
+        while (lc > 1 && lt - lc + 2 <= kMgCoarseLevels && sum + blocks(lc - 1, bt) <= m->co_most)
+            sum += blocks(--lc, bt);
+        for (int rows = 64; rows < bt; rows *= 2) {
+            sum = 1;
+            for (int l = lc; l < lt; l++) sum += blocks(l, rows);
+            if (sum <= m->co_most - m->co_most / 4) {
+                each = rows;
+                break;
+            }
+        }
+        int f = 1;
+        for (int l = lc; l < lt; l++) {
+            first[l - lc] = f;
+            f += blocks(l, each);
+        }
+        if (lc < lt) first[lt - lc] = f;
+    }
+    if (lc != m->lc || lt != m->co_lt || each != m->co_each || std::memcmp(first, m->co_first, sizeof first) != 0)
+        m->gen++;
+    m->lc = lc;
+    m->co_lt = lt;
+    m->co_each = each;
+    std::memcpy(m->co_first, first, sizeof first);
+    const int key[3] = {lc, lt, (int) sizeof(T)};
+    if (lc < lt && (m->xch_new || std::memcmp(key, m->xch_key, sizeof key) != 0)) {
+        hipError_t e;
+        for (int l = lc + 1; l <= lt; l++)
+            if ((e = fill_int((int*) m->xch[l], -1, 8 * (size_t) m->cap[l], st))) return e;
+        if ((e = fill_int(m->epoch, 0, 2, st))) return e;
+        std::memcpy(m->xch_key, key, sizeof key);
+        m->xch_new = false;
+    }
+    return hipSuccess;
+}
+
+int mg_coarse_groups(const MgWork* m) { return m && m->lc < m->co_lt ? m->co_first[m->co_lt - m->lc] : 0; }
+void mg_coarse_off(MgWork* m) {
+    m->co_most = 0;
+    m->lc = m->co_lt;
+    m->gen++;
+}
+
 // The fine level's form for this system (see MgWork::fine_mode).  A system
 // that took the additive cycle keeps it down to 7/8 of the threshold, so a
 // size near it does not switch the cycle, and with it the captured CG
@@ -1199,6 +1709,7 @@ static hipError_t mg_setup_t(MgWork* m, const Sell& A, const Hot& h, int dim, co
         if ((e = mg_alloc(&m->lsz, sizeof(int) * (kMgMaxLevels + 1)))) return e;
         if ((e = fill_int(m->lsz, 0, kMgMaxLevels + 1, st))) return e;
         if ((e = mg_alloc(&m->err, sizeof(int)))) return e;
+        if ((e = mg_alloc(&m->epoch, 2 * sizeof(int)))) return e;
         if ((e = mg_alloc(&m->desc, sizeof(MgLevelDesc) * (kMgMaxLevels + 1)))) return e;
     }
     if (R > m->fcap) {
@@ -1384,9 +1895,10 @@ static hipError_t mg_setup_t(MgWork* m, const Sell& A, const Hot& h, int dim, co
     }
     if (tail != m->tail) m->gen++;
     m->tail = tail;
+    if ((e = mg_coarse_plan<T>(m, dim, st))) return e;
     for (int k = 1; k <= l; k++)
         m->hdesc[k] = MgLevelDesc{m->cap[k], 0,         m->col[k], m->val[k],   m->diag[k],
-                                  m->dinv[k], m->agg[k], m->child[k], m->b[k], m->x[k]};
+                                  m->dinv[k], m->agg[k], m->child[k], m->b[k], m->x[k], m->xch[k]};
     if (!m->up_desc_valid || std::memcmp(m->up_desc, m->hdesc, sizeof(m->hdesc)) != 0) {
         std::memcpy(m->up_desc, m->hdesc, sizeof(m->hdesc));
         m->up_desc_valid = true;
@@ -1428,23 +1940,49 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
         hipLaunchKernelGGL((k_mg_restrict1<T>), mg_grid(m->cap[1]), dim3(kBlock), 0, st, nd + 1, m->cst1,
                            add ? r : (const T*) res0, (T*) m->b[1], done);
     T* const xf = add ? u : xx0;  // the fine level's first step up
-    for (int l = 1; l < lt; l++)
+    const bool one = m->lc < m->co_lt;  // levels lc .. L in k_mg_coarse
+    const int lc = one ? m->lc : lt;
+    for (int l = 1; l < lc; l++)
         hipLaunchKernelGGL((k_mg_down<T, W, C>), mg_grid(C * m->cap[l + 1]), dim3(kBlock), 0, st, nd + l + 1,
                            m->child[l + 1], m->cap[l + 1], m->col[l], (const T*) m->val[l], (const T*) m->diag[l],
                            (const T*) m->dinv[l], m->cap[l], (const T*) m->b[l], (T*) m->b[l + 1], om, done);
-    hipLaunchKernelGGL((k_mg_tail<T, W, C>), dim3(1), dim3(kMgTailThreads), kMgTailLds, st, m->desc, nd, lt, L, om,
-                       cf, m->sweeps, done);
-    for (int l = lt - 1; l >= 2; l--)
+    if (one) {
+        constexpr int BT = kMgCoarseThreads<T, W>;
+        MgCoarse<T> a;
+        const int k1 = m->co_lt - lc;
+        for (int k = 0; k <= k1; k++) a.lv[k] = m->hdesc[lc + k];
+        a.each = m->co_each;
+        a.all = m->desc;
+        a.nd = nd;
+        a.lc = lc;
+        a.lt = m->co_lt;
+        a.L = L;
+        std::memcpy(a.first, m->co_first, sizeof a.first);
+        a.omega = om;
+        a.cf = cf;
+        a.sweeps = m->sweeps;
+        a.polls = m->co_polls;
+        a.done = done;
+        a.epoch = m->epoch;
+        a.cst1 = m->cst1;
+        a.bf = r;
+        a.xxf = lc == 1 ? xf : nullptr;
+        hipLaunchKernelGGL((k_mg_coarse<T, W, C, BT>), dim3(m->co_first[k1]), dim3(BT), 0, st, a);
+    } else {
+        hipLaunchKernelGGL((k_mg_tail<T, W, C>), dim3(1), dim3(kMgTailThreads), kMgTailLds, st, m->desc, nd, lt, L,
+                           om, cf, m->sweeps, done);
+    }
+    for (int l = lc - 1; l >= 2; l--)
         hipLaunchKernelGGL((k_mg_up<T, W, false>), mg_grid(m->cap[l]), dim3(kBlock), 0, st, nd + l, m->col[l],
                            (const T*) m->val[l], (const T*) m->diag[l], (const T*) m->dinv[l], m->cap[l], m->agg[l],
                            (const T*) m->b[l], (const T*) m->x[l + 1], (T*) m->x[l], om, cf, done, nullptr, nullptr,
                            nullptr, nullptr);
-    if (lt >= 2)  // level 1's up pass also takes the fine level's first step up
+    if (lc >= 2)  // level 1's up pass also takes the fine level's first step up
         hipLaunchKernelGGL((k_mg_up<T, W, true>), mg_grid(m->cap[1]), dim3(kBlock), 0, st, nd + 1, m->col[1],
                            (const T*) m->val[1], (const T*) m->diag[1], (const T*) m->dinv[1], m->cap[1], m->agg[1],
                            (const T*) m->b[1], (const T*) m->x[2], (T*) m->x[1], om, cf, done, m->cst1, r, xf,
                            m->agg0b);
-    else
+    else if (!one)
         hipLaunchKernelGGL((k_mg_prolong0<T>), mg_grid(m->cap[0]), dim3(kBlock), 0, st, nd + 0, r, m->agg[0],
                            (const T*) m->x[1], xf, om, cf, done);
     if (!add)

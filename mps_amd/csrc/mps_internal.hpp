@@ -121,6 +121,23 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
     return xcd * per + (xcd < rem ? xcd : rem) + idx;
 }
 
+// A bounded wait within a kernel: expired() at every poll; true once it has
+// taken too long.
+constexpr long long kWaitTicks = 5000000;  // of the 100 MHz clock: 50 ms
+struct BoundedWait {
+    int most = 0;  // polls at most, 0: by the clock
+    int n = 0;
+    long long t0 = 0;
+    __device__ __forceinline__ bool expired() {
+        ++n;
+        if (most && n >= most) return true;
+        if ((n & 63) != 0) return false;
+        const long long t = wall_clock64();
+        if (n == 64) t0 = t;
+        return t - t0 > kWaitTicks;
+    }
+};
+
 // Sum of v[r0 .. r1) in row order, four loads in flight (the level-1
 // restriction of the multigrid cycle; the CG step forms the same sums where
 // it writes r, so both give the same bits).
@@ -1147,6 +1164,11 @@ struct MgDone {
 template <typename T, typename IDX>
 void mg_cycle(MgWork* m, const Sell& A, const IDX* fcol, const T* fval, const T* r, T* u, MgDone done, int dim,
               bool b1_given, hipStream_t st);
+// Workgroups of the cycle's coarse launch, which must all run at once (0: it
+// has none); a launch that had to wait too long sets every done flag to 2,
+// and the caller switches it off and solves again (the bits are the same).
+int mg_coarse_groups(const MgWork* m);
+void mg_coarse_off(MgWork* m);
 // When the current hierarchy's cycle restricts the fine residual r itself
 // (the additive fine level): the first fine row of each level-1 cell
 // (n1 + 1 entries, the last = rows) and the level-1 right-hand side b1[K] =

@@ -755,6 +755,7 @@ struct CgWork {
     CgExchange xch{};
     unsigned tag = 0;
     int res_groups = 0;
+    int res_most = 0;  // of all handles together: one a CU
     int res_dev = 0;
     unsigned res_ready = 0;  // kernel shapes prepared
     static constexpr int kResGraphs = 4;
@@ -775,8 +776,30 @@ struct CgWork {
 // of a launch wait for each other, so launches of several handles together
 // must not need more than run at once: a solve that would exceed it runs by
 // kernels instead, with the same bits.
+// The dispatcher deals a launch's workgroups out over the 8 XCDs in turn, so
+// they are counted in eights.
 constexpr int kResDevices = 64;
 static std::atomic<int> g_res_in_flight[kResDevices];
+struct ResidentGroups {
+    std::atomic<int>* flight = nullptr;
+    int held = 0;
+    bool take(int dev, int groups, int most) {
+        const int want = (groups + 7) & ~7;
+        std::atomic<int>& f = g_res_in_flight[dev];
+        if (f.fetch_add(want) + want > most) {
+            f.fetch_sub(want);
+            return false;
+        }
+        flight = &f;
+        held = want;
+        return true;
+    }
+    void give_back() {
+        if (flight) flight->fetch_sub(held);
+        flight = nullptr;
+    }
+    ~ResidentGroups() { give_back(); }
+};
 
 void cg_prediction_bank(CgWork* cw, int bank) { cw->pred_bank = bank ? 1 : 0; }
 
@@ -786,9 +809,10 @@ CgWork* cg_create() {
     if (const char* v = getenv("MPS_AMD_CG_FUSE")) cw->fuse_ok = atoi(v) != 0;
     const char* v = getenv("MPS_AMD_CG_RESIDENT");
     int cus = 0;
-    if ((!v || atoi(v) != 0) && hipGetDevice(&cw->res_dev) == hipSuccess && cw->res_dev < kResDevices &&
+    if (hipGetDevice(&cw->res_dev) == hipSuccess && cw->res_dev < kResDevices &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, cw->res_dev) == hipSuccess)
-        cw->res_groups = cus;  // one fits every CU (512 threads, at most 68 KB of LDS)
+        cw->res_most = cus;  // a workgroup of any of these kernels fits every CU
+    if (!v || atoi(v) != 0) cw->res_groups = cw->res_most;
     // MPS_AMD_CG_RESIDENT_HALO lowers the halo rows a workgroup of a resident
     // solve takes, so that a launch gives up and the solve runs by kernels
     // (tests; results unchanged)
@@ -1242,12 +1266,8 @@ static hipError_t resident_solve(CgWork* cw, const Sell& A, const Hot& h, const 
     const long long its = o.max_iterations > 0 ? o.max_iterations : 2ll * most;
     const long long span = resident_tags(its, max_ref);
     if (span > 0x40000000ll) return hipSuccess;
-    std::atomic<int>& flight = g_res_in_flight[cw->res_dev];
-    const int want = shape.split * cw->total_blocks;
-    if (flight.fetch_add(want) + want > cw->res_groups) {
-        flight.fetch_sub(want);
-        return hipSuccess;
-    }
+    ResidentGroups groups;
+    if (!groups.take(cw->res_dev, shape.split * cw->total_blocks, cw->res_most)) return hipSuccess;
     hipError_t e = resident_reserve(cw, A.rows, st);
     if (!e && cw->tag > 0xffffffffu - (unsigned) span) {  // tags none of the words has held
         cw->tag = 0;
@@ -1303,7 +1323,7 @@ static hipError_t resident_solve(CgWork* cw, const Sell& A, const Hot& h, const 
         }
         if (!e) e = resident_wait(cw, in.seq, st);
     }
-    flight.fetch_sub(want);
+    groups.give_back();
     if (e) return e;
     bool bail = false, all_ok = true;
     int it = 0;
@@ -1336,7 +1356,6 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
                     const double* pprev2_id,
                     double* x_s, const mps_solver_options& o, mps_solver_stats* stats, hipStream_t st,
                     std::string& msg) {
-    (void) n;
     const int rows = A.rows;
     const int nseg = A.nseg;
     for (int s = 0; s < nseg; s++) {
@@ -1399,6 +1418,22 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
         std::memcpy(&mg_bad, (const char*) buf.data() + sizeof(CgScalars) * (size_t) nseg, sizeof(int));
         if (cw->mg_on && mg_bad) cw->mg_on = 0;  // a coarse row outside the stencil: Jacobi alone
     }
+    // the cycle's coarse launch waits between its workgroups: they are counted
+    // in for the whole solve
+    ResidentGroups groups;
+    if (cw->mg_on && mg_coarse_groups(cw->mg) > 0 &&
+        !groups.take(cw->res_dev, mg_coarse_groups(cw->mg), cw->res_most))
+        mg_coarse_off(cw->mg);
+    const auto gave_up = [&]() {
+        for (int s = 0; s < nseg; s++)
+            if (cw->host[s].done == 2) return true;
+        return false;
+    };
+    const auto again = [&]() {  // from the start, by a launch a level
+        mg_coarse_off(cw->mg);
+        groups.give_back();
+        return cg_solve(cw, A, h, n, b_s, pprev_id, pprev2_id, x_s, o, stats, st, msg);
+    };
     std::vector<double> bn2(nseg), thr(nseg), rho2(nseg);
     std::vector<int> segrows(nseg), conv(nseg), total_it(nseg, 0), refinements(nseg, 0), max_it(nseg),
         restarts(nseg, 0);
@@ -1457,6 +1492,7 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
             if ((e = run_cg<double, true>(cw, 0, pass, A, A.val64, cw->y, cw->r64, cw->p64, cw->s64, cw->w64, o,
                                           st)))
                 return e;
+            if (gave_up()) return again();
             for (int s = 0; s < nseg; s++)
                 if (ran[s]) total_it[s] += cw->host[s].fin;
             launch_residual(cw, A, st);
@@ -1500,6 +1536,7 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
             if ((e = run_cg<float, false>(cw, 1, round, A, A.val32, cw->e32, cw->r32, cw->p32, cw->s32, cw->w32, o,
                                           st)))
                 return e;
+            if (gave_up()) return again();
             for (int s = 0; s < nseg; s++)
                 if (run[s]) total_it[s] += cw->host[s].fin;
             // segments that did not run keep e = 0 from k_inner_init

@@ -48,7 +48,6 @@ namespace mps {
 
 constexpr int kResHalo = 8;               // halo rows a thread updates
 constexpr int kResMaxRows = 131072;       // rows of a segment (bits of the halo map)
-constexpr long long kResWait = 5000000;   // ticks of the 100 MHz clock a wait may take (50 ms)
 constexpr int kResWaves = kCgBlock / 64;  // wavefronts of a block of the layout
 constexpr int kResMaxBlocks = 256;        // blocks of a segment
 constexpr int kResSplitSums = 128;        // wavefronts of a segment with split blocks
@@ -115,18 +114,6 @@ __device__ __forceinline__ T value_of(const unsigned long long* w) {
     else
         return __uint_as_float((unsigned) w[0]);
 }
-
-// A bounded wait: expired() every poll; true once it has taken too long.
-struct Wait {
-    int n = 0;
-    long long t0 = 0;
-    __device__ __forceinline__ bool expired() {
-        if ((++n & 63) != 0) return false;
-        const long long t = wall_clock64();
-        if (n == 64) t0 = t;
-        return t - t0 > kResWait;
-    }
-};
 
 // acc + sum of val[k] * x[idx[k]] in entry order, each product and sum
 // rounded by itself as sell_row does (contraction is off here).
@@ -259,7 +246,7 @@ __device__ __forceinline__ bool resident_exchange(ResidentPeers& P, ResidentLds<
             at[i] = q < (unsigned) nw ? q : (unsigned) tid & (kSumWords - 1);
         }
     }
-    Wait wt;
+    BoundedWait wt;
     for (;;) {
         if (SUMS) {
 #pragma unroll
