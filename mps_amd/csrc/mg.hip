@@ -988,7 +988,9 @@ __global__ void __launch_bounds__(kMgTailThreads) k_mg_tail(const MgLevelDesc* _
 // us a cycle, 2.41 -> 1.89 ms a step; 252k rows, 2D mixed 33 -> 16.5 us, 3.85 ->
 // 3.12 ms; 74k rows, 3D FP64 4.11 -> 3.19 ms; 2M rows (levels 2 and on) 35 -> 20
 // us.  Of the 10.5 us, 3 are the top level's first loads, 1.3 each exchange,
-// 1.8 the tail, 1.2 the fine level's first step up.
+// 1.8 the tail, 1.2 the fine level's first step up.  Level 1's right-hand side
+// summed here too costs 2 us more where the kernel before it took 3.9 (3D: 4.3
+// for 6.6).
 //
 // All blocks must run at once (the host sees to it); a wait is bounded, and
 // one that fails marks every segment done with the value 2, which tells the
@@ -1021,7 +1023,7 @@ __device__ __forceinline__ void mg_open(typename MgBits<T>::U* p) {
     __hip_atomic_store(p, kMgOpen<T>, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // Values at base[at[0 .. N)], once all of them are there; false after a wait
-// too long.  ahead: at[N - 1] alone is polled until it is there, then all.
+// too long.  ahead >= 0: that place is polled until it is there, then all.
 // A poll goes past the caches, and many of them at a few places are served
 // slowly: with every row polling all its places (3D, 6,500 and 36,000 rows
 // of 27 neighbours on the two finest levels) the loads of wavefronts that had
@@ -1032,15 +1034,15 @@ __device__ __forceinline__ void mg_open(typename MgBits<T>::U* p) {
 // wavefront pauses between polls and is the last of its CU to be served.
 constexpr int kMgPollMost = 8192;
 template <typename T, int N>
-__device__ __forceinline__ bool mg_get(const typename MgBits<T>::U* base, const int (&at)[N], T (&v)[N], bool ahead,
+__device__ __forceinline__ bool mg_get(const typename MgBits<T>::U* base, const int (&at)[N], T (&v)[N], int ahead,
                                        int polls) {
     using U = typename MgBits<T>::U;
     BoundedWait wt;
     wt.most = polls;
     __builtin_amdgcn_s_setprio(0);
     bool got = true;
-    if (ahead)
-        while (__hip_atomic_load(base + at[N - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kMgOpen<T>) {
+    if (ahead >= 0)
+        while (__hip_atomic_load(base + ahead, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == kMgOpen<T>) {
             if (wt.expired()) {
                 got = false;
                 break;
@@ -1082,8 +1084,10 @@ struct MgCoarse {
     int polls;   // of a wait at most (0: as long as the clock allows)
     MgDone done;
     int* epoch;  // launches so far; then the blocks that have left this one
-    // level 1 also takes the fine level's first step up (see k_mg_up)
+    // level 1 also sums its right-hand side from the fine vector res (null: it
+    // is there) and takes the fine level's first step up (see k_mg_up)
     const int* cst1;
+    const T* res;
     const T* bf;
     T* xxf;
 };
@@ -1242,14 +1246,15 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             [&](int K) {
                 const int at[1] = {K};
                 T v[1];
-                ok = mg_get<T, 1>(bt, at, v, false, a.polls);
+                ok = mg_get<T, 1>(bt, at, v, -1, a.polls);
                 return v[0];
             },
             [&](int K, T v) { mg_put<T>(xt + K, v); });
     } else if (mine) {
         const bool top = i == 0;
+        const bool sums = a.res && top;
         // the next launch's half
-        if (!top) {
+        if (!top || a.lc == 1) {
             const int threads = (a.first[i + 1] - a.first[i]) * a.each;
             for (int k = t; k < 2 * d.cap; k += threads) mg_open<T>(places(d, half ^ 1, 0) + k);
         }
@@ -1272,9 +1277,9 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             }
             const T dK = dinv[K], gK = ((const T*) d.diag)[K];
             ag[W] = d.agg[K];
-            const bool pro = a.xxf && a.lc == 1 && top;
+            const bool pro = a.xxf && top;
             int f0 = 0, f1 = 0;
-            if (pro) {
+            if (pro || sums) {
                 f0 = a.cst1[K];
                 f1 = a.cst1[K + 1];
             }
@@ -1287,7 +1292,17 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
                 ag[j] = d.agg[at[j]];
             }
             T bf[kMgProRows];
-            if (top) {
+            if (sums) {  // in row order, as cell_sum
+                T s = (T) 0;
+                for (int r = f0; r < f1; r += kMgProRows) {
+#pragma unroll
+                    for (int j = 0; j < kMgProRows; j++) bf[j] = a.res[r + j < f1 ? r + j : f1 - 1];
+#pragma unroll
+                    for (int j = 0; j < kMgProRows; j++)
+                        if (r + j < f1) s += bf[j];
+                }
+                if (live) mg_put<T>(places(d, half, 0) + K, s);
+            } else if (top) {
                 const T* const b = (const T*) d.b;
 #pragma unroll
                 for (int j = 0; j <= W; j++) bb[j] = b[at[j]];
@@ -1298,7 +1313,9 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             }
             // down
             const bool many = W > 9 || a.nd[a.lc + i] > kMgPollMost;
-            if (!top) ok = mg_get<T, W + 1>(places(d, half, 0), at, bb, many, a.polls);
+            // (where the thread itself has put its own value: a neighbour's)
+            if (!top || sums)
+                ok = mg_get<T, W + 1>(places(d, half, 0), at, bb, many ? (sums ? at[0] : K) : -1, a.polls);
             const T bK = bb[W];
             {
                 T acc = gK * (a.omega * bK * dK);
@@ -1313,7 +1330,7 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             }
             // up
             T xv[W + 1];
-            ok = mg_get<T, W + 1>(places(dp, half, 1), ag, xv, top || many, a.polls) && ok;
+            ok = mg_get<T, W + 1>(places(dp, half, 1), ag, xv, top || many ? ag[W] : -1, a.polls) && ok;
             const T xx = mg_own_corrected(a.omega, bK, dK, a.cf, xv[W]);
             T acc = gK * xx;
 #pragma unroll
@@ -1654,7 +1671,7 @@ static hipError_t mg_coarse_plan(MgWork* m, int dim, hipStream_t st) {
     const int key[3] = {lc, lt, (int) sizeof(T)};
     if (lc < lt && (m->xch_new || std::memcmp(key, m->xch_key, sizeof key) != 0)) {
         hipError_t e;
-        for (int l = lc + 1; l <= lt; l++)
+        for (int l = lc; l <= lt; l++)
             if ((e = fill_int((int*) m->xch[l], -1, 8 * (size_t) m->cap[l], st))) return e;
         if ((e = fill_int(m->epoch, 0, 2, st))) return e;
         std::memcpy(m->xch_key, key, sizeof key);
@@ -1936,12 +1953,14 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
     if (!add)
         hipLaunchKernelGGL((k_mg_down0<T, IDX>), mg_grid(m->cap[0]), dim3(kBlock), 0, st, nd + 0, A.slice_off, fcol,
                            A.anc, fval, r, res0, om, done);
-    if (!(add && b1_given))
-        hipLaunchKernelGGL((k_mg_restrict1<T>), mg_grid(m->cap[1]), dim3(kBlock), 0, st, nd + 1, m->cst1,
-                           add ? r : (const T*) res0, (T*) m->b[1], done);
-    T* const xf = add ? u : xx0;  // the fine level's first step up
+    // level 1's right-hand side: k_mg_coarse sums it where it takes level 1
     const bool one = m->lc < m->co_lt;  // levels lc .. L in k_mg_coarse
     const int lc = one ? m->lc : lt;
+    const T* const res = add ? (b1_given ? nullptr : r) : (const T*) res0;
+    if (res && !(one && lc == 1))
+        hipLaunchKernelGGL((k_mg_restrict1<T>), mg_grid(m->cap[1]), dim3(kBlock), 0, st, nd + 1, m->cst1, res,
+                           (T*) m->b[1], done);
+    T* const xf = add ? u : xx0;  // the fine level's first step up
     for (int l = 1; l < lc; l++)
         hipLaunchKernelGGL((k_mg_down<T, W, C>), mg_grid(C * m->cap[l + 1]), dim3(kBlock), 0, st, nd + l + 1,
                            m->child[l + 1], m->cap[l + 1], m->col[l], (const T*) m->val[l], (const T*) m->diag[l],
@@ -1965,6 +1984,7 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
         a.done = done;
         a.epoch = m->epoch;
         a.cst1 = m->cst1;
+        a.res = lc == 1 ? res : nullptr;
         a.bf = r;
         a.xxf = lc == 1 ? xf : nullptr;
         hipLaunchKernelGGL((k_mg_coarse<T, W, C, BT>), dim3(m->co_first[k1]), dim3(BT), 0, st, a);
