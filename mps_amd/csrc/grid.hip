@@ -90,6 +90,12 @@ __global__ void __launch_bounds__(kScanTopThreads) k_scan_top(int* __restrict__ 
     if (threadIdx.x == 0) part[nb] = tot;
 }
 
+// What precedes a block's tile: already scanned in part[block] (kScanned),
+// the sum of the tiles' sums part[0 .. block) (kSums), or the sum of the input
+// itself before the tile (kInput: no other launch at all).
+enum ScanFrom { kScanned, kSums, kInput };
+
+template <ScanFrom FROM>
 __global__ void __launch_bounds__(kBlock) k_scan_final(const int* __restrict__ in, int m,
                                                        const int* __restrict__ part,
                                                        int* __restrict__ out, int nb) {
@@ -101,6 +107,23 @@ __global__ void __launch_bounds__(kBlock) k_scan_final(const int* __restrict__ i
         int i = base + k * kBlock + threadIdx.x;
         tile[k * kBlock + threadIdx.x] = i < m ? in[i] : 0;
     }
+    int before = 0;
+    if (FROM == kScanned) {
+        before = part[blockIdx.x];
+    } else {
+        int s = 0;
+        if (FROM == kSums) {
+            for (int k = threadIdx.x; k < (int) blockIdx.x; k += kBlock) s += part[k];
+        } else {
+            const int4* const v = (const int4*) in;
+#pragma unroll 8
+            for (int k = threadIdx.x; k < base / 4; k += kBlock) {
+                const int4 q = v[k];
+                s += q.x + q.y + q.z + q.w;
+            }
+        }
+        block_exclusive_scan(s, lds, &before);
+    }
     __syncthreads();
     int loc[kScanItems];
     int s = 0;
@@ -110,7 +133,7 @@ __global__ void __launch_bounds__(kBlock) k_scan_final(const int* __restrict__ i
         s += tile[threadIdx.x * kScanItems + k];
     }
     int tot;
-    int ex = block_exclusive_scan(s, lds, &tot) + part[blockIdx.x];
+    int ex = block_exclusive_scan(s, lds, &tot) + before;
 #pragma unroll
     for (int k = 0; k < kScanItems; k++) tile[threadIdx.x * kScanItems + k] = ex + loc[k];
     __syncthreads();
@@ -119,19 +142,34 @@ __global__ void __launch_bounds__(kBlock) k_scan_final(const int* __restrict__ i
         int i = base + k * kBlock + threadIdx.x;
         if (i < m) out[i] = tile[k * kBlock + threadIdx.x];
     }
-    if (blockIdx.x == nb - 1 && threadIdx.x == 0) out[m] = part[nb];
+    if ((int) blockIdx.x == nb - 1 && threadIdx.x == 0) out[m] = before + tot;
 }
 
 size_t scan_tmp_ints(int m) { return (size_t) ((m + kScanTile - 1) / kScanTile) + 2; }
 
-// out[0..m] = exclusive prefix sums of in[0..m-1], out[m] = total.
+// out[0..m] = exclusive prefix sums of in[0..m-1], out[m] = total; in and out
+// are not the same array.  A step makes 5 to 10 scans, and a launch costs the
+// host 4-5 us and the device 3-4: up to kScanInputTiles tiles a block adds up
+// the input before its tile itself (16 tiles: 128 KB for the last one, 3 us),
+// up to kScanSumTiles it adds up the tiles' sums (8 loads a thread), and only
+// beyond are those scanned by a launch of their own.
+constexpr int kScanInputTiles = 16;
+constexpr int kScanSumTiles = 2048;
 hipError_t scan_exclusive(const int* in, int* out, int m, int* tmp, hipStream_t st) {
     if (m <= 0) return fill_int(out, 0, 1, st);
     const int nb = (m + kScanTile - 1) / kScanTile;
     if (nb > kScanTopThreads * 64) return hipErrorInvalidValue;  // > 134M elements
+    if (nb <= kScanInputTiles && ((uintptr_t) in & 15) == 0) {
+        hipLaunchKernelGGL(k_scan_final<kInput>, dim3(nb), dim3(kBlock), 0, st, in, m, tmp, out, nb);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_scan_partials, dim3(nb), dim3(kBlock), 0, st, in, m, tmp);
+    if (nb <= kScanSumTiles) {
+        hipLaunchKernelGGL(k_scan_final<kSums>, dim3(nb), dim3(kBlock), 0, st, in, m, tmp, out, nb);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kScanTopThreads), 0, st, tmp, nb);
-    hipLaunchKernelGGL(k_scan_final, dim3(nb), dim3(kBlock), 0, st, in, m, tmp, out, nb);
+    hipLaunchKernelGGL(k_scan_final<kScanned>, dim3(nb), dim3(kBlock), 0, st, in, m, tmp, out, nb);
     return hipGetLastError();
 }
 
