@@ -1071,6 +1071,149 @@ __device__ __forceinline__ bool mg_get(const typename MgBits<T>::U* base, const 
 }
 
 constexpr int kMgCoarseLevels = 10;  // levels lc .. lt at most
+
+// The operator rows of levels lc .. lt - 1 as k_mg_coarse's threads take them,
+// every array entry-major over all its threads with a row (n of them), so that
+// each load is whole lines: in the levels' own arrays a wavefront's rows, the
+// children of 8 or 16 parents, are scattered over some 30 lines a load.
+// Entries are at their places in the stencil (the row itself in the middle and
+// where there is no neighbour, value 0), so the parents of all neighbours are
+// the 2^dim at the places (px, py, pz): 0 the row's own, 1 the other that is
+// next to it in that direction.  (3D polls 8 words a row for 28, 2D 4 for 10.)
+// Measured, rows where they are -> packed: 1M particles, 3D mixed 48 -> 42 us a
+// cycle; 2M, 2D 20.5 -> 17.5; 254k 19.0 -> 18.3; 35k FP64 unchanged at 13.9.
+// Packing is a launch of 8-20 us a step.
+template <typename T>
+struct MgPacked {
+    int n;
+    int* row;   // the row; ~(a row of its wavefront) for a thread without one
+    T* val;     // W
+    T* dinv;    // W: of the neighbours
+    T* diag;
+    int* at;    // W: the neighbours
+    int* up;    // C: the parents
+};
+
+// The same from one value a parent to one a neighbour: v[place of the parent]
+// of a row whose cell is odd in the directions of the bits of q.
+template <typename T, int W, int C>
+__device__ __forceinline__ void mg_of_parents(const T (&v)[C], int q, T (&out)[W]) {
+    constexpr int NZ = C / 4;
+    const bool ox = q & 1, oy = q & 2, oz = q & 4;
+    T e[NZ][3][3];
+#pragma unroll
+    for (int z = 0; z < NZ; z++) {
+        T f[2][3];
+#pragma unroll
+        for (int y = 0; y < 2; y++) {
+            const T own = v[4 * z + 2 * y], other = v[4 * z + 2 * y + 1];
+            f[y][0] = ox ? own : other;
+            f[y][1] = own;
+            f[y][2] = ox ? other : own;
+        }
+#pragma unroll
+        for (int x = 0; x < 3; x++) {
+            e[z][0][x] = oy ? f[0][x] : f[1][x];
+            e[z][1][x] = f[0][x];
+            e[z][2][x] = oy ? f[1][x] : f[0][x];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const T own = e[0][k / 3][k % 3], other = e[NZ - 1][k / 3][k % 3];
+        if constexpr (W == 9) {
+            out[k] = own;
+        } else {
+            out[k] = oz ? own : other;
+            out[9 + k] = own;
+            out[18 + k] = oz ? other : own;
+        }
+    }
+}
+
+// What k_mg_pack reads of levels lc .. lt.
+struct MgPackIn {
+    MgLevelDesc lv[kMgCoarseLevels];
+    const int* coord[kMgCoarseLevels];
+    const int* scene[kMgCoarseLevels];
+    const MgDims* dims[kMgCoarseLevels];
+    int rows[kMgCoarseLevels];
+    int first[kMgCoarseLevels];
+    int levels;  // lt - lc
+    int each;
+};
+
+// Fills MgPacked: a thread for each of k_mg_coarse's that may have a row, in
+// its blocks (its tail's left out).
+template <typename T, int W, int C>
+__global__ void __launch_bounds__(512) k_mg_pack(MgPackIn a, MgPacked<T> o) {
+    const int block = (int) blockIdx.x + 1, tid = threadIdx.x;
+    int i = 0;
+    while (i + 1 < a.levels && block >= a.first[i + 1]) i++;
+    const MgLevelDesc& d = a.lv[i];
+    const int t = (block - a.first[i]) * a.each + tid;
+    const int g = (int) blockIdx.x * a.each + tid;
+    const int P = t / C, q = t % C;
+    const int Kc = P < a.rows[i + 1] ? a.lv[i + 1].child[(size_t) q * a.lv[i + 1].cap + P] : -1;
+    // a thread without a row follows one of its wavefront that has (each
+    // parent has a child): with all of them on one row, its places were
+    // polled thousands of times at once
+    const unsigned long long rows = __ballot(Kc >= 0);
+    if (!rows) {
+        o.row[g] = ~0;
+        return;
+    }
+    const int some = __shfl(Kc, __ffsll(rows) - 1, 64);
+    const int K = Kc >= 0 ? Kc : some;
+    o.row[g] = Kc >= 0 ? K : ~K;
+    const T dK = ((const T*) d.dinv)[K];
+    const int up = d.agg[K];
+    o.diag[g] = ((const T*) d.diag)[K];
+    const size_t n = (size_t) o.n;
+    for (int j = 0; j < W; j++) {
+        o.val[j * n + g] = (T) 0;
+        o.dinv[j * n + g] = dK;
+        o.at[j * n + g] = K;
+    }
+    for (int c = 0; c < C; c++) o.up[c * n + g] = up;
+    if (Kc < 0) return;
+    const MgDims dm = a.dims[i][a.scene[i][K]];
+    const int key = a.coord[i][K];
+    // in rounds of kMgBatch, each round's loads issued together (read one by
+    // one the 27 entries of 3D took 35 us)
+    for (int k0 = 0; k0 < W; k0 += kMgBatch) {
+        int c[kMgBatch], ck[kMgBatch], ca[kMgBatch];
+        T v[kMgBatch], di[kMgBatch];
+#pragma unroll
+        for (int k = 0; k < kMgBatch; k++) {
+            c[k] = d.col[(size_t) (k0 + k) * d.cap + K];
+            v[k] = ((const T*) d.val)[(size_t) (k0 + k) * d.cap + K];
+        }
+        if (c[0] < 0) break;  // padding, column -1, follows the row's entries
+#pragma unroll
+        for (int k = 0; k < kMgBatch; k++) {
+            const int cc = c[k] >= 0 ? c[k] : K;
+            ck[k] = a.coord[i][cc];
+            ca[k] = d.agg[cc];
+            di[k] = ((const T*) d.dinv)[cc];
+        }
+#pragma unroll
+        for (int k = 0; k < kMgBatch; k++) {
+            if (c[k] < 0) continue;
+            const int j = mg_stencil_of_cells<W>(key, ck[k], dm);
+            if (j < 0) continue;  // the assembly has reported it
+            o.val[j * n + g] = v[k];
+            o.dinv[j * n + g] = di[k];
+            o.at[j * n + g] = c[k];
+            int place = 0;
+            const int off[3] = {j % 3, j / 3 % 3, W == 9 ? 1 : j / 9};
+            for (int x = 0; x < 3; x++)
+                if (off[x] != 1 && (off[x] == 2) == ((q >> x & 1) != 0)) place |= 1 << x;
+            if (place) o.up[place * n + g] = ca[k];
+        }
+    }
+}
+
 template <typename T>
 struct MgCoarse {
     MgLevelDesc lv[kMgCoarseLevels];   // of levels lc ..
@@ -1090,6 +1233,7 @@ struct MgCoarse {
     const T* res;
     const T* bf;
     T* xxf;
+    MgPacked<T> pk;
 };
 
 // The tail of k_mg_coarse: levels l0 .. L, a thread for every row of all of
@@ -1221,12 +1365,13 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
     const MgLevelDesc& d = a.lv[i];
     const MgLevelDesc& dp = a.lv[tail ? i : i + 1];
     const int t = ((int) blockIdx.x - a.first[i]) * a.each + tid;
+    const int g = ((int) blockIdx.x - 1) * a.each + tid;
     const int P = t / C, q = t % C;
     const bool mine = !tail && tid < a.each;
     int np = 0, Kc = -1;
     if (mine) {
         np = a.nd[a.lc + i + 1];
-        Kc = P < dp.cap ? dp.child[(size_t) q * dp.cap + P] : -1;
+        Kc = a.pk.row[g];
     }
     if (tid == 0) {
         s_half = *(volatile const int*) a.epoch & 1;
@@ -1259,37 +1404,26 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             for (int k = t; k < 2 * d.cap; k += threads) mg_open<T>(places(d, half ^ 1, 0) + k);
         }
         if ((t & ~63) / C < np) {  // else no row of this wavefront exists
-            const bool live = P < np && Kc >= 0;
-            // a thread without a row follows one of its wavefront that has (each
-            // parent has a child) and stores nothing: with all of them on one
-            // row, its places were polled thousands of times at once
-            const unsigned long long rows = __ballot(live);  // all lanes are here: not inside the choice below
-            const int some = __shfl(Kc, rows ? __ffsll(rows) - 1 : 0, 64);
-            const int K = live ? Kc : (rows ? some : 0);
-            const T* const val = (const T*) d.val;
-            const T* const dinv = (const T*) d.dinv;
-            int at[W + 1], ag[W + 1];
-            T v[W], pre[W], bb[W + 1];
+            const bool live = Kc >= 0;
+            const int K = live ? Kc : ~Kc;  // without a row: another's, and nothing is stored
+            const size_t n = (size_t) a.pk.n;
+            int at[W], ag[C];
+            T v[W], pre[W], bb[W];
+#pragma unroll
+            for (int j = 0; j < W; j++) at[j] = a.pk.at[j * n + g];
 #pragma unroll
             for (int j = 0; j < W; j++) {
-                at[j] = d.col[(size_t) j * d.cap + K];
-                v[j] = val[(size_t) j * d.cap + K];  // 0 where there is no neighbour
+                v[j] = a.pk.val[j * n + g];  // 0 where there is no neighbour
+                pre[j] = a.pk.dinv[j * n + g];
             }
-            const T dK = dinv[K], gK = ((const T*) d.diag)[K];
-            ag[W] = d.agg[K];
+#pragma unroll
+            for (int c = 0; c < C; c++) ag[c] = a.pk.up[c * n + g];
+            const T dK = pre[W / 2], gK = a.pk.diag[g];
             const bool pro = a.xxf && top;
             int f0 = 0, f1 = 0;
             if (pro || sums) {
                 f0 = a.cst1[K];
                 f1 = a.cst1[K + 1];
-            }
-#pragma unroll
-            for (int j = 0; j < W; j++) at[j] = at[j] >= 0 ? at[j] : K;
-            at[W] = K;
-#pragma unroll
-            for (int j = 0; j < W; j++) {
-                pre[j] = dinv[at[j]];
-                ag[j] = d.agg[at[j]];
             }
             T bf[kMgProRows];
             if (sums) {  // in row order, as cell_sum
@@ -1305,7 +1439,7 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             } else if (top) {
                 const T* const b = (const T*) d.b;
 #pragma unroll
-                for (int j = 0; j <= W; j++) bb[j] = b[at[j]];
+                for (int j = 0; j < W; j++) bb[j] = b[at[j]];
             }
             if (pro) {
 #pragma unroll
@@ -1315,8 +1449,8 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             const bool many = W > 9 || a.nd[a.lc + i] > kMgPollMost;
             // (where the thread itself has put its own value: a neighbour's)
             if (!top || sums)
-                ok = mg_get<T, W + 1>(places(d, half, 0), at, bb, many ? (sums ? at[0] : K) : -1, a.polls);
-            const T bK = bb[W];
+                ok = mg_get<T, W>(places(d, half, 0), at, bb, many ? (sums ? at[0] : K) : -1, a.polls);
+            const T bK = bb[W / 2];
             {
                 T acc = gK * (a.omega * bK * dK);
 #pragma unroll
@@ -1329,9 +1463,10 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
                 if (P < np && q == 0) mg_put<T>(places(dp, half, 0) + P, res);
             }
             // up
-            T xv[W + 1];
-            ok = mg_get<T, W + 1>(places(dp, half, 1), ag, xv, top || many ? ag[W] : -1, a.polls) && ok;
-            const T xx = mg_own_corrected(a.omega, bK, dK, a.cf, xv[W]);
+            T xp[C], xv[W];
+            ok = mg_get<T, C>(places(dp, half, 1), ag, xp, top || many ? ag[0] : -1, a.polls) && ok;
+            mg_of_parents<T, W, C>(xp, q, xv);
+            const T xx = mg_own_corrected(a.omega, bK, dK, a.cf, xp[0]);
             T acc = gK * xx;
 #pragma unroll
             for (int j = 0; j < W; j++) acc = mg_fma(v[j], mg_corrected(pre[j], a.cf, xv[j]), acc);
@@ -1486,6 +1621,8 @@ struct MgWork {
     int* epoch = nullptr;
     int xch_key[3] = {};
     bool xch_new = false;            // some level's places were reallocated
+    void* pack = nullptr;            // MgPacked's arrays
+    size_t pack_cap = 0;             // its bytes
 };
 
 void mg_set_params(MgWork* m, double omega, double cf, int sweeps) {
@@ -1545,7 +1682,7 @@ void mg_destroy(MgWork* m) {
         hipFree(m->d_goff[l]);
     }
     void* ps[] = {m->nd,  m->err,   m->cst1,  m->head,     m->hscan, m->rkey,     m->agg0b,
-                  m->res0, m->xx0, m->flag, m->pscan, m->scan_tmp, m->desc, m->lsz, m->epoch};
+                  m->res0, m->xx0, m->flag, m->pscan, m->scan_tmp, m->desc, m->lsz, m->epoch, m->pack};
     for (void* p : ps) hipFree(p);
     mailbox_free(m->mb);
     delete m;
@@ -1696,6 +1833,66 @@ static bool mg_fine_additive(const MgWork* m, const Sell& A) {
     if (A.nseg != 1) return false;
     const size_t lim = m->fine_additive ? kMgAdditiveEntries - kMgAdditiveEntries / 8 : kMgAdditiveEntries;
     return A.entries >= lim;
+}
+
+// MgPacked in m->pack (sizes as planned).
+template <typename T>
+static MgPacked<T> mg_packed(const MgWork* m, size_t* bytes = nullptr) {
+    MgPacked<T> o{};
+    const int k1 = m->co_lt - m->lc;
+    const size_t n = (size_t) (m->co_first[k1] - 1) * m->co_each, W = (size_t) m->W, C = (size_t) m->C;
+    o.n = (int) n;
+    unsigned char* p = (unsigned char*) m->pack;
+    const auto take = [&](size_t b) {
+        unsigned char* const at = p;
+        p += (b + 255) & ~(size_t) 255;
+        return at;
+    };
+    o.val = (T*) take(sizeof(T) * W * n);
+    o.dinv = (T*) take(sizeof(T) * W * n);
+    o.diag = (T*) take(sizeof(T) * n);
+    o.at = (int*) take(sizeof(int) * W * n);
+    o.up = (int*) take(sizeof(int) * C * n);
+    o.row = (int*) take(sizeof(int) * n);
+    if (bytes) *bytes = (size_t) (p - (unsigned char*) m->pack);
+    return o;
+}
+
+// Packs the levels of k_mg_coarse once their operators are there.
+template <typename T>
+static hipError_t mg_pack(MgWork* m, int dim, hipStream_t st) {
+    const int k1 = m->co_lt - m->lc;
+    if (k1 <= 0) return hipSuccess;
+    size_t need = 0;
+    (void) mg_packed<T>(m, &need);
+    if (need > m->pack_cap) {
+        hipFree(m->pack);
+        m->pack = nullptr;
+        m->pack_cap = 0;
+        const size_t cap = need + need / 4;
+        hipError_t e = mg_alloc(&m->pack, cap);
+        if (e) return e;
+        m->pack_cap = cap;
+        m->gen++;
+    }
+    MgPackIn a{};
+    for (int k = 0; k <= k1; k++) {
+        a.lv[k] = m->hdesc[m->lc + k];
+        a.coord[k] = m->coord[m->lc + k];
+        a.scene[k] = m->scene[m->lc + k];
+        a.dims[k] = m->d_sdims[m->lc + k];
+        a.rows[k] = m->n[m->lc + k];
+        a.first[k] = m->co_first[k];
+    }
+    a.levels = k1;
+    a.each = m->co_each;
+    const MgPacked<T> o = mg_packed<T>(m);
+    const dim3 gr(m->co_first[k1] - 1), bl(m->co_each);
+    if (dim == 2)
+        hipLaunchKernelGGL((k_mg_pack<T, 9, 4>), gr, bl, 0, st, a, o);
+    else
+        hipLaunchKernelGGL((k_mg_pack<T, 27, 8>), gr, bl, 0, st, a, o);
+    return hipSuccess;
 }
 
 template <typename T, typename IDX>
@@ -1916,6 +2113,7 @@ static hipError_t mg_setup_t(MgWork* m, const Sell& A, const Hot& h, int dim, co
     for (int k = 1; k <= l; k++)
         m->hdesc[k] = MgLevelDesc{m->cap[k], 0,         m->col[k], m->val[k],   m->diag[k],
                                   m->dinv[k], m->agg[k], m->child[k], m->b[k], m->x[k], m->xch[k]};
+    if ((e = mg_pack<T>(m, dim, st))) return e;
     if (!m->up_desc_valid || std::memcmp(m->up_desc, m->hdesc, sizeof(m->hdesc)) != 0) {
         std::memcpy(m->up_desc, m->hdesc, sizeof(m->hdesc));
         m->up_desc_valid = true;
@@ -1987,6 +2185,7 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
         a.res = lc == 1 ? res : nullptr;
         a.bf = r;
         a.xxf = lc == 1 ? xf : nullptr;
+        a.pk = mg_packed<T>(m);
         hipLaunchKernelGGL((k_mg_coarse<T, W, C, BT>), dim3(m->co_first[k1]), dim3(BT), 0, st, a);
     } else {
         hipLaunchKernelGGL((k_mg_tail<T, W, C>), dim3(1), dim3(kMgTailThreads), kMgTailLds, st, m->desc, nd, lt, L,
