@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "mps_internal.hpp"
@@ -1214,6 +1215,40 @@ __global__ void __launch_bounds__(512) k_mg_pack(MgPackIn a, MgPacked<T> o) {
     }
 }
 
+// The fine level in k_mg_coarse (multiplicative cycle): a thread a row.  Its
+// residual goes to level 1 through places of its own and x of level 1 comes
+// back through level 1's, so the cycle is one launch.
+// Measured, 32k rows FP64 (2D): k_mg_down0 4.6 + k_mg_up0 4.8 us, 2 us of gaps
+// and this launch without them 14.0 -> 19.4 us; 36.1 -> 32.5 ms per 20 steps.
+// What is added to the launch is two exchanges (1.3 us each) and a row product.
+template <typename T>
+struct MgFine {
+    const int* slice_pos;
+    const void* col;
+    const int* anc;
+    const T* val;
+    const int* agg0;
+    T* u;
+    void* xch;  // 2 halves x cap values, all ones while not yet computed
+    int cap;
+};
+// Entries of a row that are kept in registers between the two products; the
+// rest is read again.  Rows wider than that on average are left to k_mg_down0
+// and k_mg_up0: what is read again waits for level 1 by fours.
+template <int W>
+constexpr int kMgFineEntries = W == 9 ? 16 : 36;
+
+template <typename T>
+__device__ __forceinline__ T mg_fine_residual(T omega, T b, T acc) {
+#pragma clang fp contract(fast)
+    return b - omega * acc;
+}
+template <typename T>
+__device__ __forceinline__ T mg_fine_smoothed(T xx, T omega, T b, T acc) {
+#pragma clang fp contract(fast)
+    return xx + omega * (b - acc);
+}
+
 template <typename T>
 struct MgCoarse {
     MgLevelDesc lv[kMgCoarseLevels];   // of levels lc ..
@@ -1234,6 +1269,7 @@ struct MgCoarse {
     const T* bf;
     T* xxf;
     MgPacked<T> pk;
+    MgFine<T> f;
 };
 
 // The tail of k_mg_coarse: levels l0 .. L, a thread for every row of all of
@@ -1350,7 +1386,72 @@ __device__ __forceinline__ void mg_tail_rows(const MgLevelDesc* __restrict__ lv,
 
 constexpr int kMgProRows = 8;  // fine rows of a cell in a round
 
-template <typename T, int W, int C, int BT>
+// Fine row r of the cycle (see MgFine); x1 is level 1's places of x.  Every
+// lane of a wavefront that has a row calls it.
+template <typename T, int W, typename IDX>
+__device__ __forceinline__ bool mg_fine_rows(const MgCoarse<T>& a, int r, int nr, typename MgBits<T>::U* put,
+                                             const typename MgBits<T>::U* x1) {
+    constexpr int E = kMgFineEntries<W>;
+    const MgFine<T>& f = a.f;
+    const bool live = r < nr;
+    const int row = live ? r : nr - 1;  // a lane past the rows follows the last one
+    const IDX* const col = (const IDX*) f.col;
+    const int s0 = f.slice_pos[row >> 6], w = f.slice_pos[(row >> 6) + 1] - s0;
+    const size_t base = (size_t) s0 * 64 + (row & 63);
+    int lo, hi;
+    sell_anchors<IDX>(f.anc, row, lo, hi);
+    int at[E + 1];
+    T v[E], bv[E];
+#pragma unroll
+    for (int k = 0; k < E; k++) {
+        at[k] = row;
+        v[k] = (T) 0;
+        if (k < w) {  // the same in every lane
+            at[k] = sell_col<IDX>(col, base + (size_t) k * 64, row, lo, hi);
+            v[k] = f.val[base + (size_t) k * 64];
+        }
+    }
+    const T b = a.bf[row];
+#pragma unroll
+    for (int k = 0; k < E; k++) bv[k] = a.bf[at[k]];
+    at[E] = f.agg0[row];
+#pragma unroll
+    for (int k = 0; k < E; k++) at[k] = f.agg0[at[k]];
+    T acc = b;
+#pragma unroll
+    for (int k = 0; k < E; k++) acc = mg_fma(v[k], bv[k], acc);
+    for (int k = E; k < w; k++) {
+        const size_t i = base + (size_t) k * 64;
+        acc = mg_fma(f.val[i], a.bf[sell_col<IDX>(col, i, row, lo, hi)], acc);
+    }
+    if (live) mg_put<T>(put + r, mg_fine_residual(a.omega, b, acc));
+    // up
+    T xv[E + 1];
+    bool ok = mg_get<T, E + 1>(x1, at, xv, at[E], a.polls);
+    const T xx = mg_fine_start(a.omega, b, a.cf, xv[E]);
+    acc = xx;
+#pragma unroll
+    for (int k = 0; k < E; k++) acc = mg_fma(v[k], mg_fine_start(a.omega, bv[k], a.cf, xv[k]), acc);
+    for (int k = E; k < w; k += 4) {
+        int c[4], ca[4];
+        T cv[4], cx[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const size_t i = base + (size_t) (k + j < w ? k + j : w - 1) * 64;
+            c[j] = sell_col<IDX>(col, i, row, lo, hi);
+            cv[j] = k + j < w ? f.val[i] : (T) 0;
+            ca[j] = f.agg0[c[j]];
+        }
+        ok = mg_get<T, 4>(x1, ca, cx, -1, a.polls) && ok;
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc = mg_fma(cv[j], mg_fine_start(a.omega, a.bf[c[j]], a.cf, cx[j]), acc);
+    }
+    if (live) f.u[r] = mg_fine_smoothed(xx, a.omega, b, acc);
+    return ok;
+}
+
+// IDX: the fine columns' type, void without the fine level.
+template <typename T, int W, int C, int BT, typename IDX>
 __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
     using U = typename MgBits<T>::U;
     __shared__ int s_half, s_bad;
@@ -1358,16 +1459,18 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
     __builtin_amdgcn_s_setprio(2);
     // the block's level (level lt: block 0, the tail) and the thread's row,
     // read together with the flags
+    constexpr bool kFine = !std::is_void<IDX>::value;
     int i = 0;
     while (i + 1 < a.lt - a.lc && (int) blockIdx.x >= a.first[i + 1]) i++;
     const bool tail = blockIdx.x == 0;
+    const bool fine = kFine && (int) blockIdx.x >= a.first[a.lt - a.lc];
     if (tail) i = a.lt - a.lc;
     const MgLevelDesc& d = a.lv[i];
     const MgLevelDesc& dp = a.lv[tail ? i : i + 1];
     const int t = ((int) blockIdx.x - a.first[i]) * a.each + tid;
     const int g = ((int) blockIdx.x - 1) * a.each + tid;
     const int P = t / C, q = t % C;
-    const bool mine = !tail && tid < a.each;
+    const bool mine = !tail && !fine && tid < a.each;
     int np = 0, Kc = -1;
     if (mine) {
         np = a.nd[a.lc + i + 1];
@@ -1395,9 +1498,17 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
                 return v[0];
             },
             [&](int K, T v) { mg_put<T>(xt + K, v); });
+    } else if (kFine && fine) {
+        if constexpr (kFine) {
+            const int r = ((int) blockIdx.x - a.first[a.lt - a.lc]) * BT + tid, nr = a.nd[0];
+            U* const xch = (U*) a.f.xch;
+            if (r < a.f.cap) mg_open<T>(xch + (size_t) (half ^ 1) * a.f.cap + r);
+            if ((r & ~63) < nr)
+                ok = mg_fine_rows<T, W, IDX>(a, r, nr, xch + (size_t) half * a.f.cap, places(a.lv[0], half, 1));
+        }
     } else if (mine) {
         const bool top = i == 0;
-        const bool sums = a.res && top;
+        const bool sums = (kFine || a.res) && top;
         // the next launch's half
         if (!top || a.lc == 1) {
             const int threads = (a.first[i + 1] - a.first[i]) * a.each;
@@ -1419,7 +1530,7 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
 #pragma unroll
             for (int c = 0; c < C; c++) ag[c] = a.pk.up[c * n + g];
             const T dK = pre[W / 2], gK = a.pk.diag[g];
-            const bool pro = a.xxf && top;
+            const bool pro = !kFine && a.xxf && top;
             int f0 = 0, f1 = 0;
             if (pro || sums) {
                 f0 = a.cst1[K];
@@ -1429,8 +1540,17 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             if (sums) {  // in row order, as cell_sum
                 T s = (T) 0;
                 for (int r = f0; r < f1; r += kMgProRows) {
+                    if constexpr (kFine) {
+                        int fr[kMgProRows];
 #pragma unroll
-                    for (int j = 0; j < kMgProRows; j++) bf[j] = a.res[r + j < f1 ? r + j : f1 - 1];
+                        for (int j = 0; j < kMgProRows; j++) fr[j] = r + j < f1 ? r + j : f1 - 1;
+                        ok = mg_get<T, kMgProRows>((const U*) a.f.xch + (size_t) half * a.f.cap, fr, bf, fr[0],
+                                                   a.polls) &&
+                             ok;
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < kMgProRows; j++) bf[j] = a.res[r + j < f1 ? r + j : f1 - 1];
+                    }
 #pragma unroll
                     for (int j = 0; j < kMgProRows; j++)
                         if (r + j < f1) s += bf[j];
@@ -1449,7 +1569,7 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             const bool many = W > 9 || a.nd[a.lc + i] > kMgPollMost;
             // (where the thread itself has put its own value: a neighbour's)
             if (!top || sums)
-                ok = mg_get<T, W>(places(d, half, 0), at, bb, many ? (sums ? at[0] : K) : -1, a.polls);
+                ok = mg_get<T, W>(places(d, half, 0), at, bb, many ? (sums ? at[0] : K) : -1, a.polls) && ok;
             const T bK = bb[W / 2];
             {
                 T acc = gK * (a.omega * bK * dK);
@@ -1472,8 +1592,8 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             for (int j = 0; j < W; j++) acc = mg_fma(v[j], mg_corrected(pre[j], a.cf, xv[j]), acc);
             const T xK = mg_smoothed(xx, a.omega, dK, bK, acc);
             if (live) {
-                if (!top) mg_put<T>(places(d, half, 1) + K, xK);
-                if (top && !pro) ((T*) d.x)[K] = xK;
+                if (kFine || !top) mg_put<T>(places(d, half, 1) + K, xK);
+                if (!kFine && top && !pro) ((T*) d.x)[K] = xK;
                 if (pro) {
                     for (int r = f0;;) {
 #pragma unroll
@@ -1619,8 +1739,10 @@ struct MgWork {
     int co_first[kMgCoarseLevels] = {};
     void* xch[kMgMaxLevels + 1] = {};
     int* epoch = nullptr;
-    int xch_key[3] = {};
+    int xch_key[4] = {};
     bool xch_new = false;            // some level's places were reallocated
+    int co_fine = 0;                 // blocks of the fine level in it (0: not there)
+    void* xch0 = nullptr;            // its places, for fcap rows
     void* pack = nullptr;            // MgPacked's arrays
     size_t pack_cap = 0;             // its bytes
 };
@@ -1682,7 +1804,7 @@ void mg_destroy(MgWork* m) {
         hipFree(m->d_goff[l]);
     }
     void* ps[] = {m->nd,  m->err,   m->cst1,  m->head,     m->hscan, m->rkey,     m->agg0b,
-                  m->res0, m->xx0, m->flag, m->pscan, m->scan_tmp, m->desc, m->lsz, m->epoch, m->pack};
+                  m->res0, m->xx0, m->flag, m->pscan, m->scan_tmp, m->desc, m->lsz, m->epoch, m->pack, m->xch0};
     for (void* p : ps) hipFree(p);
     mailbox_free(m->mb);
     delete m;
@@ -1766,7 +1888,7 @@ constexpr int kMgCoarseThreads = W == 27 && sizeof(T) == 8 ? 256 : 512;
 // the finest level whose blocks, with those of the levels below, all run at
 // once (counted one a CU).
 template <typename T>
-static hipError_t mg_coarse_plan(MgWork* m, int dim, hipStream_t st) {
+static hipError_t mg_coarse_plan(MgWork* m, int dim, bool fine_ok, hipStream_t st) {
     const int bt = dim == 2 ? kMgCoarseThreads<T, 9> : kMgCoarseThreads<T, 27>;
     int lt = m->L + 1, rows = 0;
     while (lt > 1 && rows + m->n[lt - 1] <= bt) {
@@ -1780,18 +1902,32 @@ static hipError_t mg_coarse_plan(MgWork* m, int dim, hipStream_t st) {
     // rows 2), up to three quarters of the blocks there may be
     int lc = lt, each = bt, first[kMgCoarseLevels] = {};
     const auto blocks = [&](int l, int rows) { return (m->C * m->cap[l + 1] + rows - 1) / rows; };
-    if (lt <= m->L) {
+    const auto choose = [&](int most) {
         int sum = 1;
-        while (lc > 1 && lt - lc + 2 <= kMgCoarseLevels && sum + blocks(lc - 1, bt) <= m->co_most)
+        lc = lt;
+        each = bt;
+        while (lc > 1 && lt - lc + 2 <= kMgCoarseLevels && sum + blocks(lc - 1, bt) <= most)
             sum += blocks(--lc, bt);
         for (int rows = 64; rows < bt; rows *= 2) {
             sum = 1;
             for (int l = lc; l < lt; l++) sum += blocks(l, rows);
-            if (sum <= m->co_most - m->co_most / 4) {
+            if (sum <= most - most / 4) {
                 each = rows;
                 break;
             }
         }
+    };
+    int fine = 0;
+    if (lt <= m->L) {
+        // the fine level too where its blocks fit beside those of all levels:
+        // up to some 65k rows in 2D (a level left to launches of its own would
+        // cost more than the two that the fine level saves)
+        const int fb = (m->fcap + bt - 1) / bt;
+        if (fine_ok && fb < m->co_most) {
+            choose(m->co_most - fb);
+            if (lc == 1 && lc < lt) fine = fb;
+        }
+        if (!fine) choose(m->co_most);
         int f = 1;
         for (int l = lc; l < lt; l++) {
             first[l - lc] = f;
@@ -1799,17 +1935,20 @@ static hipError_t mg_coarse_plan(MgWork* m, int dim, hipStream_t st) {
         }
         if (lc < lt) first[lt - lc] = f;
     }
-    if (lc != m->lc || lt != m->co_lt || each != m->co_each || std::memcmp(first, m->co_first, sizeof first) != 0)
+    if (lc != m->lc || lt != m->co_lt || each != m->co_each || fine != m->co_fine ||
+        std::memcmp(first, m->co_first, sizeof first) != 0)
         m->gen++;
     m->lc = lc;
     m->co_lt = lt;
     m->co_each = each;
+    m->co_fine = fine;
     std::memcpy(m->co_first, first, sizeof first);
-    const int key[3] = {lc, lt, (int) sizeof(T)};
+    const int key[4] = {lc, lt, (int) sizeof(T), fine};
     if (lc < lt && (m->xch_new || std::memcmp(key, m->xch_key, sizeof key) != 0)) {
         hipError_t e;
         for (int l = lc; l <= lt; l++)
             if ((e = fill_int((int*) m->xch[l], -1, 8 * (size_t) m->cap[l], st))) return e;
+        if ((e = fill_int((int*) m->xch0, -1, 4 * (size_t) m->fcap, st))) return e;
         if ((e = fill_int(m->epoch, 0, 2, st))) return e;
         std::memcpy(m->xch_key, key, sizeof key);
         m->xch_new = false;
@@ -1817,7 +1956,7 @@ static hipError_t mg_coarse_plan(MgWork* m, int dim, hipStream_t st) {
     return hipSuccess;
 }
 
-int mg_coarse_groups(const MgWork* m) { return m && m->lc < m->co_lt ? m->co_first[m->co_lt - m->lc] : 0; }
+int mg_coarse_groups(const MgWork* m) { return m && m->lc < m->co_lt ? m->co_first[m->co_lt - m->lc] + m->co_fine : 0; }
 void mg_coarse_off(MgWork* m) {
     m->co_most = 0;
     m->lc = m->co_lt;
@@ -1927,13 +2066,15 @@ static hipError_t mg_setup_t(MgWork* m, const Sell& A, const Hot& h, int dim, co
         if ((e = mg_alloc(&m->desc, sizeof(MgLevelDesc) * (kMgMaxLevels + 1)))) return e;
     }
     if (R > m->fcap) {
-        void* ps[] = {m->head, m->hscan, m->rkey, m->res0, m->xx0, m->cst1, m->agg0b};
+        void* ps[] = {m->head, m->hscan, m->rkey, m->res0, m->xx0, m->cst1, m->agg0b, m->xch0};
         for (void* p : ps) hipFree(p);
+        m->xch0 = nullptr;
+        m->xch_new = true;
         const int cap = R + R / 4 + 1024;
         if ((e = mg_alloc(&m->head, sizeof(int) * (size_t) cap)) || (e = mg_alloc(&m->hscan, sizeof(int) * (cap + 1))) ||
             (e = mg_alloc(&m->agg0b, (size_t) cap)) ||
             (e = mg_alloc(&m->rkey, sizeof(int) * (size_t) cap)) || (e = mg_alloc(&m->res0, 8 * (size_t) cap)) ||
-            (e = mg_alloc(&m->xx0, 8 * (size_t) cap)) || (e = mg_alloc(&m->cst1, sizeof(int) * (cap + 1))))
+            (e = mg_alloc(&m->xx0, 8 * (size_t) cap)) || (e = mg_alloc(&m->xch0, 2 * 8 * (size_t) cap)) || (e = mg_alloc(&m->cst1, sizeof(int) * (cap + 1))))
             return e;
         m->fcap = cap;
         m->gen++;
@@ -2109,7 +2250,9 @@ static hipError_t mg_setup_t(MgWork* m, const Sell& A, const Hot& h, int dim, co
     }
     if (tail != m->tail) m->gen++;
     m->tail = tail;
-    if ((e = mg_coarse_plan<T>(m, dim, st))) return e;
+    const int most_w = dim == 2 ? kMgFineEntries<9> : kMgFineEntries<27>;
+    const bool fine_ok = !m->fine_additive && sizeof(IDX) == 2 && A.entries <= (size_t) most_w * R;
+    if ((e = mg_coarse_plan<T>(m, dim, fine_ok, st))) return e;
     for (int k = 1; k <= l; k++)
         m->hdesc[k] = MgLevelDesc{m->cap[k], 0,         m->col[k], m->val[k],   m->diag[k],
                                   m->dinv[k], m->agg[k], m->child[k], m->b[k], m->x[k], m->xch[k]};
@@ -2148,11 +2291,12 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
     T* res0 = (T*) m->res0;
     T* xx0 = (T*) m->xx0;
     const bool add = m->fine_additive;
-    if (!add)
+    const bool one = m->lc < m->co_lt;  // levels lc .. L in k_mg_coarse
+    const bool fine = one && m->co_fine > 0;  // and the fine level
+    if (!add && !fine)
         hipLaunchKernelGGL((k_mg_down0<T, IDX>), mg_grid(m->cap[0]), dim3(kBlock), 0, st, nd + 0, A.slice_off, fcol,
                            A.anc, fval, r, res0, om, done);
     // level 1's right-hand side: k_mg_coarse sums it where it takes level 1
-    const bool one = m->lc < m->co_lt;  // levels lc .. L in k_mg_coarse
     const int lc = one ? m->lc : lt;
     const T* const res = add ? (b1_given ? nullptr : r) : (const T*) res0;
     if (res && !(one && lc == 1))
@@ -2186,7 +2330,13 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
         a.bf = r;
         a.xxf = lc == 1 ? xf : nullptr;
         a.pk = mg_packed<T>(m);
-        hipLaunchKernelGGL((k_mg_coarse<T, W, C, BT>), dim3(m->co_first[k1]), dim3(BT), 0, st, a);
+        a.f = MgFine<T>{A.slice_off, fcol, A.anc, fval, m->agg[0], u, m->xch0, m->fcap};
+        if constexpr (sizeof(IDX) == 2) {
+            if (fine)
+                hipLaunchKernelGGL((k_mg_coarse<T, W, C, BT, IDX>), dim3(m->co_first[k1] + m->co_fine), dim3(BT), 0, st,
+                                   a);
+        }
+        if (!fine) hipLaunchKernelGGL((k_mg_coarse<T, W, C, BT, void>), dim3(m->co_first[k1]), dim3(BT), 0, st, a);
     } else {
         hipLaunchKernelGGL((k_mg_tail<T, W, C>), dim3(1), dim3(kMgTailThreads), kMgTailLds, st, m->desc, nd, lt, L,
                            om, cf, m->sweeps, done);
@@ -2204,7 +2354,7 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
     else if (!one)
         hipLaunchKernelGGL((k_mg_prolong0<T>), mg_grid(m->cap[0]), dim3(kBlock), 0, st, nd + 0, r, m->agg[0],
                            (const T*) m->x[1], xf, om, cf, done);
-    if (!add)
+    if (!add && !fine)
         hipLaunchKernelGGL((k_mg_up0<T, IDX>), mg_grid(m->cap[0]), dim3(kBlock), 0, st, nd + 0, A.slice_off, fcol,
                            A.anc, fval, r, xx0, u, om, done);
 }
