@@ -1385,6 +1385,13 @@ __device__ __forceinline__ void mg_tail_rows(const MgLevelDesc* __restrict__ lv,
 }
 
 constexpr int kMgProRows = 8;  // fine rows of a cell in a round
+// Lanes that share a cell in the fine level's first step up, in 3D and in
+// blocks of kMgProShared rows or more.  There a lane a cell (20 rows) made every
+// load and store of a wavefront some 50 lines, 5-14 us of the 42 us a cycle at
+// 1M particles mixed, 512 rows a block: 42 -> 35 us.  With one wavefront a block
+// (101k FP64, 64 rows) sharing is slower, 23.5 -> 25.3 us, and in 2D (9 rows a
+// cell, 256 rows a block) 18.3 -> 18.8.
+constexpr int kMgProLanes = 32, kMgProShared = 256;
 
 // Fine row r of the cycle (see MgFine); x1 is level 1's places of x.  Every
 // lane of a wavefront that has a row calls it.
@@ -1561,7 +1568,18 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
 #pragma unroll
                 for (int j = 0; j < W; j++) bb[j] = b[at[j]];
             }
-            if (pro) {
+            constexpr int G = kMgProLanes;
+            T bp[W == 27 ? G : 1];
+            const int sub = tid & (G - 1), grp = (tid & 63) / G;
+            const bool share = pro && W == 27 && a.each >= kMgProShared;
+            if (share) {
+                if (!live) f1 = f0;
+#pragma unroll
+                for (int j = 0; j < (W == 27 ? G : 0); j++) {
+                    const int c = j * (64 / G) + grp, r = __shfl(f0, c, 64) + sub;
+                    bp[j] = r < __shfl(f1, c, 64) ? a.bf[r] : (T) 0;
+                }
+            } else if (pro) {
 #pragma unroll
                 for (int j = 0; j < kMgProRows; j++) bf[j] = a.bf[f0 + j < f1 ? f0 + j : f0];
             }
@@ -1594,7 +1612,7 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
             if (live) {
                 if (kFine || !top) mg_put<T>(places(d, half, 1) + K, xK);
                 if (!kFine && top && !pro) ((T*) d.x)[K] = xK;
-                if (pro) {
+                if (pro && !share) {
                     for (int r = f0;;) {
 #pragma unroll
                         for (int j = 0; j < kMgProRows; j++)
@@ -1604,6 +1622,16 @@ __global__ void __launch_bounds__(BT) k_mg_coarse(MgCoarse<T> a) {
 #pragma unroll
                         for (int j = 0; j < kMgProRows; j++) bf[j] = a.bf[r + j < f1 ? r + j : f0];
                     }
+                }
+            }
+            if (share) {
+#pragma unroll
+                for (int j = 0; j < (W == 27 ? G : 0); j++) {
+                    const int c = j * (64 / G) + grp, e = __shfl(f1, c, 64);
+                    const T xc = __shfl(xK, c, 64);
+                    int r = __shfl(f0, c, 64) + sub;
+                    if (r < e) a.xxf[r] = mg_fine_start(a.omega, bp[j], a.cf, xc);
+                    for (r += G; r < e; r += G) a.xxf[r] = mg_fine_start(a.omega, a.bf[r], a.cf, xc);
                 }
             }
         }
