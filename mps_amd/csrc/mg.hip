@@ -1221,6 +1221,10 @@ __global__ void __launch_bounds__(512) k_mg_pack(MgPackIn a, MgPacked<T> o) {
 // Measured, 32k rows FP64 (2D): k_mg_down0 4.6 + k_mg_up0 4.8 us, 2 us of gaps
 // and this launch without them 14.0 -> 19.4 us; 36.1 -> 32.5 ms per 20 steps.
 // What is added to the launch is two exchanges (1.3 us each) and a row product.
+// Steps by launches -> in it: 2D 10k rows FP64 1.39 -> 1.34 ms, mixed 1.80 ->
+// 1.70; 46k 1.93 -> 1.74, 2.23 -> 2.06; 82k (the most that fit) 2.08 -> 1.97,
+// 2.09 -> 2.04.  3D FP64 10k 2.30 -> 2.06, 32k 2.60 -> 2.42; 3D mixed, whose
+// blocks take 512 rows of 32 entries, 19k 2.11 -> 2.15, 32k 2.60 -> 2.62.
 template <typename T>
 struct MgFine {
     const int* slice_pos;
@@ -1948,7 +1952,7 @@ static hipError_t mg_coarse_plan(MgWork* m, int dim, bool fine_ok, hipStream_t s
     int fine = 0;
     if (lt <= m->L) {
         // the fine level too where its blocks fit beside those of all levels:
-        // up to some 65k rows in 2D (a level left to launches of its own would
+        // up to some 80k rows in 2D, 35k in 3D (a level left to launches of its own would
         // cost more than the two that the fine level saves)
         const int fb = (m->fcap + bt - 1) / bt;
         if (fine_ok && fb < m->co_most) {
@@ -2278,8 +2282,10 @@ static hipError_t mg_setup_t(MgWork* m, const Sell& A, const Hot& h, int dim, co
     }
     if (tail != m->tail) m->gen++;
     m->tail = tail;
+    // 3D in FP32 is left out (see MgFine)
     const int most_w = dim == 2 ? kMgFineEntries<9> : kMgFineEntries<27>;
-    const bool fine_ok = !m->fine_additive && sizeof(IDX) == 2 && A.entries <= (size_t) most_w * R;
+    const bool fine_ok = !m->fine_additive && sizeof(IDX) == 2 && (dim == 2 || sizeof(T) == 8) &&
+                         A.entries <= (size_t) most_w * R;
     if ((e = mg_coarse_plan<T>(m, dim, fine_ok, st))) return e;
     for (int k = 1; k <= l; k++)
         m->hdesc[k] = MgLevelDesc{m->cap[k], 0,         m->col[k], m->val[k],   m->diag[k],
@@ -2359,7 +2365,7 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
         a.xxf = lc == 1 ? xf : nullptr;
         a.pk = mg_packed<T>(m);
         a.f = MgFine<T>{A.slice_off, fcol, A.anc, fval, m->agg[0], u, m->xch0, m->fcap};
-        if constexpr (sizeof(IDX) == 2) {
+        if constexpr (sizeof(IDX) == 2 && (W == 9 || sizeof(T) == 8)) {
             if (fine)
                 hipLaunchKernelGGL((k_mg_coarse<T, W, C, BT, IDX>), dim3(m->co_first[k1] + m->co_fine), dim3(BT), 0, st,
                                    a);
