@@ -211,8 +211,15 @@ int mps_clear_debug_events(mps_handle* h);
  *   out[7] = CG iterations enqueued by the handle's solves, counting those
  *            of a chunk that return at once after convergence,
  *   out[8] = CG chunk graphs captured (one per solver and chunk length while
- *            the pointers they bake in stay; out[0] counts the drops).
- * Writes min(cap, 9) values. */
+ *            the pointers they bake in stay; out[0] counts the drops),
+ *   out[9] = solves that ran as one resident launch,
+ *   out[10] = resident launches that gave up,
+ *   out[11] = of out[7], those whose multigrid cycle took the coarse launch,
+ *   out[12] = of out[11], those with the fine level in it,
+ *   out[13] = solves whose coarse launch gave up,
+ *   out[14] = solves refused a resident or coarse launch because other
+ *            handles held the workgroups.
+ * Writes min(cap, 15) values. */
 int mps_debug_counters(const mps_handle* h, int64_t* out, int32_t cap);
 
 /* Bucket grid geometry (src/bucket.hpp:11-14). */

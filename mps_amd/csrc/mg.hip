@@ -1989,6 +1989,7 @@ static hipError_t mg_coarse_plan(MgWork* m, int dim, bool fine_ok, hipStream_t s
 }
 
 int mg_coarse_groups(const MgWork* m) { return m && m->lc < m->co_lt ? m->co_first[m->co_lt - m->lc] + m->co_fine : 0; }
+bool mg_coarse_fine(const MgWork* m) { return mg_coarse_groups(m) > 0 && m->co_fine > 0; }
 void mg_coarse_off(MgWork* m) {
     m->co_most = 0;
     m->lc = m->co_lt;

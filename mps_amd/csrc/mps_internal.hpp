@@ -1168,6 +1168,7 @@ void mg_cycle(MgWork* m, const Sell& A, const IDX* fcol, const T* fval, const T*
 // has none); a launch that had to wait too long sets every done flag to 2,
 // and the caller switches it off and solves again (the bits are the same).
 int mg_coarse_groups(const MgWork* m);
+bool mg_coarse_fine(const MgWork* m);  // the fine level is in it
 void mg_coarse_off(MgWork* m);
 // When the current hierarchy's cycle restricts the fine residual r itself
 // (the additive fine level): the first fine row of each level-1 cell
@@ -1189,7 +1190,12 @@ void cg_prediction_bank(CgWork* cw, int bank);
 hipError_t stage_stats_read(long long out[4]);
 hipError_t cg_reserve(CgWork* cw, int rows);
 // [0] times a solver's cached graphs were dropped, [1] CG vector reallocations
-void cg_debug_counts(const CgWork* cw, long long out[4]);
+// [2] CG iterations enqueued, [3] chunk graphs captured, [4] resident solves,
+// [5] resident launches that gave up, [6] iterations with the coarse launch,
+// [7] of those with the fine level in it, [8] coarse launches that gave up,
+// [9] solves refused either launch for want of workgroups
+constexpr int kCgCounts = 10;
+void cg_debug_counts(const CgWork* cw, long long out[kCgCounts]);
 // Solves A x = b for the Inner rows.  b_s / x_s in slot order; x0_id (id order,
 // may be NULL) gives the warm start.  Fills stats.
 // stats: one entry per segment.

@@ -746,6 +746,12 @@ struct CgWork {
     long long graph_rebuilds = 0;  // times a solver's cached graphs were dropped
     long long vec_reallocs = 0;    // times the CG vectors were reallocated
     long long launched = 0;        // CG iterations enqueued, including those past convergence
+    long long coarse = 0;          // of those, with the cycle's coarse launch
+    long long coarse_fine = 0;     // and the fine level in it
+    long long coarse_gave_up = 0;  // solves done again because it waited too long
+    long long resident = 0;        // resident solves
+    long long resident_gave_up = 0;
+    long long refused = 0;         // solves refused either launch for want of workgroups
     // resident solves (resident.hip): exchange memory, the last tag handed
     // out, the most workgroups that can run at once (0: off, as set by
     // MPS_AMD_CG_RESIDENT=0 or after a launch that gave up), the launches'
@@ -879,11 +885,17 @@ bool tight_caps() {
     return v && atoi(v) != 0;
 }
 
-void cg_debug_counts(const CgWork* cw, long long out[4]) {
+void cg_debug_counts(const CgWork* cw, long long out[kCgCounts]) {
     out[0] = cw->graph_rebuilds;
     out[1] = cw->vec_reallocs;
     out[2] = cw->launched;
     out[3] = cw->graph_captures;
+    out[4] = cw->resident;
+    out[5] = cw->resident_gave_up;
+    out[6] = cw->coarse;
+    out[7] = cw->coarse_fine;
+    out[8] = cw->coarse_gave_up;
+    out[9] = cw->refused;
 }
 
 hipError_t cg_reserve(CgWork* cw, int rows) {
@@ -1034,6 +1046,10 @@ static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* c
         }
         launched += chunk;
         cw->launched += chunk;
+        if (cw->mg_on && mg_coarse_groups(cw->mg) > 0) {
+            cw->coarse += chunk;
+            if (mg_coarse_fine(cw->mg)) cw->coarse_fine += chunk;
+        }
         if (o.use_graph) {
             int slot = -1;
             for (int j = 0; j < CgWork::kGraphSlots; j++)
@@ -1267,7 +1283,10 @@ static hipError_t resident_solve(CgWork* cw, const Sell& A, const Hot& h, const 
     const long long span = resident_tags(its, max_ref);
     if (span > 0x40000000ll) return hipSuccess;
     ResidentGroups groups;
-    if (!groups.take(cw->res_dev, shape.split * cw->total_blocks, cw->res_most)) return hipSuccess;
+    if (!groups.take(cw->res_dev, shape.split * cw->total_blocks, cw->res_most)) {
+        cw->refused++;
+        return hipSuccess;
+    }
     hipError_t e = resident_reserve(cw, A.rows, st);
     if (!e && cw->tag > 0xffffffffu - (unsigned) span) {  // tags none of the words has held
         cw->tag = 0;
@@ -1333,9 +1352,11 @@ static hipError_t resident_solve(CgWork* cw, const Sell& A, const Hot& h, const 
     }
     if (bail) {  // a halo too large, or CUs held by others: this handle stays with the kernels
         cw->res_groups = 0;
+        cw->resident_gave_up++;
         return hipSuccess;
     }
     cw->launched += it;
+    cw->resident++;
     for (int k = 0; k < cw->nseg; k++) {
         const ResidentOut& r = cw->res_out[k];
         stats[k].rows = cw->h_row[k + 1] - cw->h_row[k];
@@ -1422,14 +1443,17 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
     // in for the whole solve
     ResidentGroups groups;
     if (cw->mg_on && mg_coarse_groups(cw->mg) > 0 &&
-        !groups.take(cw->res_dev, mg_coarse_groups(cw->mg), cw->res_most))
+        !groups.take(cw->res_dev, mg_coarse_groups(cw->mg), cw->res_most)) {
+        cw->refused++;
         mg_coarse_off(cw->mg);
+    }
     const auto gave_up = [&]() {
         for (int s = 0; s < nseg; s++)
             if (cw->host[s].done == 2) return true;
         return false;
     };
     const auto again = [&]() {  // from the start, by a launch a level
+        cw->coarse_gave_up++;
         mg_coarse_off(cw->mg);
         groups.give_back();
         return cg_solve(cw, A, h, n, b_s, pprev_id, pprev2_id, x_s, o, stats, st, msg);

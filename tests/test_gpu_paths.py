@@ -1,0 +1,160 @@
+"""Which launches a solve took.  The tests that compare a launch's bits with
+those of the launches it replaces would pass as well if it never ran, so the
+same scenes are run here for their counters."""
+import threading
+
+import numpy as np
+import pytest
+
+from mps_amd import capi, configs
+from test_gpu_coarse import FP64, MIXED, _run, _same, _scene
+from test_gpu_resident import SCENES, _scene_2d
+
+pytestmark = pytest.mark.gpu
+
+PRECISIONS = pytest.mark.parametrize("precision", [FP64, MIXED])
+ENV = ("MPS_AMD_MG_COARSE", "MPS_AMD_MG_FINE", "MPS_AMD_CG_RESIDENT", "MPS_AMD_CG_RESIDENT_HALO")
+
+
+def _sim(members, precision, multigrid, monkeypatch, env=None, **opt):
+    for k in ENV:
+        monkeypatch.delenv(k, raising=False)
+    for k, v in (env or {}).items():
+        monkeypatch.setenv(k, v)
+    sim = capi.Simulation(members) if len(members) > 1 else capi.Simulation(*members[0])
+    pre = capi.MPS_PRECOND_MULTIGRID if multigrid else capi.MPS_PRECOND_JACOBI
+    sim.set_solver(precision=precision, tolerance=1e-12, warm_start=True, preconditioner=pre, **opt)
+    sim.load_initial_state()
+    return sim
+
+
+def _counts(*args, steps=2, **kw):
+    sim = _sim(*args, **kw)
+    for _ in range(steps):
+        sim.step()
+    c = sim.debug_counters()
+    sim.close()
+    return c
+
+
+# ---- the coarse launch of the multigrid cycle
+
+
+@PRECISIONS
+@pytest.mark.parametrize("coarse", [None, "60", "12"])
+@pytest.mark.parametrize("dim,n", [(2, (110, 80)), (2, (251, 139)), (2, (502, 403)), (3, (22, 20, 21)),
+                                   (3, (41, 30, 33))])
+def test_coarse_launch_runs(dim, n, coarse, precision, monkeypatch):
+    c = _counts([_scene(dim, *n)], precision, True, monkeypatch, {"MPS_AMD_MG_COARSE": coarse} if coarse else None)
+    assert c["coarse_cycles"] == c["cg_launched"] > 0 and c["coarse_gave_up"] == c["refused"] == 0, c
+
+
+@PRECISIONS
+def test_coarse_launch_runs_with_options_and_scenes(precision, monkeypatch):
+    one, three = [_scene(2, 251, 139)], [_scene(2, 120, 90), _scene(2, 60, 61), _scene(2, 9, 7)]
+    for c in (_counts(one, precision, True, monkeypatch, {"MPS_AMD_MG_FINE": "additive"}),
+              _counts(one, precision, True, monkeypatch, use_graph=False),
+              _counts(three, precision, True, monkeypatch)):
+        assert c["coarse_cycles"] == c["cg_launched"] > 0, c
+    c = _counts(one, precision, True, monkeypatch, {"MPS_AMD_MG_COARSE": "0"})
+    assert c["coarse_cycles"] == 0 < c["cg_launched"], c
+
+
+@PRECISIONS
+def test_coarse_launch_gives_up(precision, monkeypatch):
+    c = _counts([_scene(2, 110, 80)], precision, True, monkeypatch, {"MPS_AMD_MG_COARSE": "256,1"})
+    assert c["coarse_gave_up"] == 1, c
+
+
+@PRECISIONS
+@pytest.mark.parametrize("dim,n,fits", [(2, (203, 207), True), (2, (420, 330), False), (3, (27, 25, 26), True)])
+def test_fine_level_in_the_coarse_launch(dim, n, fits, precision, monkeypatch):
+    c = _counts([_scene(dim, *n)], precision, True, monkeypatch)
+    if dim == 3 and precision == MIXED:
+        fits = False  # its fine level stays with its own launches
+    assert c["coarse_fine_cycles"] == (c["coarse_cycles"] if fits else 0), c
+    assert c["coarse_cycles"] > 0
+
+
+# the fewest rows but two that take the multigrid cycle (8,192); rows that
+# end at a wavefront
+@PRECISIONS
+@pytest.mark.parametrize("n,rows", [((85, 92), 8194), ((86, 96), 8640)])
+def test_fine_level_of_the_fewest_rows(n, rows, precision, monkeypatch):
+    m = [_scene(2, *n)]
+    sim = _sim(m, precision, True, monkeypatch)
+    sim.step()
+    assert sim.solver_stats()["rows"] == rows
+    sim.step()
+    c = sim.debug_counters()
+    sim.close()
+    assert c["coarse_fine_cycles"] == c["cg_launched"] > 0, c
+    _same(_run(m, precision, monkeypatch, None), _run(m, precision, monkeypatch, "0"))
+
+
+@PRECISIONS
+def test_fine_level_with_rows_wider_than_it_keeps(precision, monkeypatch):
+    s, sc = _scene(2, 140, 120)
+    c = (sc.pos[:, 0] < 0.25) & (sc.pos[:, 1] < 0.25) & (sc.type == 0)
+    sc.pos[c, 0] *= 0.8
+    sim = _sim([(s, sc)], precision, True, monkeypatch)
+    sim.set_snapshot(True)
+    sim.step()
+    widest = int(np.diff(sim.pressure_system()["row_ptr"]).max())
+    counts = sim.debug_counters()
+    sim.close()
+    assert widest > 16 and counts["coarse_fine_cycles"] == counts["cg_launched"] > 0, (widest, counts)
+
+
+def test_fine_level_while_the_rows_change(monkeypatch):
+    sim = _sim([_scene(2, 130, 101)], MIXED, True, monkeypatch)
+    rows = set()
+    for _ in range(12):
+        sim.step()
+        rows.add(sim.solver_stats()["rows"])
+    c = sim.debug_counters()
+    sim.close()
+    assert len(rows) > 1 and c["coarse_fine_cycles"] == c["cg_launched"] > 0, (rows, c)
+
+
+# ---- resident solves
+
+
+@PRECISIONS
+@pytest.mark.parametrize("name", sorted(SCENES))
+def test_resident_solve_runs(name, precision, monkeypatch):
+    c = _counts([SCENES[name]()], precision, False, monkeypatch)
+    assert c["resident_solves"] == 2 and c["resident_gave_up"] == c["refused"] == 0, c
+
+
+@PRECISIONS
+def test_resident_solve_runs_with_options_and_scenes(precision, monkeypatch):
+    seven = [(m[0], m[1]) for m in configs.ensemble_members(seed=7, count=7, l0_choices=(0.02, 0.015, 0.01))]
+    wide = [_scene_2d(41, 53, 3.1)]
+    for c in (_counts(seven, precision, False, monkeypatch),
+              _counts(seven, precision, False, monkeypatch, use_graph=False),
+              _counts(wide, precision, False, monkeypatch, max_iterations=7)):
+        assert c["resident_solves"] == 2 and c["resident_gave_up"] == 0, c
+
+
+@PRECISIONS
+@pytest.mark.parametrize("halo", ["0", "150"])
+def test_resident_solve_gives_up(halo, precision, monkeypatch):
+    c = _counts([_scene_2d(41, 53, 2.1)], precision, False, monkeypatch, {"MPS_AMD_CG_RESIDENT_HALO": halo})
+    assert c["resident_solves"] == 0 < c["resident_gave_up"], c
+
+
+def test_handles_that_ask_for_more_than_the_chip(monkeypatch):
+    """Two handles of 149 workgroups each step at the same time: one is
+    refused at least once, and no launch gives up."""
+    sims = [_sim([_scene_2d(301, 253, 2.1)], FP64, False, monkeypatch) for _ in range(2)]
+    ts = [threading.Thread(target=sim.run_steps, args=(12,)) for sim in sims]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    cs = [sim.debug_counters() for sim in sims]
+    for sim in sims:
+        sim.close()
+    assert sum(c["refused"] for c in cs) > 0, cs
+    assert all(c["resident_solves"] + c["refused"] == 12 and c["resident_gave_up"] == 0 for c in cs), cs
