@@ -1761,10 +1761,12 @@ struct MgWork {
     bool fine_additive = false;      // the current hierarchy's choice
     int tail_rows = kMgTailRows;
     // k_mg_coarse: the most workgroups it may take (0: off, by
-    // MPS_AMD_MG_COARSE or after a launch that gave up), its levels lc ..
+    // MPS_AMD_MG_COARSE), whether the current solve takes it, its levels lc ..
     // co_lt - 1 (none: not used) and its tail co_lt .. L, their first blocks,
     // the exchange places and what they were last cleared for
     int co_most = 0;
+    bool co_on = true;
+    BackOff co_back;
     int co_polls = 0;
     int lc = 1, co_lt = 1;
     int co_each = 0;                 // rows of a block
@@ -1988,12 +1990,15 @@ static hipError_t mg_coarse_plan(MgWork* m, int dim, bool fine_ok, hipStream_t s
     return hipSuccess;
 }
 
-int mg_coarse_groups(const MgWork* m) { return m && m->lc < m->co_lt ? m->co_first[m->co_lt - m->lc] + m->co_fine : 0; }
+int mg_coarse_groups(const MgWork* m) {
+    return m && m->co_on && m->lc < m->co_lt ? m->co_first[m->co_lt - m->lc] + m->co_fine : 0;
+}
 bool mg_coarse_fine(const MgWork* m) { return mg_coarse_groups(m) > 0 && m->co_fine > 0; }
-void mg_coarse_off(MgWork* m) {
-    m->co_most = 0;
-    m->lc = m->co_lt;
-    m->gen++;
+void mg_coarse_skip(MgWork* m, bool gave_up) {
+    m->co_on = false;
+    if (!gave_up) return;
+    m->co_back.start();
+    m->xch_new = true;  // what a launch left half done: its places and its epoch
 }
 
 // The fine level's form for this system (see MgWork::fine_mode).  A system
@@ -2288,10 +2293,11 @@ static hipError_t mg_setup_t(MgWork* m, const Sell& A, const Hot& h, int dim, co
     const bool fine_ok = !m->fine_additive && sizeof(IDX) == 2 && (dim == 2 || sizeof(T) == 8) &&
                          A.entries <= (size_t) most_w * R;
     if ((e = mg_coarse_plan<T>(m, dim, fine_ok, st))) return e;
+    m->co_on = !m->co_back.skip();
     for (int k = 1; k <= l; k++)
         m->hdesc[k] = MgLevelDesc{m->cap[k], 0,         m->col[k], m->val[k],   m->diag[k],
                                   m->dinv[k], m->agg[k], m->child[k], m->b[k], m->x[k], m->xch[k]};
-    if ((e = mg_pack<T>(m, dim, st))) return e;
+    if (m->co_on && (e = mg_pack<T>(m, dim, st))) return e;
     if (!m->up_desc_valid || std::memcmp(m->up_desc, m->hdesc, sizeof(m->hdesc)) != 0) {
         std::memcpy(m->up_desc, m->hdesc, sizeof(m->hdesc));
         m->up_desc_valid = true;
@@ -2326,7 +2332,7 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
     T* res0 = (T*) m->res0;
     T* xx0 = (T*) m->xx0;
     const bool add = m->fine_additive;
-    const bool one = m->lc < m->co_lt;  // levels lc .. L in k_mg_coarse
+    const bool one = mg_coarse_groups(m) > 0;  // levels lc .. L in k_mg_coarse
     const bool fine = one && m->co_fine > 0;  // and the fine level
     if (!add && !fine)
         hipLaunchKernelGGL((k_mg_down0<T, IDX>), mg_grid(m->cap[0]), dim3(kBlock), 0, st, nd + 0, A.slice_off, fcol,

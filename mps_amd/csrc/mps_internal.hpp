@@ -138,6 +138,25 @@ struct BoundedWait {
     }
 };
 
+// Solves that leave out a launch that gave up.  A wait given up costs its 50 ms
+// and a second solve, and what held the workgroups (another process, most
+// likely) may stay or go: the launch is tried again after 256 solves (a wait
+// then adds 0.2 ms a solve at most), and after twice as many each time, up to
+// 4096, where it gives up again.
+struct BackOff {
+    int left = 0;
+    int next = 256;
+    bool skip() {
+        if (left == 0) return false;
+        left--;
+        return true;
+    }
+    void start() {
+        left = next;
+        next = next < 4096 ? 2 * next : 4096;
+    }
+};
+
 // Sum of v[r0 .. r1) in row order, four loads in flight (the level-1
 // restriction of the multigrid cycle; the CG step forms the same sums where
 // it writes r, so both give the same bits).
@@ -1166,10 +1185,13 @@ void mg_cycle(MgWork* m, const Sell& A, const IDX* fcol, const T* fval, const T*
               bool b1_given, hipStream_t st);
 // Workgroups of the cycle's coarse launch, which must all run at once (0: it
 // has none); a launch that had to wait too long sets every done flag to 2,
-// and the caller switches it off and solves again (the bits are the same).
+// and the caller solves again without it (the bits are the same).
 int mg_coarse_groups(const MgWork* m);
 bool mg_coarse_fine(const MgWork* m);  // the fine level is in it
-void mg_coarse_off(MgWork* m);
+// The current solve runs by a launch a level: its workgroups are not to be
+// had now, or (gave_up) its launch waited too long, after which some of the
+// next solves leave it out too.
+void mg_coarse_skip(MgWork* m, bool gave_up);
 // When the current hierarchy's cycle restricts the fine residual r itself
 // (the additive fine level): the first fine row of each level-1 cell
 // (n1 + 1 entries, the last = rows) and the level-1 right-hand side b1[K] =

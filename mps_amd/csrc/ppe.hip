@@ -718,17 +718,20 @@ struct CgWork {
     int2* step_cells = nullptr;  // kMaxBlocks + 1
     const int* f_cst1 = nullptr;
     void* f_b1 = nullptr;
-    // chunk graphs of the FP64 CG [0] and the FP32 inner CG [1], one per
-    // chunk length (the first chunk of a solve is sized by prediction)
+    // chunk graphs of the FP64 CG [0] and the FP32 inner CG [1], and of either
+    // with the cycle's coarse launch [2, 3] (a solve that does not get its
+    // workgroups leaves the captured ones alone), one per chunk length (the
+    // first chunk of a solve is sized by prediction)
     // Chunk lengths are even and at most 64, so 32 slots hold every length a
     // solver can ask for: once captured, a length is never captured again
     // while the signature below holds (with 8 slots replaced in turn, the
     // mixed path's inner solves cycled through more lengths than that and
     // captured a graph again every few steps, ~1.3 ms each at 2M).
     static constexpr int kGraphSlots = 32;
-    hipGraphExec_t graph[2][kGraphSlots] = {};
-    int graph_chunk[2][kGraphSlots] = {};
-    long long graph_used[2][kGraphSlots] = {};  // last use, for replacing the least recent
+    static constexpr int kGraphSets = 4;
+    hipGraphExec_t graph[kGraphSets][kGraphSlots] = {};
+    int graph_chunk[kGraphSets][kGraphSlots] = {};
+    long long graph_used[kGraphSets][kGraphSlots] = {};  // last use, for replacing the least recent
     long long graph_clock = 0;
     long long graph_captures = 0;  // chunk graphs captured
     // everything a captured chunk bakes in: every device pointer its kernels
@@ -736,7 +739,7 @@ struct CgWork {
     // Any difference (a buffer reallocated by a larger system, another
     // column width) drops the cached graphs of that solver.
     static constexpr int kSig = 24;
-    uintptr_t graph_sig[2][kSig] = {};
+    uintptr_t graph_sig[kGraphSets][kSig] = {};
     static constexpr int kPredSolves = 4;
     bool predict = true;  // MPS_AMD_CG_PREDICT=0: fixed chunks of the check interval
     // last step's iterations per solve of a step; bank 1 holds the adjoint
@@ -852,7 +855,7 @@ void cg_destroy(CgWork* cw) {
     hipHostFree(cw->res_out);
     for (int k = 0; k < CgWork::kResGraphs; k++)
         if (cw->res_graph[k]) hipGraphExecDestroy(cw->res_graph[k]);
-    for (int k = 0; k < 2; k++)
+    for (int k = 0; k < CgWork::kGraphSets; k++)
         for (int j = 0; j < CgWork::kGraphSlots; j++)
             if (cw->graph[k][j]) hipGraphExecDestroy(cw->graph[k][j]);
     mg_destroy(cw->mg);
@@ -912,7 +915,7 @@ hipError_t cg_reserve(CgWork* cw, int rows) {
         (e = hipMalloc(&cw->u32, f)))
         return e;
     cw->cap = cap;
-    for (int k = 0; k < 2; k++)
+    for (int k = 0; k < CgWork::kGraphSets; k++)
         for (int j = 0; j < CgWork::kGraphSlots; j++) {
             if (cw->graph[k][j]) hipGraphExecDestroy(cw->graph[k][j]);
             cw->graph[k][j] = nullptr;
@@ -1007,7 +1010,7 @@ static bool all_done(const CgWork* cw) {
 // cover the prediction rounded down to even (at most 64 each), then, once it
 // is used up, 2, 4, 8, ... 64; else chunks of the check interval.
 template <typename T, typename IDX, bool WEIGHTED>
-static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* col, const T* val, T* y, T* r, T* p,
+static hipError_t run_cg_loop(CgWork* cw, int set, const Sell& A, const IDX* col, const T* val, T* y, T* r, T* p,
                               T* s, T* w, const mps_solver_options& o, int pred, hipStream_t st) {
     const int interval = std::max(2, (o.check_interval + 1) & ~1);
     const int idx16 = sizeof(IDX) == 4 ? 0 : (static_cast<IDX>(-1) < 0 ? 1 : 2);
@@ -1022,13 +1025,13 @@ static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* c
             (uintptr_t) cw->nseg,    (uintptr_t) cw->total_blocks, (uintptr_t) idx16,
             (uintptr_t) (cw->mg_on ? mg_generation(cw->mg) + 1 : 0), (uintptr_t) cw->mg_on,
             (uintptr_t) (cw->mg_on && cw->fused), (uintptr_t) cw->step_cells, 0};
-        if (std::memcmp(sig, cw->graph_sig[which], sizeof(sig)) != 0) {
+        if (std::memcmp(sig, cw->graph_sig[set], sizeof(sig)) != 0) {
             for (int j = 0; j < CgWork::kGraphSlots; j++) {
-                if (cw->graph[which][j]) hipGraphExecDestroy(cw->graph[which][j]);
-                cw->graph[which][j] = nullptr;
-                cw->graph_chunk[which][j] = 0;
+                if (cw->graph[set][j]) hipGraphExecDestroy(cw->graph[set][j]);
+                cw->graph[set][j] = nullptr;
+                cw->graph_chunk[set][j] = 0;
             }
-            std::memcpy(cw->graph_sig[which], sig, sizeof(sig));
+            std::memcpy(cw->graph_sig[set], sig, sizeof(sig));
             cw->graph_rebuilds++;
         }
     }
@@ -1053,31 +1056,31 @@ static hipError_t run_cg_loop(CgWork* cw, int which, const Sell& A, const IDX* c
         if (o.use_graph) {
             int slot = -1;
             for (int j = 0; j < CgWork::kGraphSlots; j++)
-                if (cw->graph[which][j] && cw->graph_chunk[which][j] == chunk) slot = j;
+                if (cw->graph[set][j] && cw->graph_chunk[set][j] == chunk) slot = j;
             if (slot < 0) {
                 // a free slot, else the least recently used one
                 slot = 0;
                 for (int j = 0; j < CgWork::kGraphSlots; j++) {
-                    if (!cw->graph[which][j]) {
+                    if (!cw->graph[set][j]) {
                         slot = j;
                         break;
                     }
-                    if (cw->graph_used[which][j] < cw->graph_used[which][slot]) slot = j;
+                    if (cw->graph_used[set][j] < cw->graph_used[set][slot]) slot = j;
                 }
-                if (cw->graph[which][slot]) hipGraphExecDestroy(cw->graph[which][slot]);
-                cw->graph[which][slot] = nullptr;
+                if (cw->graph[set][slot]) hipGraphExecDestroy(cw->graph[set][slot]);
+                cw->graph[set][slot] = nullptr;
                 hipGraph_t gph;
                 if ((e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal))) return e;
                 enqueue_chunk<T, IDX, WEIGHTED>(cw, A, col, val, y, r, p, s, w, chunk, st);
                 if ((e = hipStreamEndCapture(st, &gph))) return e;
-                e = hipGraphInstantiate(&cw->graph[which][slot], gph, nullptr, nullptr, 0);
+                e = hipGraphInstantiate(&cw->graph[set][slot], gph, nullptr, nullptr, 0);
                 hipGraphDestroy(gph);
                 if (e) return e;
-                cw->graph_chunk[which][slot] = chunk;
+                cw->graph_chunk[set][slot] = chunk;
                 cw->graph_captures++;
             }
-            cw->graph_used[which][slot] = ++cw->graph_clock;
-            if ((e = hipGraphLaunch(cw->graph[which][slot], st))) return e;
+            cw->graph_used[set][slot] = ++cw->graph_clock;
+            if ((e = hipGraphLaunch(cw->graph[set][slot], st))) return e;
         } else {
             enqueue_chunk<T, IDX, WEIGHTED>(cw, A, col, val, y, r, p, s, w, chunk, st);
         }
@@ -1126,14 +1129,15 @@ static hipError_t run_cg(CgWork* cw, int which, int solve, const Sell& A, const 
     const int slot = solve < CgWork::kPredSolves ? solve : CgWork::kPredSolves - 1;
     int* const last = &cw->pred[cw->pred_bank][which][slot];
     const int pred = cw->predict ? *last : 0;
+    const int set = which + (cw->mg_on && mg_coarse_groups(cw->mg) > 0 ? 2 : 0);
     hipError_t e;
     if (A.use16 && A.dim == 3)
-        e = run_cg_loop<T, unsigned short, WEIGHTED>(cw, which, A, (const unsigned short*) A.dcol, val, y, r, p, s, w, o,
+        e = run_cg_loop<T, unsigned short, WEIGHTED>(cw, set, A, (const unsigned short*) A.dcol, val, y, r, p, s, w, o,
                                                      pred, st);
     else if (A.use16)
-        e = run_cg_loop<T, short, WEIGHTED>(cw, which, A, A.dcol, val, y, r, p, s, w, o, pred, st);
+        e = run_cg_loop<T, short, WEIGHTED>(cw, set, A, A.dcol, val, y, r, p, s, w, o, pred, st);
     else
-        e = run_cg_loop<T, int, WEIGHTED>(cw, which, A, A.col, val, y, r, p, s, w, o, pred, st);
+        e = run_cg_loop<T, int, WEIGHTED>(cw, set, A, A.col, val, y, r, p, s, w, o, pred, st);
     if (e) return e;
     int it = 0;  // the segment that took longest sets the chunk
     for (int k = 0; k < cw->nseg; k++) it = std::max(it, cw->host[k].fin);
@@ -1445,7 +1449,7 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
     if (cw->mg_on && mg_coarse_groups(cw->mg) > 0 &&
         !groups.take(cw->res_dev, mg_coarse_groups(cw->mg), cw->res_most)) {
         cw->refused++;
-        mg_coarse_off(cw->mg);
+        mg_coarse_skip(cw->mg, false);
     }
     const auto gave_up = [&]() {
         for (int s = 0; s < nseg; s++)
@@ -1454,7 +1458,7 @@ hipError_t cg_solve(CgWork* cw, const Sell& A, const Hot& h, int n, const double
     };
     const auto again = [&]() {  // from the start, by a launch a level
         cw->coarse_gave_up++;
-        mg_coarse_off(cw->mg);
+        mg_coarse_skip(cw->mg, true);
         groups.give_back();
         return cg_solve(cw, A, h, n, b_s, pprev_id, pprev2_id, x_s, o, stats, st, msg);
     };

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from mps_amd import capi, configs
-from test_gpu_coarse import FP64, MIXED, _run, _same, _scene
+from test_gpu_coarse import FIELDS, FP64, MIXED, _run, _same, _scene
 from test_gpu_resident import SCENES, _scene_2d
 
 pytestmark = pytest.mark.gpu
@@ -115,6 +115,53 @@ def test_fine_level_while_the_rows_change(monkeypatch):
     c = sim.debug_counters()
     sim.close()
     assert len(rows) > 1 and c["coarse_fine_cycles"] == c["cg_launched"] > 0, (rows, c)
+
+
+def test_coarse_launch_is_tried_again_after_it_gave_up(monkeypatch):
+    """Waits of one poll: the launch gives up, and again 256 solves later."""
+    m = [_scene(2, 110, 80)]
+    off = _sim(m, MIXED, True, monkeypatch, {"MPS_AMD_MG_COARSE": "0"})
+    sim = _sim(m, MIXED, True, monkeypatch, {"MPS_AMD_MG_COARSE": "256,1"})
+    for s in (off, sim):
+        s.run_steps(256)
+    assert sim.debug_counters()["coarse_gave_up"] == 1
+    for s in (off, sim):
+        s.step()
+    assert sim.debug_counters()["coarse_gave_up"] == 2
+    a, b = sim.state(), off.state()
+    sim.close()
+    off.close()
+    for k in FIELDS:
+        assert (a[k] == b[k]).all(), k
+
+
+def test_coarse_launch_comes_back_after_a_refusal(monkeypatch):
+    """A handle whose workgroups another one holds solves by a launch a level
+    then, and takes the coarse launch again once they are free."""
+    m = [_scene(2, 251, 139)]
+    off = _sim(m, MIXED, True, monkeypatch, {"MPS_AMD_MG_COARSE": "0"})
+    sims = [_sim(m, MIXED, True, monkeypatch) for _ in range(2)]
+    ts = [threading.Thread(target=s.run_steps, args=(60,)) for s in sims]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    off.run_steps(62)
+    want = off.state()
+    off.close()
+    refused = 0
+    for s in sims:
+        before = s.debug_counters()
+        s.run_steps(2)
+        after = s.debug_counters()
+        got = s.state()
+        s.close()
+        refused += before["refused"]
+        assert after["refused"] == before["refused"] and after["coarse_gave_up"] == 0, after
+        assert after["coarse_cycles"] - before["coarse_cycles"] == after["cg_launched"] - before["cg_launched"] > 0
+        for k in FIELDS:
+            assert (got[k] == want[k]).all(), k
+    assert refused > 0
 
 
 # ---- resident solves
