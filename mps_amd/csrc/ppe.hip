@@ -757,8 +757,8 @@ struct CgWork {
     long long refused = 0;         // solves refused either launch for want of workgroups
     // resident solves (resident.hip): exchange memory, the last tag handed
     // out, the most workgroups that can run at once (0: off, as set by
-    // MPS_AMD_CG_RESIDENT=0 or after a launch that gave up), the launches'
-    // captured graphs (one per signature: the particle arrays alternate) and
+    // MPS_AMD_CG_RESIDENT=0), the solves left to the kernels after a launch
+    // that gave up, the launches' captured graphs (one per signature: the particle arrays alternate) and
     // the pinned blocks through which a solve's options go in and its
     // results come out
     CgExchange xch{};
@@ -766,6 +766,7 @@ struct CgWork {
     int res_groups = 0;
     int res_most = 0;  // of all handles together: one a CU
     int res_dev = 0;
+    BackOff res_back;
     unsigned res_ready = 0;  // kernel shapes prepared
     static constexpr int kResGraphs = 4;
     hipGraphExec_t res_graph[kResGraphs] = {};
@@ -1280,7 +1281,7 @@ static hipError_t resident_solve(CgWork* cw, const Sell& A, const Hot& h, const 
     const bool mixed = o.precision == MPS_PREC_MIXED;
     const int max_ref = mixed ? (o.max_refinements > 0 ? o.max_refinements : 20) : kMaxRestarts;
     const ResidentShape shape = resident_fits(cw, A, o.precision, max_ref);
-    if (!shape.split) return hipSuccess;
+    if (!shape.split || cw->res_back.skip()) return hipSuccess;
     int most = 0;
     for (int k = 0; k < cw->nseg; k++) most = std::max(most, cw->h_row[k + 1] - cw->h_row[k]);
     const long long its = o.max_iterations > 0 ? o.max_iterations : 2ll * most;
@@ -1354,8 +1355,11 @@ static hipError_t resident_solve(CgWork* cw, const Sell& A, const Hot& h, const 
         bail = bail || cw->res_out[k].bail;
         it = std::max(it, cw->res_out[k].iterations);
     }
-    if (bail) {  // a halo too large, or CUs held by others: this handle stays with the kernels
-        cw->res_groups = 0;
+    // A halo too large, or CUs held by others.  (Where a split block's halo is
+    // too large whole blocks would hold it, four times as many rows; in 3D at 3.6
+    // and 4.1 l0, 1,300-7,800 rows, they took 2-23 % longer than the kernels.)
+    if (bail) {
+        cw->res_back.start();
         cw->resident_gave_up++;
         return hipSuccess;
     }

@@ -191,6 +191,24 @@ def test_resident_solve_gives_up(halo, precision, monkeypatch):
     assert c["resident_solves"] == 0 < c["resident_gave_up"], c
 
 
+def test_resident_solve_is_tried_again_after_it_gave_up(monkeypatch):
+    """No halo fits: the launch gives up, and again 257 solves later."""
+    m = [_scene_2d(41, 53, 2.1)]
+    off = _sim(m, FP64, False, monkeypatch, {"MPS_AMD_CG_RESIDENT": "0"})
+    sim = _sim(m, FP64, False, monkeypatch, {"MPS_AMD_CG_RESIDENT_HALO": "0"})
+    for s in (off, sim):
+        s.run_steps(257)
+    assert sim.debug_counters()["resident_gave_up"] == 1
+    for s in (off, sim):
+        s.step()
+    assert sim.debug_counters()["resident_gave_up"] == 2
+    a, b = sim.state(), off.state()
+    sim.close()
+    off.close()
+    for k in FIELDS:
+        assert (a[k] == b[k]).all(), k
+
+
 def test_handles_that_ask_for_more_than_the_chip(monkeypatch):
     """Two handles of 149 workgroups each step at the same time: one is
     refused at least once, and no launch gives up."""
