@@ -778,6 +778,7 @@ struct CgWork {
     ResidentOut* res_out = nullptr;
     int* res_count = nullptr;  // device, per segment: workgroups that have left
     int res_segs = 0;          // segments res_out and res_count hold
+    unsigned res_seq = 0;      // the last solve's number, never 0: what res_out holds before the first
     std::vector<int> up_row, up_blk;  // segment layout the device holds
     Seg seg() const { return Seg{nseg, blk_off, row_off}; }
 };
@@ -1201,6 +1202,7 @@ static hipError_t resident_reserve(CgWork* cw, int rows, hipStream_t st) {
         if ((e = hipMalloc(&cw->res_count, sizeof(int) * (size_t) cw->nseg))) return e;
         if ((e = hipHostMalloc((void**) &cw->res_in, sizeof(ResidentIn), flags))) return e;
         if ((e = hipHostMalloc((void**) &cw->res_out, sizeof(ResidentOut) * (size_t) cw->nseg, flags))) return e;
+        std::memset(cw->res_in, 0, sizeof(ResidentIn));
         std::memset(cw->res_out, 0, sizeof(ResidentOut) * (size_t) cw->nseg);
         if ((e = fill_int(cw->res_count, 0, (size_t) cw->nseg, st))) return e;
         cw->res_segs = cw->nseg;
@@ -1307,7 +1309,8 @@ static hipError_t resident_solve(CgWork* cw, const Sell& A, const Hot& h, const 
         in.max_refinements = max_ref;
         in.tag0 = cw->tag;
         in.poison = cw->tag + (unsigned) span;
-        in.seq++;
+        if (++cw->res_seq == 0) cw->res_seq = 1;
+        in.seq = cw->res_seq;
         cw->tag += (unsigned) span;
         ResidentArgs a;
         std::memset(&a, 0, sizeof a);  // compared as bytes
@@ -1345,7 +1348,7 @@ static hipError_t resident_solve(CgWork* cw, const Sell& A, const Hot& h, const 
             else
                 e = resident_enqueue<double, int>(cw, shape, a, g, st);
         }
-        if (!e) e = resident_wait(cw, in.seq, st);
+        if (!e) e = resident_wait(cw, cw->res_seq, st);
     }
     groups.give_back();
     if (e) return e;
