@@ -773,6 +773,7 @@ struct CgWork {
     ResidentArgs res_sig[kResGraphs] = {};
     ResidentShape res_shape[kResGraphs] = {};
     int res_grid[kResGraphs] = {};
+    unsigned res_kernel[kResGraphs] = {};
     long long res_used[kResGraphs] = {};
     ResidentIn* res_in = nullptr;
     ResidentOut* res_out = nullptr;
@@ -1228,6 +1229,8 @@ template <typename T, typename IDX>
 static hipError_t resident_enqueue(CgWork* cw, const ResidentShape& shape, const ResidentArgs& a, bool graph,
                                    hipStream_t st) {
     const int idx16 = sizeof(IDX) == 4 ? 0 : (static_cast<IDX>(-1) < 0 ? 1 : 2);
+    // which kernel: the column and value types are not in the arguments, whose
+    // pointers storage that moved may share with another type's
     const unsigned kernel = 1u << (8 * idx16 + 4 * (int) (sizeof(T) == 8) + 2 * (int) (shape.split > 1) +
                                    (int) (shape.emax > 16));
     hipError_t e;
@@ -1239,7 +1242,8 @@ static hipError_t resident_enqueue(CgWork* cw, const ResidentShape& shape, const
     if (!graph) return resident_launch<T, IDX>(shape, grid, a, st);
     int slot = -1;
     for (int k = 0; k < CgWork::kResGraphs; k++)
-        if (cw->res_graph[k] && cw->res_grid[k] == grid && std::memcmp(&cw->res_sig[k], &a, sizeof a) == 0 &&
+        if (cw->res_graph[k] && cw->res_kernel[k] == kernel && cw->res_grid[k] == grid &&
+            std::memcmp(&cw->res_sig[k], &a, sizeof a) == 0 &&
             std::memcmp(&cw->res_shape[k], &shape, sizeof shape) == 0)
             slot = k;
     if (slot < 0) {  // a free slot, else the least recently used one
@@ -1263,6 +1267,7 @@ static hipError_t resident_enqueue(CgWork* cw, const ResidentShape& shape, const
         std::memcpy(&cw->res_sig[slot], &a, sizeof a);
         std::memcpy(&cw->res_shape[slot], &shape, sizeof shape);
         cw->res_grid[slot] = grid;
+        cw->res_kernel[slot] = kernel;
         cw->graph_rebuilds++;
         cw->graph_captures++;
     }
