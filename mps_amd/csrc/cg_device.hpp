@@ -286,8 +286,10 @@ struct ResidentShape {
     size_t lds;
 };
 // The shape for segments of at most max_rows rows in at most max_nb blocks,
-// total_blocks in all, with at most `most` workgroups at once.
-ResidentShape resident_shape(int max_rows, int max_nb, int total_blocks, int mean_width, int most, bool mixed);
+// total_rows and total_blocks in all, mean_width entries a row of entry_bytes
+// each (value and column), with at most `most` workgroups at once.
+ResidentShape resident_shape(int max_rows, int max_nb, int total_rows, int total_blocks, int mean_width,
+                             int entry_bytes, int most, bool mixed);
 // Tags a launch may use: its iterations and rounds bound its exchanges.
 long long resident_tags(long long max_iterations, int max_rounds);
 // Places for partial sums (CgExchange::p_sums) a launch needs, and the words

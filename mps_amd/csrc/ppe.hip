@@ -1166,8 +1166,9 @@ static ResidentShape resident_fits(const CgWork* cw, const Sell& A, int precisio
         most = std::max(most, rows);
         most_nb = std::max(most_nb, nb);
     }
-    return resident_shape(most, most_nb, cw->total_blocks, mean_width(A), cw->res_groups,
-                          precision == MPS_PREC_MIXED);
+    const bool mixed = precision == MPS_PREC_MIXED;
+    return resident_shape(most, most_nb, A.rows, cw->total_blocks, mean_width(A),
+                          (mixed ? 4 : 8) + (A.use16 ? 2 : 4), cw->res_groups, mixed);
 }
 
 static hipError_t resident_reserve(CgWork* cw, int rows, hipStream_t st) {

@@ -40,6 +40,7 @@
 // poisoned tag and leaves, and the host then solves by launches.
 #pragma clang fp contract(off)
 
+#include <algorithm>
 #include <cstring>
 
 #include "cg_device.hpp"
@@ -712,11 +713,33 @@ static size_t resident_lds(int max_rows, int threads) {
 
 // Entries held in registers: 16 covers a 2D system at 2.1 l0 (12-14 a row),
 // 36 one at 3.1 l0 (28-34) and 3D at 2.1 l0 (32-36); a wider row reads the
-// rest from memory every iteration.
+// rest from memory every iteration, one entry after the other, with its place
+// looked up anew.  That pays up to some width and, where less than half of a row
+// is held, while the L2s (4 MB an XCD) keep what is read again; beyond, the
+// kernels win, which gather by fours with more wavefronts.  The FP64 kernel's
+// spilled registers want their part of the L2s.  Measured, ms a step by kernels /
+// resident:
+//   w entries a row      FP64                        mixed
+//   28   (2D, 120k rows) 10.6 / 5.1                  11.3 / 4.5
+//   48   (2D, 124k)      10.4 / 7.5                  10.2 / 5.2
+//   68   (2D)            69k 8.3 / 8.0, 123k 11.4 / 10.1     123k 11.3 / 9.3
+//   88   (2D)            33k rows 5.8 / 5.0          87k 11.0 / 10.6
+//                        37k 6.3 / 6.6, 79k 10.0 / 10.6    99k 12.0 / 12.4
+//   116  (3D, 3.1 l0)    20k 3.9 / 4.0               46k 7.2 / 7.1
+//                        25k 4.5 / 5.9               52k 7.5 / 8.0
+//   120  (2D)            12k 5.7 / 5.1, 24k 7.5 / 8.6      44k 14.0 / 12.5, 61k 18.0 / 24.6
+//   158  (2D, 8k)        5.2 / 5.0                   6.7 / 7.1
+//   170  (3D, 15k)       4.8 / 6.6                   5.7 / 6.5
+// and split blocks (7,800 rows and fewer):
+//   209  (2D)            6.1 / 5.7                   8.1 / 8.0
+//   252  (2D)            5.7 / 5.4                   7.4 / 7.6
+//   439  (2D)            8.5 / 8.9                   10.3 / 12.3
 constexpr int kResFew = 16, kResMany = 36;
+constexpr int kResWide = 144, kResWideSplit = 240;                    // widest mean row
+constexpr double kResReread64 = 17.5e6, kResReread32 = 24e6;          // bytes read again an iteration
 
-ResidentShape resident_shape(int max_rows, int max_nb, int total_blocks, int mean_width, int most, bool mixed) {
-    (void) mixed;
+ResidentShape resident_shape(int max_rows, int max_nb, int total_rows, int total_blocks, int mean_width,
+                             int entry_bytes, int most, bool mixed) {
     ResidentShape s;
     std::memset(&s, 0, sizeof s);  // compared as bytes
     if (max_rows > kResMaxRows || max_nb > kResMaxBlocks || total_blocks > most) return s;
@@ -726,6 +749,10 @@ ResidentShape resident_shape(int max_rows, int max_nb, int total_blocks, int mea
     // the threads of a split workgroup can wait for.
     s.split = max_nb > 1 && max_nb * kResWaves <= kResSplitSums && kResSplit * total_blocks <= most ? kResSplit : 1;
     s.emax = mean_width <= kResFew ? kResFew : kResMany;
+    const double reread = (double) std::max(mean_width - s.emax, 0) * entry_bytes * total_rows;
+    if (mean_width > (s.split > 1 ? kResWideSplit : kResWide) ||
+        (mean_width > 2 * s.emax && reread > (mixed ? kResReread32 : kResReread64)))
+        s.split = 0;
     s.lds = resident_lds(max_rows, kCgBlock / s.split);
     return s;
 }

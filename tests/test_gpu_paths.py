@@ -8,7 +8,7 @@ import pytest
 
 from mps_amd import capi, configs
 from test_gpu_coarse import FIELDS, FP64, MIXED, _run, _same, _scene
-from test_gpu_resident import SCENES, _scene_2d
+from test_gpu_resident import SCENES, _scene_2d, _scene_3d
 
 pytestmark = pytest.mark.gpu
 
@@ -189,6 +189,43 @@ def test_resident_solve_runs_with_options_and_scenes(precision, monkeypatch):
 def test_resident_solve_gives_up(halo, precision, monkeypatch):
     c = _counts([_scene_2d(41, 53, 2.1)], precision, False, monkeypatch, {"MPS_AMD_CG_RESIDENT_HALO": halo})
     assert c["resident_solves"] == 0 < c["resident_gave_up"], c
+
+
+def _wide(dim, n, radius):
+    s, sc = _scene_2d(*n, radius) if dim == 2 else _scene_3d(*n)
+    s.ratio_pressure = s.ratio_surface = radius
+    return [(s, sc)]
+
+
+# rows wider than the 36 entries a thread holds: split blocks, whole ones
+@PRECISIONS
+@pytest.mark.parametrize("dim,n,radius", [(3, (27, 12, 12), 3.1), (2, (70, 50), 6.1), (3, (27, 14, 16), 3.1),
+                                          (2, (120, 90), 5.1)])
+def test_rows_wider_than_a_thread_holds(dim, n, radius, precision, monkeypatch):
+    m = _wide(dim, n, radius)
+    got = []
+    for env in ({}, {"MPS_AMD_CG_RESIDENT": "0"}):
+        sim = _sim(m, precision, False, monkeypatch, env)
+        sim.set_snapshot(True)
+        sim.run_steps(3)
+        got.append((sim.state(), sim.solver_stats(), sim.debug_counters()["resident_solves"]))
+        rp = sim.pressure_system()["row_ptr"]
+        sim.close()
+    assert got[0][2] == 3 and got[1][2] == 0
+    assert rp[-1] > 36 * got[0][1]["rows"]
+    assert got[0][1] == got[1][1]
+    for k in FIELDS:
+        assert (got[0][0][k] == got[1][0][k]).all(), k
+
+
+# rows wider than pays (144 entries, split blocks 240); more bytes than the L2s
+# keep in FP64 (79 entries a row are read again), not in mixed precision
+@pytest.mark.parametrize("dim,n,radius,taken", [(2, (100, 85), 7.1, (0, 0)), (2, (60, 50), 10.1, (0, 0)),
+                                                (3, (40, 26, 25), 3.1, (0, 2))])
+def test_rows_too_wide_are_left_to_the_kernels(dim, n, radius, taken, monkeypatch):
+    for precision, want in zip((FP64, MIXED), taken):
+        c = _counts(_wide(dim, n, radius), precision, False, monkeypatch)
+        assert c["resident_solves"] == want and c["resident_gave_up"] == 0, (precision, c)
 
 
 def test_resident_solve_is_tried_again_after_it_gave_up(monkeypatch):
