@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import argparse
 import os
+import re
 import subprocess
 import sys
 from concurrent.futures import ThreadPoolExecutor
@@ -44,11 +45,12 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     f"-I{INCLUDE}",
 ]
-# Flags of single sources.  The resident solver is written to keep its uniform
-# values within the scalar registers; where a compiler runs out of them all the
-# same they go to scratch memory, not to lanes of vector registers: from there
-# some came back wrong in this kernel (mixed precision, 128 threads).
-SOURCE_FLAGS = {"resident.hip": ["-mllvm", "-amdgpu-spill-sgpr-to-vgpr=0"]}
+# Kernels whose uniform values must all stay in scalar registers: an earlier
+# form of the resident solver spilled some to lanes of vector registers, and
+# there (mixed precision, 128 threads) they came back wrong; why was not found.
+# It is written not to spill since, and the build fails where a compiler or a
+# change makes it, or the other kernel that polls while it waits.
+NO_SCALAR_SPILLS = {"resident.hip": "k_solve_resident", "mg.hip": "k_mg_coarse"}
 
 
 def _stale(target, deps):
@@ -58,15 +60,45 @@ def _stale(target, deps):
     return any(os.path.getmtime(d) > t for d in deps)
 
 
+def _scalar_spills(remarks, kernel):
+    """{mangled name: spilled scalar registers} of the instances of `kernel` in
+    the compiler's resource remarks."""
+    found, name = {}, None
+    for line in remarks.splitlines():
+        m = re.search(r"remark:\s+(Function Name|SGPRs Spill): (\S+)", line)
+        if m and m.group(1) == "Function Name":
+            name = m.group(2)
+        elif m and name and kernel in name:
+            found[name] = int(m.group(2))
+    return found
+
+
 def _compile(src, force):
     obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
     path = os.path.join(CSRC, src)
-    if not force and not _stale(obj, [path] + HEADERS):
-        return obj, None
-    cmd = [HIPCC] + FLAGS + SOURCE_FLAGS.get(src, []) + ["-c", path, "-o", obj]
+    kernel = NO_SCALAR_SPILLS.get(src)
+    cmd = [HIPCC] + FLAGS + (["-Rpass-analysis=kernel-resource-usage"] if kernel else []) + ["-c", path, "-o", obj]
+    # the command an object was made with stands beside it
+    made = obj + ".cmd"
+    line = " ".join(cmd)
+    if not force and not _stale(obj, [path] + HEADERS) and os.path.exists(made):
+        with open(made) as f:
+            if f.read() == line:
+                return obj, None
+    if os.path.exists(made):
+        os.remove(made)
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
-        return obj, f"$ {' '.join(cmd)}\n{r.stdout}\n{r.stderr}"
+        return obj, f"$ {line}\n{r.stdout}\n{r.stderr}"
+    if kernel:
+        spills = _scalar_spills(r.stderr, kernel)
+        if not spills:
+            return obj, f"{src}: no resource remark of {kernel}"
+        bad = {k: v for k, v in spills.items() if v}
+        if bad:
+            return obj, f"{src}: scalar registers of {kernel} spilled: {bad}"
+    with open(made, "w") as f:
+        f.write(line)
     return obj, None
 
 
