@@ -191,6 +191,23 @@ def test_resident_solve_gives_up(halo, precision, monkeypatch):
     assert c["resident_solves"] == 0 < c["resident_gave_up"], c
 
 
+# 184 and 247 blocks of the 256 that a launch may take
+@PRECISIONS
+@pytest.mark.parametrize("n,radius", [((431, 209), 2.1), ((500, 245), 3.1)])
+def test_resident_solve_of_many_blocks(n, radius, precision, monkeypatch):
+    m = [_scene_2d(*n, radius)]
+    got = []
+    for env in ({}, {"MPS_AMD_CG_RESIDENT": "0"}):
+        sim = _sim(m, precision, False, monkeypatch, env)
+        sim.run_steps(2)
+        got.append((sim.state(), sim.solver_stats(), sim.debug_counters()["resident_solves"]))
+        sim.close()
+    assert got[0][2] == 2 and got[1][2] == 0 and got[0][1] == got[1][1]
+    assert got[0][1]["rows"] > 150 * 512
+    for k in FIELDS:
+        assert (got[0][0][k] == got[1][0][k]).all(), k
+
+
 def _wide(dim, n, radius):
     s, sc = _scene_2d(*n, radius) if dim == 2 else _scene_3d(*n)
     s.ratio_pressure = s.ratio_surface = radius
