@@ -1241,6 +1241,11 @@ struct MgFine {
 // and k_mg_up0: what is read again waits for level 1 by fours.
 template <int W>
 constexpr int kMgFineEntries = W == 9 ? 16 : 36;
+// The fine columns and values it is built for: the plane's and the space's
+// 16-bit columns, and not 3D in FP32 (see above).
+template <typename T, typename IDX, int W>
+constexpr bool kMgFineIn =
+    sizeof(IDX) == 2 && (static_cast<IDX>(-1) < 0) == (W == 9) && (W == 9 || sizeof(T) == 8);
 
 template <typename T>
 __device__ __forceinline__ T mg_fine_residual(T omega, T b, T acc) {
@@ -2288,9 +2293,8 @@ static hipError_t mg_setup_t(MgWork* m, const Sell& A, const Hot& h, int dim, co
     }
     if (tail != m->tail) m->gen++;
     m->tail = tail;
-    // 3D in FP32 is left out (see MgFine)
     const int most_w = dim == 2 ? kMgFineEntries<9> : kMgFineEntries<27>;
-    const bool fine_ok = !m->fine_additive && sizeof(IDX) == 2 && (dim == 2 || sizeof(T) == 8) &&
+    const bool fine_ok = !m->fine_additive && (dim == 2 ? kMgFineIn<T, IDX, 9> : kMgFineIn<T, IDX, 27>) &&
                          A.entries <= (size_t) most_w * R;
     if ((e = mg_coarse_plan<T>(m, dim, fine_ok, st))) return e;
     m->co_on = !m->co_back.skip();
@@ -2372,7 +2376,7 @@ static void mg_cycle_t(MgWork* m, const Sell& A, const IDX* fcol, const T* fval,
         a.xxf = lc == 1 ? xf : nullptr;
         a.pk = mg_packed<T>(m);
         a.f = MgFine<T>{A.slice_off, fcol, A.anc, fval, m->agg[0], u, m->xch0, m->fcap};
-        if constexpr (sizeof(IDX) == 2 && (W == 9 || sizeof(T) == 8)) {
+        if constexpr (kMgFineIn<T, IDX, W>) {
             if (fine)
                 hipLaunchKernelGGL((k_mg_coarse<T, W, C, BT, IDX>), dim3(m->co_first[k1] + m->co_fine), dim3(BT), 0, st,
                                    a);
