@@ -300,12 +300,15 @@ static void scene_consts(const mps_settings& s, Consts& c) {
 // first page faults) while the device fills the others.
 // Measured, a pass with its read: 458 particles 575 -> 472 us (one step), 2M
 // (150 MB) 81.7 -> 73.5 ms (10 steps), 254k 61.5 -> 59.2 ms (20 steps).
-// kReadThreadMin: below it one thread copies it out before eight have started.
+// kReadThreadMin: below it one thread copies it out before eight have started
+// (the state of 32k, 43k and 59k particles, 2.1-3.9 MB, into touched memory: in
+// one go 163, 191 and 268 us, by threads 227, 256 and 326, pageable 176, 215 and
+// 297; of 72k, 4.7 MB, into new arrays: 405, 370 and 423).
 constexpr int kReadPieces = 6;
 constexpr size_t kStateReadBytes = 2 * 3 * sizeof(double) + 2 * sizeof(double) + 2;  // of a particle, all arrays
 constexpr size_t kReadSlot = (size_t) 2 << 20;
 constexpr size_t kReadSlots = 8;
-constexpr size_t kReadThreadMin = (size_t) 2 << 20;
+constexpr size_t kReadThreadMin = (size_t) 4 << 20;
 
 struct ReadPiece {
     void* dst;

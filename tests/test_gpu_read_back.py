@@ -65,3 +65,16 @@ def test_arrays_one_at_a_time():
         sim._check(sim.L.mps_download(sim.h, *args))
         assert (got == want[k]).all(), k
     sim.close()
+
+
+# either side of 4 MiB in all (63,550 particles): one copy, several threads
+@pytest.mark.parametrize("nx,ny,large", [(225, 264, False), (225, 265, True)])
+def test_state_where_the_threads_start(nx, ny, large):
+    sim = _sim(nx, ny)
+    assert (66 * sim.n >= 4 << 20) == large
+    want = _slot(sim)
+    for _ in range(2):
+        got = sim.state()
+        for k, v in want.items():
+            assert (got[k] == v).all(), k
+    sim.close()
