@@ -288,7 +288,7 @@ struct ResidentShape {
 // The shape for segments of at most max_rows rows in at most max_nb blocks,
 // total_rows and total_blocks in all, mean_width entries a row of entry_bytes
 // each (value and column), with at most `most` workgroups at once.
-ResidentShape resident_shape(int max_rows, int max_nb, int total_rows, int total_blocks, int mean_width,
+ResidentShape resident_shape(int dim, int max_rows, int max_nb, int total_rows, int total_blocks, int mean_width,
                              int entry_bytes, int most, bool mixed);
 // Tags a launch may use: its iterations and rounds bound its exchanges.
 long long resident_tags(long long max_iterations, int max_rounds);

@@ -1167,7 +1167,7 @@ static ResidentShape resident_fits(const CgWork* cw, const Sell& A, int precisio
         most_nb = std::max(most_nb, nb);
     }
     const bool mixed = precision == MPS_PREC_MIXED;
-    return resident_shape(most, most_nb, A.rows, cw->total_blocks, mean_width(A),
+    return resident_shape(A.dim, most, most_nb, A.rows, cw->total_blocks, mean_width(A),
                           (mixed ? 4 : 8) + (A.use16 ? 2 : 4), cw->res_groups, mixed);
 }
 

@@ -725,8 +725,6 @@ static size_t resident_lds(int max_rows, int threads) {
 //   68   (2D)            69k 8.3 / 8.0, 123k 11.4 / 10.1     123k 11.3 / 9.3
 //   88   (2D)            33k rows 5.8 / 5.0          87k 11.0 / 10.6
 //                        37k 6.3 / 6.6, 79k 10.0 / 10.6    99k 12.0 / 12.4
-//   116  (3D, 3.1 l0)    20k 3.9 / 4.0               46k 7.2 / 7.1
-//                        25k 4.5 / 5.9               52k 7.5 / 8.0
 //   120  (2D)            12k 5.7 / 5.1, 24k 7.5 / 8.6      44k 14.0 / 12.5, 61k 18.0 / 24.6
 //   158  (2D, 8k)        5.2 / 5.0                   6.7 / 7.1
 //   170  (3D, 15k)       4.8 / 6.6                   5.7 / 6.5
@@ -734,11 +732,19 @@ static size_t resident_lds(int max_rows, int threads) {
 //   209  (2D)            6.1 / 5.7                   8.1 / 8.0
 //   252  (2D)            5.7 / 5.4                   7.4 / 7.6
 //   439  (2D)            8.5 / 8.9                   10.3 / 12.3
+// In 3D the columns' anchors make what is read again dearer, and the kernels are
+// quick on a few rows:
+//   85-92 (2.9 l0)       18k 3.3 / 3.3               18k 4.1 / 3.7, 36k 5.1 / 4.7
+//   95    (3.1 l0)       630 rows 1.5 / 1.7          1.8 / 2.0
+//   105   (3.1 l0)       2k 2.3 / 2.3                2.8 / 2.9
+//   111   (3.1 l0)       5k (split) 3.0 / 2.6        3.6 / 3.2
+//   115   (3.1 l0)       18k 4.0 / 4.2, 25k 4.5 / 5.9      18k 5.2 / 5.3, 52k 7.5 / 8.0
 constexpr int kResFew = 16, kResMany = 36;
-constexpr int kResWide = 144, kResWideSplit = 240;                    // widest mean row
+constexpr int kResWide = 144, kResWideSplit = 240, kResWide3 = 93;    // widest mean row
+constexpr int kResWide3Rows = 4096;                                   // kResWide from here, split blocks
 constexpr double kResReread64 = 17.5e6, kResReread32 = 24e6;          // bytes read again an iteration
 
-ResidentShape resident_shape(int max_rows, int max_nb, int total_rows, int total_blocks, int mean_width,
+ResidentShape resident_shape(int dim, int max_rows, int max_nb, int total_rows, int total_blocks, int mean_width,
                              int entry_bytes, int most, bool mixed) {
     ResidentShape s;
     std::memset(&s, 0, sizeof s);  // compared as bytes
@@ -750,7 +756,9 @@ ResidentShape resident_shape(int max_rows, int max_nb, int total_rows, int total
     s.split = max_nb > 1 && max_nb * kResWaves <= kResSplitSums && kResSplit * total_blocks <= most ? kResSplit : 1;
     s.emax = mean_width <= kResFew ? kResFew : kResMany;
     const double reread = (double) std::max(mean_width - s.emax, 0) * entry_bytes * total_rows;
-    if (mean_width > (s.split > 1 ? kResWideSplit : kResWide) ||
+    const int widest = dim == 3 ? (s.split > 1 && total_rows >= kResWide3Rows ? kResWide : kResWide3)
+                                : (s.split > 1 ? kResWideSplit : kResWide);
+    if (mean_width > widest ||
         (mean_width > 2 * s.emax && reread > (mixed ? kResReread32 : kResReread64)))
         s.split = 0;
     s.lds = resident_lds(max_rows, kCgBlock / s.split);
