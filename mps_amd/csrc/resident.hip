@@ -717,32 +717,29 @@ static size_t resident_lds(int max_rows, int threads) {
 // looked up anew.  That pays up to some width and, where less than half of a row
 // is held, while the L2s (4 MB an XCD) keep what is read again; beyond, the
 // kernels win, which gather by fours with more wavefronts.  The FP64 kernel's
-// spilled registers want their part of the L2s.  Measured, ms a step by kernels /
-// resident:
-//   w entries a row      FP64                        mixed
-//   28   (2D, 120k rows) 10.6 / 5.1                  11.3 / 4.5
-//   48   (2D, 124k)      10.4 / 7.5                  10.2 / 5.2
-//   68   (2D)            69k 8.3 / 8.0, 123k 11.4 / 10.1     123k 11.3 / 9.3
-//   88   (2D)            33k rows 5.8 / 5.0          87k 11.0 / 10.6
-//                        37k 6.3 / 6.6, 79k 10.0 / 10.6    99k 12.0 / 12.4
-//   120  (2D)            12k 5.7 / 5.1, 24k 7.5 / 8.6      44k 14.0 / 12.5, 61k 18.0 / 24.6
-//   158  (2D, 8k)        5.2 / 5.0                   6.7 / 7.1
-//   170  (3D, 15k)       4.8 / 6.6                   5.7 / 6.5
-// and split blocks (7,800 rows and fewer):
-//   209  (2D)            6.1 / 5.7                   8.1 / 8.0
-//   252  (2D)            5.7 / 5.4                   7.4 / 7.6
-//   439  (2D)            8.5 / 8.9                   10.3 / 12.3
-// In 3D the columns' anchors make what is read again dearer, and the kernels are
-// quick on a few rows:
-//   85-92 (2.9 l0)       18k 3.3 / 3.3               18k 4.1 / 3.7, 36k 5.1 / 4.7
-//   95    (3.1 l0)       630 rows 1.5 / 1.7          1.8 / 2.0
-//   105   (3.1 l0)       2k 2.3 / 2.3                2.8 / 2.9
-//   111   (3.1 l0)       5k (split) 3.0 / 2.6        3.6 / 3.2
-//   115   (3.1 l0)       18k 4.0 / 4.2, 25k 4.5 / 5.9      18k 5.2 / 5.3, 52k 7.5 / 8.0
+// spilled registers want their part of the L2s; in 3D the columns' anchors make
+// what is read again dearer.  Measured, ms a step by kernels / resident, 25-45
+// iterations a solve, graphs captured before:
+//   entries a row          FP64                             mixed
+//   2D  48   124k rows     1.27 / 1.12                      1.32 / 0.98
+//       68   59k           1.30 / 1.33                      1.27 / 1.13
+//       68   124k          1.57 / 1.57                      1.56 / 1.51
+//       88                 32k 1.23 / 1.20, 39k 1.29 / 1.46   62k 1.51 / 1.36, 89k 1.61 / 1.70
+//       97   20k           1.24 / 1.23                      1.36 / 1.35
+//       103  12k           1.34 / 1.36                      1.40 / 1.42
+//       119  9k            1.35 / 1.45                      1.46 / 1.55
+//       158  12k           1.60 / 1.88                      1.73 / 2.11
+//       119  714, split    1.04 / 1.07                      1.15 / 1.23
+//       119  7k, split     1.29 / 1.27                      1.40 / 1.40
+//       209  7k, split     2.00 / 2.16                      2.11 / 2.38
+//   3D  92   (2.9 l0)      20k 2.09 / 2.04, 32k 2.19 / 2.32   46k 2.31 / 2.25
+//       95   (3.1 l0, 630) 1.34 / 1.51                      1.58 / 1.69
+//       111  5k, split     2.11 / 2.05                      2.28 / 2.20
+//       115                12k 2.20 / 2.29, 36k 2.71 / 3.45   36k 2.62 / 2.73
 constexpr int kResFew = 16, kResMany = 36;
-constexpr int kResWide = 144, kResWideSplit = 240, kResWide3 = 93;    // widest mean row
-constexpr int kResWide3Rows = 4096;                                   // kResWide from here, split blocks
-constexpr double kResReread64 = 17.5e6, kResReread32 = 24e6;          // bytes read again an iteration
+// the widest mean row; in 3D split blocks of kResWide3Rows rows take up to kResWide3
+constexpr int kResWide = 93, kResWide3 = 144, kResWide3Rows = 4096;
+constexpr double kResReread64 = 16.5e6, kResReread32 = 24e6;  // bytes read again an iteration
 
 ResidentShape resident_shape(int dim, int max_rows, int max_nb, int total_rows, int total_blocks, int mean_width,
                              int entry_bytes, int most, bool mixed) {
@@ -756,11 +753,12 @@ ResidentShape resident_shape(int dim, int max_rows, int max_nb, int total_rows, 
     s.split = max_nb > 1 && max_nb * kResWaves <= kResSplitSums && kResSplit * total_blocks <= most ? kResSplit : 1;
     s.emax = mean_width <= kResFew ? kResFew : kResMany;
     const double reread = (double) std::max(mean_width - s.emax, 0) * entry_bytes * total_rows;
-    const int widest = dim == 3 ? (s.split > 1 && total_rows >= kResWide3Rows ? kResWide : kResWide3)
-                                : (s.split > 1 ? kResWideSplit : kResWide);
+    const int widest = dim == 3 && s.split > 1 && total_rows >= kResWide3Rows ? kResWide3 : kResWide;
     if (mean_width > widest ||
-        (mean_width > 2 * s.emax && reread > (mixed ? kResReread32 : kResReread64)))
+        (mean_width > 2 * s.emax && reread > (mixed ? kResReread32 : kResReread64))) {
         s.split = 0;
+        return s;
+    }
     s.lds = resident_lds(max_rows, kCgBlock / s.split);
     return s;
 }

@@ -216,7 +216,7 @@ def _wide(dim, n, radius):
 
 # rows wider than the 36 entries a thread holds: split blocks, whole ones
 @PRECISIONS
-@pytest.mark.parametrize("dim,n,radius", [(3, (27, 12, 12), 3.1), (2, (70, 50), 6.1), (3, (27, 16, 18), 2.9),
+@pytest.mark.parametrize("dim,n,radius", [(3, (27, 12, 12), 3.1), (2, (70, 50), 5.1), (3, (27, 16, 18), 2.9),
                                           (2, (120, 90), 5.1)])
 def test_rows_wider_than_a_thread_holds(dim, n, radius, precision, monkeypatch):
     m = _wide(dim, n, radius)
@@ -235,10 +235,10 @@ def test_rows_wider_than_a_thread_holds(dim, n, radius, precision, monkeypatch):
         assert (got[0][0][k] == got[1][0][k]).all(), k
 
 
-# rows wider than pays (144 entries, split blocks 240, 3D 93 but for split blocks
-# of 4,096 rows or more); more bytes than the L2s keep in FP64 (56 entries a row
-# are read again), not in mixed precision
-@pytest.mark.parametrize("dim,n,radius,taken", [(2, (100, 85), 7.1, (0, 0)), (2, (60, 50), 10.1, (0, 0)),
+# rows wider than pays (93 entries; 3D, split blocks of 4,096 rows or more 144);
+# more bytes than the L2s keep in FP64 (56 entries a row are read again), not in
+# mixed precision
+@pytest.mark.parametrize("dim,n,radius,taken", [(2, (120, 90), 6.6, (0, 0)), (2, (70, 50), 6.6, (0, 0)),
                                                 (3, (9, 11, 8), 3.1, (0, 0)), (3, (27, 16, 18), 3.1, (0, 0)),
                                                 (3, (44, 28, 28), 2.9, (0, 2))])
 def test_rows_too_wide_are_left_to_the_kernels(dim, n, radius, taken, monkeypatch):
