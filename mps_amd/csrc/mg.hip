@@ -985,13 +985,15 @@ __global__ void __launch_bounds__(kMgTailThreads) k_mg_tail(const MgLevelDesc* _
 // no row writes now are clean when the level grows.  A launch knows its half
 // by an epoch that the last block to leave advances.
 //
-// Measured (launches a level and the tail -> this): 32k rows, 2D FP64 27 -> 10.5
-// us a cycle, 2.41 -> 1.89 ms a step; 252k rows, 2D mixed 33 -> 16.5 us, 3.85 ->
-// 3.12 ms; 74k rows, 3D FP64 4.11 -> 3.19 ms; 2M rows (levels 2 and on) 35 -> 20
-// us.  Of the 10.5 us, 3 are the top level's first loads, 1.3 each exchange,
-// 1.8 the tail, 1.2 the fine level's first step up.  Level 1's right-hand side
-// summed here too costs 2 us more where the kernel before it took 3.9 (3D: 4.3
-// for 6.6).
+// Measured, ms a step by a launch a level -> by this (2.1 l0): 2D, 9k rows FP64
+// 1.64 -> 1.27, 46k 2.30 -> 1.57, 151k mixed 2.94 -> 2.23, 1M mixed 5.65 -> 5.07;
+// 3D, 15k FP64 3.00 -> 2.15, 96k 4.13 -> 3.11, 1.1M mixed 13.7 -> 11.2.  The
+// launch takes, 32k rows 2D FP64 with the fine level in it, 19.4 us; 252k rows 2D
+// mixed 18.4; 74k rows 3D FP64 23.2; 857k rows 3D mixed 35.2; 2M rows 2D mixed
+// (levels 2 and on) 17.5.  The coarse levels of 32k rows alone were 27 us by
+// launches and 10.5 here: 3 the top level's first loads, 1.3 each exchange, 1.8
+// the tail, 1.2 the fine level's first step up.  Level 1's right-hand side summed
+// here adds 2 us where the kernel before it took 3.9 (3D: 4.3 for 6.6).
 //
 // All blocks must run at once (the host sees to it); a wait is bounded, and
 // one that fails marks every segment done with the value 2, which tells the
@@ -1082,7 +1084,8 @@ constexpr int kMgCoarseLevels = 10;  // levels lc .. lt at most
 // the 2^dim at the places (px, py, pz): 0 the row's own, 1 the other that is
 // next to it in that direction.  (3D polls 8 words a row for 28, 2D 4 for 10.)
 // Measured, rows where they are -> packed: 1M particles, 3D mixed 48 -> 42 us a
-// cycle; 2M, 2D 20.5 -> 17.5; 254k 19.0 -> 18.3; 35k FP64 unchanged at 13.9.
+// cycle (35 since, see kMgProLanes); 2M, 2D 20.5 -> 17.5; 254k 19.0 -> 18.3; 35k
+// FP64 unchanged.
 // Packing is a launch of 8-20 us a step.
 template <typename T>
 struct MgPacked {
@@ -1218,8 +1221,9 @@ __global__ void __launch_bounds__(512) k_mg_pack(MgPackIn a, MgPacked<T> o) {
 // The fine level in k_mg_coarse (multiplicative cycle): a thread a row.  Its
 // residual goes to level 1 through places of its own and x of level 1 comes
 // back through level 1's, so the cycle is one launch.
-// Measured, 32k rows FP64 (2D): k_mg_down0 4.6 + k_mg_up0 4.8 us, 2 us of gaps
-// and this launch without them 14.0 -> 19.4 us; 36.1 -> 32.5 ms per 20 steps.
+// Measured, 32k rows FP64 (2D): k_mg_down0 4.6 us, k_mg_up0 4.8, gaps 2 and this
+// launch without the fine level 14.0, together 25.4 -> 19.4 us; 36.1 -> 32.5 ms
+// per 20 steps.
 // What is added to the launch is two exchanges (1.3 us each) and a row product.
 // Steps by launches -> in it: 2D 10k rows FP64 1.39 -> 1.34 ms, mixed 1.80 ->
 // 1.70; 46k 1.93 -> 1.74, 2.23 -> 2.06; 82k (the most that fit) 2.08 -> 1.97,

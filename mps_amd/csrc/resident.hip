@@ -7,11 +7,16 @@
 // launch, block start-up and first loads, and every restart or refinement is
 // five more launches and a host read.  Here every block of the same layout
 // stays on its CU for the whole solve: one row a thread, the row's matrix
-// entries and its p, s, y in registers, r of the block's rows and of the rows
-// they couple to (the halo) in LDS.  An iteration exchanges A r of the halo
-// rows and each block's three partial sums once, and every block applies the
-// update to its halo rows itself (s = A r + beta s, r -= alpha s), so one
-// exchange an iteration is enough; a residual is one more, of r and its norm.
+// entries (16 or 36, see resident_shape) and its p, s, y in registers, r of
+// the block's rows and of the rows they couple to (the halo) in LDS.  512
+// threads leave a thread 256 registers: whole blocks in FP64 spill 15 of them
+// at 16 entries a row and some 100, 300 bytes a lane, at 36.  Even so 2D at
+// 3.1 l0 takes 0.63 ms a step where the kernels take 0.94 (40k rows, 50
+// iterations; the mixed kernel, which spills one at most, 0.57 and 1.05).  An
+// iteration exchanges A r of the halo rows and each block's three partial sums
+// once, and every block applies the update to its halo rows itself (s = A r +
+// beta s, r -= alpha s), so one exchange an iteration is enough; a residual is
+// one more, of r and its norm.
 //
 // The exchange is of tagged words: 32 bits of the value below a 32-bit tag,
 // stored and polled as relaxed device-scope 64-bit atomics.  A word carries
@@ -20,7 +25,12 @@
 // workgroups spread over the 8 XCDs; on one XCD it is the same).  Two halves
 // alternate: a block writes a half again only after it has every block's
 // partials of the exchange between, which each block sends after it has read
-// the half.
+// the half.  The exchange of y alone has no partials.  The one after it writes
+// the half of the one before it, whose readers are the blocks that have a row
+// of this block in their halo.  The matrix couples rows both ways (a pair is
+// in range for both or for neither, and padding names its own row), so those
+// are the blocks of this block's halo; they sent their y, which this block has
+// by then, after they had read that half.
 //
 // Measured (2D, FP64, launches -> resident CG -> resident solve): 492 rows,
 // ~60 iterations a step at machine epsilon 1.15 -> 0.78 -> 0.64 ms a step,
